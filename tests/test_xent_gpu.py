@@ -62,3 +62,28 @@ def test_xent_rejects_unsupported(dev):
     from naylis_amd.mom_kernels.hip_xent import cross_entropy_rows
     with pytest.raises(RuntimeError, match="multiple of"):
         cross_entropy_rows(torch.randn(4, 1000, device=dev).bfloat16(), torch.zeros(4, dtype=torch.long, device=dev))
+
+
+@pytest.mark.parametrize("chunks", [1, 4, 5, 8, 9, 17])
+def test_xent_forward_masked_rows(chunks, dev):
+    """Rows around the forward's register tiles (4 or 8 chunks of 2048), with
+    -inf and lowest-value masks over whole threads, chunks and rows, against
+    fp64.  The sum's terms carry a relative error of at most (|x - m| + 2) 2^-23
+    and |x - m| e^(x - m) is at most 1/e, so the log-sum-exp is within 2^-21 of
+    a logarithm plus its own rounding, 2^-23 |loss| with the label's."""
+    from naylis_amd.mom_kernels.hip_xent import cross_entropy_rows
+    V = 2048 * chunks
+    x = (torch.randn(6, V, generator=torch.Generator().manual_seed(chunks)) * 5).bfloat16()
+    x[1, 1:] = -float("inf")                   # one finite value
+    x[2, : V - 100] = torch.finfo(torch.bfloat16).min
+    x[3] = torch.finfo(torch.bfloat16).min     # a row of the lowest value: log V
+    x[4, : V // 2] = -float("inf")
+    x[5] = 200 * x[5]                          # the largest value decides
+    labels = torch.tensor([3, 0, V - 1, 7, V - 1, int(x[5].argmax())])
+    want = -torch.log_softmax(x.double(), -1).gather(1, labels[:, None])[:, 0]
+    got = cross_entropy_rows(x.to(dev), labels.to(dev)).double().cpu()
+    scale = x.double().gather(1, labels[:, None])[:, 0].abs() + want.abs()
+    scale[3] = float(torch.finfo(torch.bfloat16).max)  # lse and the label's logit are this large and cancel
+    assert bool(((got - want).abs() <= 2.0 ** -21 + 2.0 ** -22 * scale).all()), (got, want)
+    x[0] = -float("inf")                       # nothing to choose from: NaN, as log_softmax
+    assert bool(cross_entropy_rows(x.to(dev), labels.to(dev))[0].isnan())
