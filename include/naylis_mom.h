@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define NAYLIS_MOM_ABI_VERSION 17
+#define NAYLIS_MOM_ABI_VERSION 18
 
 #define NAYLIS_OK 0
 #define NAYLIS_ERR_ARG 1       /* invalid shape / argument (the reference raises RuntimeError) */
@@ -285,6 +285,19 @@ int naylis_mom_add_rmsnorm_bwd(const void* s, const void* weight, const float* r
 int naylis_mom_rope(const void* q, const void* k, const void* cos, const void* sin, void* q_out, void* k_out,
                     int dtype, int backward, int64_t B, int64_t S, int64_t H, int64_t head_dim, int64_t cos_batch,
                     void* stream);
+
+/* ------------------------------------------------------------- attention ---
+ * Causal self-attention of the decoder layer's Llama attention
+ * (model.py:279-345): out = softmax(scale q k^T, k <= q) v per head, in fp32
+ * with bf16 operands and outputs.  q, k, v, out and their gradients
+ * (B, S, H, head_dim) row-major bf16, 16-byte aligned; head_dim 64; scale > 0.
+ * lse (B, H, S) fp32: log2-domain log-sum-exp, from the forward to the
+ * backward; delta (B, H, S) fp32: scratch of the backward.  Deterministic. */
+int naylis_mom_attn_fwd(const void* q, const void* k, const void* v, void* out, float* lse, float scale, int64_t B,
+                        int64_t S, int64_t H, int64_t head_dim, void* stream);
+int naylis_mom_attn_bwd(const void* q, const void* k, const void* v, const void* out, const float* lse,
+                        const void* dout, void* dq, void* dk, void* dv, float* delta, float scale, int64_t B,
+                        int64_t S, int64_t H, int64_t head_dim, void* stream);
 
 /* -------------------------------------------------------------- SwiGLU ---
  * The decoder MLP's activation (transformers' LlamaMLP inside each Naylis

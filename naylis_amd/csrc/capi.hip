@@ -12,6 +12,7 @@
 #include <string.h>
 
 #include <atomic>
+#include <cmath>
 #include <initializer_list>
 #include <mutex>
 #include <string>
@@ -591,6 +592,41 @@ int naylis_mom_rope(const void* q, const void* k, const void* cos, const void* s
   return hip_status(launch_rope(q, k, cos, sin, q_out, k_out, dtype == NAYLIS_DTYPE_BF16, backward != 0, (long)B,
                                 (int)S, (int)H, (int)head_dim, (int)cos_batch, (hipStream_t)stream),
                     "mom_rope");
+}
+
+static int check_attn(int64_t B, int64_t S, int64_t H, int64_t head_dim, float scale,
+                      std::initializer_list<const void*> ptrs, const char* who) {
+  if (B < 0 || S < 0 || H < 0)
+    return fail(NAYLIS_ERR_ARG, "%s: bad shape B=%lld S=%lld H=%lld", who, (long long)B, (long long)S, (long long)H);
+  if (head_dim != 64) return fail(NAYLIS_ERR_ARG, "%s: head_dim %lld must be 64", who, (long long)head_dim);
+  if (!(scale > 0.f) || !std::isfinite(scale)) return fail(NAYLIS_ERR_ARG, "%s: scale must be positive", who);
+  if (B * S * H == 0) return NAYLIS_OK;
+  if (!attn_supported((long)B, (long)S, (long)H))
+    return fail(NAYLIS_ERR_ARG, "%s: B=%lld S=%lld H=%lld is too large", who, (long long)B, (long long)S,
+                (long long)H);
+  for (const void* p : ptrs) {
+    if (!p) return fail(NAYLIS_ERR_ARG, "%s: null pointer argument", who);
+    if (!aligned16(p)) return fail(NAYLIS_ERR_ARG, "%s: all tensors must be 16-byte aligned", who);
+  }
+  return NAYLIS_OK;
+}
+
+int naylis_mom_attn_fwd(const void* q, const void* k, const void* v, void* out, float* lse, float scale, int64_t B,
+                        int64_t S, int64_t H, int64_t head_dim, void* stream) {
+  int rc = check_attn(B, S, H, head_dim, scale, {q, k, v, out, lse}, "mom_attn_fwd");
+  if (rc || B * S * H == 0) return rc;
+  return hip_status(launch_attn_fwd(q, k, v, out, lse, scale, (long)B, (long)S, (long)H, (hipStream_t)stream),
+                    "mom_attn_fwd");
+}
+
+int naylis_mom_attn_bwd(const void* q, const void* k, const void* v, const void* out, const float* lse,
+                        const void* dout, void* dq, void* dk, void* dv, float* delta, float scale, int64_t B,
+                        int64_t S, int64_t H, int64_t head_dim, void* stream) {
+  int rc = check_attn(B, S, H, head_dim, scale, {q, k, v, out, lse, dout, dq, dk, dv, delta}, "mom_attn_bwd");
+  if (rc || B * S * H == 0) return rc;
+  return hip_status(launch_attn_bwd(q, k, v, out, lse, dout, dq, dk, dv, delta, scale, (long)B, (long)S, (long)H,
+                                    (hipStream_t)stream),
+                    "mom_attn_bwd");
 }
 
 static int check_swiglu(int dtype, int64_t n, std::initializer_list<const void*> ptrs, const char* who) {

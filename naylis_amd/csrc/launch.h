@@ -112,6 +112,15 @@ hipError_t launch_rmsnorm_bwd(const void* x, bool bf16, const void* w, const flo
 hipError_t launch_rope(const void* q, const void* k, const void* cs, const void* sn, void* qo, void* ko, bool bf16,
                        bool bwd, long B, int S, int H, int HD, int cos_batch, hipStream_t st);
 
+// Causal attention of the decoder (attention.hip): q, k, v, o and their
+// gradients (B, S, H, 64) bf16, lse (log2 domain) and delta (B * H, S) fp32.
+bool attn_supported(long B, long S, long H);
+hipError_t launch_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse, float scale, long B,
+                           long S, long H, hipStream_t st);
+hipError_t launch_attn_bwd(const void* q, const void* k, const void* v, const void* o, const float* lse,
+                           const void* dout, void* dq, void* dk, void* dv, float* delta, float scale, long B, long S,
+                           long H, hipStream_t st);
+
 // SwiGLU of the decoder MLP (swiglu.hip): h = silu(g) * u forward; backward
 // writes dg and du from dh; n elements, a multiple of 8.
 hipError_t launch_swiglu(const void* g, const void* u, const void* dh, void* h_or_dg, void* du, bool bf16, bool bwd,

@@ -4,8 +4,9 @@ transformers' ``apply_rotary_pos_emb`` (called by the Llama attention of each
 Naylis decoder layer, model.py:279-345) rotates q and k with five elementwise
 ops per tensor; ``rope`` does q and k in one library pass each way with the
 same roundings (bitwise equal in bf16 and fp32).  ``NaylisAttention`` is the
-Llama attention with that rotation, the same parameters and the same
-attention backend (SDPA).
+Llama attention with that rotation and the same parameters; plain causal bf16
+attention with heads of 64 runs on the library's kernels
+(``hip_attention.causal_attention``), any other on the configured backend.
 """
 from __future__ import annotations
 
@@ -13,6 +14,7 @@ import torch
 from transformers.models.llama.modeling_llama import ALL_ATTENTION_FUNCTIONS, LlamaAttention, eager_attention_forward
 
 from .. import _lib
+from .hip_attention import causal_attention, causal_attention_supported
 from .hip_linear import shared_input_linear
 
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -84,6 +86,14 @@ class NaylisAttention(LlamaAttention):
     """LlamaAttention with the fused rotation (no cache: the decoder trains and
     evaluates full sequences); other cases run transformers' forward."""
 
+    def _plain_causal(self, attention_mask, kwargs):
+        """The SDPA call is softmax(q k^T) v over the causal triangle and
+        nothing else: no mask, no dropout, no option of its own, and torch's
+        flash backend (the same arithmetic) not switched off by the program."""
+        return (self.config._attn_implementation == "sdpa" and attention_mask is None and not kwargs
+                and self.is_causal and self.scaling > 0 and not (self.training and self.attention_dropout)
+                and torch.backends.cuda.flash_sdp_enabled())
+
     def forward(self, hidden_states, position_embeddings=None, attention_mask=None, past_key_values=None,
                 **kwargs):
         B, S, _ = hidden_states.shape
@@ -96,10 +106,12 @@ class NaylisAttention(LlamaAttention):
             return super().forward(hidden_states, position_embeddings=position_embeddings,
                                    attention_mask=attention_mask, past_key_values=past_key_values, **kwargs)
         q, k, v = shared_input_linear(hidden_states, (self.q_proj, self.k_proj, self.v_proj))
-        q, k, v = q.view(shape), k.view(shape), v.view(shape).transpose(1, 2)
+        q, k, v = q.view(shape), k.view(shape), v.view(shape)
         q, k = rope(q, k, cos, sin)
+        if self._plain_causal(attention_mask, kwargs) and causal_attention_supported(q, k, v):
+            return self.o_proj(causal_attention(q, k, v, self.scaling).view(B, S, -1)), None
         interface = ALL_ATTENTION_FUNCTIONS.get_interface(self.config._attn_implementation, eager_attention_forward)
-        out, weights = interface(self, q.transpose(1, 2), k.transpose(1, 2), v, attention_mask,
+        out, weights = interface(self, q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), attention_mask,
                                  dropout=0.0 if not self.training else self.attention_dropout, scaling=self.scaling,
                                  **kwargs)
         return self.o_proj(out.reshape(B, S, -1).contiguous()), weights

@@ -1,0 +1,90 @@
+"""Causal attention kernels (naylis_mom_attn_*) against fp64 attention on the
+same bf16 inputs: sequence lengths around the tiles (32-row products, 64-row
+stages, 128-row workgroups), one head and many."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CASES = [(1, 1, 1), (2, 31, 1), (1, 33, 3), (1, 64, 2), (2, 65, 2), (1, 127, 4), (1, 129, 1), (2, 257, 3),
+         (1, 1021, 16), (24, 700, 8), (64, 257, 8), (3, 2048, 32)]
+
+
+def _reference(q, k, v, scale, dout):
+    """fp64 attention per head with its gradients and, for each result, the
+    largest error that bf16 P / dS and one bf16 rounding of the result allow:
+    a bf16 rounding is at most 2^-8 relative (half of the 2^-7 spacing at 1), so
+    two are 2^-7 of the sum of the terms' magnitudes, plus the fp32 exponent's
+    2^-16."""
+    q, k, v, dout = (t.double().transpose(1, 2) for t in (q, k, v, dout))
+    S = q.shape[2]
+    s = q @ k.transpose(-1, -2) * scale
+    s.masked_fill_(torch.ones(S, S, dtype=torch.bool, device=q.device).triu(1), -math.inf)
+    p = torch.softmax(s, -1)
+    o = p @ v
+    dp = dout @ v.transpose(-1, -2)
+    delta = (dout * o).sum(-1, keepdim=True)
+    ds = p * (dp - delta) * scale
+    # |dS|'s own error: P and o rounded to bf16 inside delta
+    ads = p * (dp.abs() + delta.abs() + (dout.abs() * o.abs()).sum(-1, keepdim=True)) * scale
+    pt, dst, adst = p.transpose(-1, -2), ds.transpose(-1, -2), ads.transpose(-1, -2)
+    res = {"o": (o, p @ v.abs()), "dq": (ds @ k, ads @ k.abs()), "dk": (dst @ q, adst @ q.abs()),
+           "dv": (pt @ dout, pt @ dout.abs())}
+    return {n: (a.transpose(1, 2), b.transpose(1, 2) * (2.0 ** -7 + 2.0 ** -16)) for n, (a, b) in res.items()}
+
+
+@pytest.mark.parametrize("B,S,H", CASES)
+def test_attention_matches_fp64(B, S, H, dev):
+    from naylis_amd.mom_kernels.hip_attention import causal_attention
+    g = torch.Generator(device=dev).manual_seed(S)
+    q, k, v, dout = (torch.randn(B, S, H, 64, generator=g, device=dev).bfloat16() for _ in range(4))
+    q[:, S // 2:] *= 6  # sharp rows: the running reference has to move
+    q, k, v = (t.requires_grad_() for t in (q, k, v))
+    o = causal_attention(q, k, v, 0.125)
+    o.backward(dout)
+    with torch.no_grad():
+        for b in range(B):  # one sequence at a time bounds the fp64 scores
+            ref = _reference(q[b:b + 1], k[b:b + 1], v[b:b + 1], 0.125, dout[b:b + 1])
+            got = {"o": o[b:b + 1], "dq": q.grad[b:b + 1], "dk": k.grad[b:b + 1], "dv": v.grad[b:b + 1]}
+            for n, (want, bound) in ref.items():
+                err = (got[n].double() - want).abs()
+                assert bool((err <= bound + 1e-30).all()), (n, b, float((err / (bound + 1e-30)).max()))
+
+
+def test_attention_is_deterministic_and_causal(dev):
+    from naylis_amd.mom_kernels.hip_attention import causal_attention
+    g = torch.Generator(device=dev).manual_seed(1)
+    x = [torch.randn(2, 333, 4, 64, generator=g, device=dev).bfloat16() for _ in range(4)]
+
+    def run(q, k, v, d):
+        q, k, v = (t.clone().requires_grad_() for t in (q, k, v))
+        o = causal_attention(q, k, v, 0.125)
+        o.backward(d)
+        return [o.detach(), q.grad, k.grad, v.grad]
+
+    a, b = run(*x), run(*x)
+    assert all(torch.equal(s, t) for s, t in zip(a, b))
+    y = [t.clone() for t in x]
+    for t in y[:3]:
+        t[:, 200:] *= 7     # the future reaches no earlier output, bit for bit
+    assert torch.equal(run(*y)[0][:, :200], a[0][:, :200])
+
+
+def test_attention_module_route(dev):
+    """NaylisAttention takes the kernels for plain causal bf16 attention and the
+    configured backend with a mask or another head size; both agree."""
+    from naylis_amd.decoder import naylis_config
+    from naylis_amd.mom_kernels import hip_rope
+    cfg = naylis_config(vocab_size=256, d_model=256, n_layers=1, n_heads=4, intermediate_size=256, seq_len=96)
+    attn = hip_rope.NaylisAttention(cfg, 0).to(dev).bfloat16().eval()
+    x = torch.randn(2, 96, 256, generator=torch.Generator().manual_seed(0)).bfloat16().to(dev)
+    cos, sin = (torch.rand(1, 96, 64, device=dev).bfloat16() for _ in range(2))
+    mask = torch.full((96, 96), -math.inf, device=dev).triu(1).bfloat16()[None, None].expand(2, 1, 96, 96)
+    assert attn._plain_causal(None, {}) and not attn._plain_causal(mask, {}) and not attn._plain_causal(None, {"x": 1})
+    with torch.no_grad():
+        got = attn(hidden_states=x, position_embeddings=(cos, sin))[0]
+        want = attn(hidden_states=x, position_embeddings=(cos, sin), attention_mask=mask)[0]
+    # bf16 P and one rounding of the attention's output each side, then the o projection
+    assert float((got.float() - want.float()).norm() / want.float().norm()) < 2.0 ** -7
