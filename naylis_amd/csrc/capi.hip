@@ -838,6 +838,18 @@ static int wgrad_splits(int64_t N, int64_t D_in, int64_t D_out) {
   return (int)s;
 }
 
+// fp32 partials of a weight gradient with `splits` K splits, or of the K ranges
+// that take its place where they apply
+static size_t wgrad_partial_bytes(int64_t N, int64_t D_in, int64_t D_out, int splits) {
+  if (gemm_ranges_ok((int)D_out, (int)D_in, (int)N)) return gemm_ranges_ws_bytes((int)D_out, (int)D_in, (int)N);
+  return gemm_ws_bytes(1, (int)D_out, (int)D_in, splits);
+}
+
+static hipError_t launch_wgrad(const GemmLaunch& g, hipStream_t st) {
+  return gemm_ranges_ok(g.M, g.N, g.K) ? launch_gemm_ranges(g, "linear_wgrad", st)
+                                       : launch_gemm(g, "linear_wgrad", st);
+}
+
 static int check_wgrad_dims(int64_t N, int64_t D_in, int64_t D_out) {
   if (N < 0 || D_in <= 0 || D_out <= 0 || N > ((int64_t)1 << 30) || D_in > 65536 || D_out > 65536)
     return fail(NAYLIS_ERR_ARG, "linear_wgrad: bad shape N=%lld D_in=%lld D_out=%lld", (long long)N, (long long)D_in,
@@ -850,7 +862,7 @@ static int check_wgrad_dims(int64_t N, int64_t D_in, int64_t D_out) {
 
 size_t naylis_mom_linear_wgrad_workspace_bytes(int64_t N, int64_t D_in, int64_t D_out) {
   if (check_wgrad_dims(N, D_in, D_out) != NAYLIS_OK) return 0;
-  const size_t b = gemm_ws_bytes(1, (int)D_out, (int)D_in, wgrad_splits(N, D_in, D_out));
+  const size_t b = wgrad_partial_bytes(N, D_in, D_out, wgrad_splits(N, D_in, D_out));
   return b ? b : 256;
 }
 
@@ -861,7 +873,7 @@ int naylis_mom_linear_wgrad(const void* x, const void* dy, void* dw, int dw_dtyp
   if ((rc = check_dtype(dw_dtype, "linear_wgrad"))) return rc;
   if (!dw || (N > 0 && (!x || !dy))) return fail(NAYLIS_ERR_ARG, "linear_wgrad: null pointer argument");
   const int splits = wgrad_splits(N, D_in, D_out);
-  const size_t need = gemm_ws_bytes(1, (int)D_out, (int)D_in, splits);
+  const size_t need = wgrad_partial_bytes(N, D_in, D_out, splits);
   if (need && (!workspace || workspace_bytes < need))
     return fail(NAYLIS_ERR_WORKSPACE, "linear_wgrad: workspace of %zu bytes is smaller than the %zu required",
                 workspace_bytes, need);
@@ -883,7 +895,7 @@ int naylis_mom_linear_wgrad(const void* x, const void* dy, void* dw, int dw_dtyp
   g.job[0].ldc = D_in;
   if (!gemm_supported(g))
     return fail(NAYLIS_ERR_ARG, "linear_wgrad: needs 16-byte aligned pointers and N * max(D_in, D_out) < 2^30");
-  return hip_status(launch_gemm(g, "linear_wgrad", (hipStream_t)stream), "linear_wgrad");
+  return hip_status(launch_wgrad(g, (hipStream_t)stream), "linear_wgrad");
 }
 
 // The gated weight gradient: at least two K splits, so the gate epilogue of
@@ -893,7 +905,7 @@ static int gated_wgrad_splits(int64_t N, int64_t D_in, int64_t D_out) {
 }
 
 static size_t gated_wgrad_part_off(int64_t N, int64_t D_in, int64_t D_out) {
-  return (gemm_ws_bytes(1, (int)D_out, (int)D_in, gated_wgrad_splits(N, D_in, D_out)) + 255) & ~(size_t)255;
+  return (wgrad_partial_bytes(N, D_in, D_out, gated_wgrad_splits(N, D_in, D_out)) + 255) & ~(size_t)255;
 }
 
 size_t naylis_mom_gated_wgrad_workspace_bytes(int64_t N, int64_t D_in, int64_t D_out) {
@@ -938,7 +950,7 @@ int naylis_mom_gated_wgrad(const void* x, const void* dy, const void* w, const f
   g.gate_part = part;
   if (!gemm_supported(g))
     return fail(NAYLIS_ERR_ARG, "gated_wgrad: needs 16-byte aligned pointers and N * max(D_in, D_out) < 2^30");
-  hipError_t e = launch_gemm(g, "linear_wgrad", st);
+  hipError_t e = launch_wgrad(g, st);
   if (e == hipSuccess) e = launch_rezero_reduce(part, gemm_gate_parts((int)D_out, (int)D_in), ds, st);
   return hip_status(e, "gated_wgrad");
 }

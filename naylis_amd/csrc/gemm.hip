@@ -17,6 +17,8 @@
 // A grouped launch runs up to 48 GEMMs of one shape in one grid (the bank
 // projection of all decoder layers), optionally adding their products into
 // one output in job order.
+// Products that fill the chip with 256 x 128 tiles, and long weight gradients,
+// run on the pipelined kernel of gemm_pipe.hip instead.
 #include "common.h"
 #include "launch_gemm.h"
 #include "timing.h"
@@ -511,6 +513,7 @@ hipError_t launch_gemm(const GemmLaunch& g, const char* name, hipStream_t st) {
   splits = (g.K + kper - 1) / kper;
   GemmLaunch gl = g;
   gl.K1 = g.K1 < g.K ? g.K1 : g.K;
+  if (splits == 1 && g.gate_w == nullptr && gemm_pipe_ok(gl)) return launch_gemm_pipe(gl, name, st);
   // the largest tile that still gives at least one workgroup per CU
   auto wgs = [&](int bm, int bn) {
     return (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * splits * g.njobs;

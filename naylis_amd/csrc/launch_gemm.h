@@ -53,6 +53,18 @@ bool gemm_supported(const GemmLaunch& g);
 size_t gemm_ws_bytes(int njobs, int M, int N, int splits);
 hipError_t launch_gemm(const GemmLaunch& g, const char* timer_name, hipStream_t st);
 
+// Pipelined 256 x 128 tiles (gemm_pipe.hip).  gemm_pipe_ok: a launch without
+// K splits whose tiles fill the chip; launch_gemm then takes it (C is bitwise
+// the same: every element sums its K in the same order).  gemm_ranges_ok: a
+// row-contiguous product (a weight gradient) cut into K ranges, one per CU,
+// with fp32 partials in ws (gemm_ranges_ws_bytes) and a fixed-order reduction,
+// the gate epilogue included.
+bool gemm_pipe_ok(const GemmLaunch& g);
+hipError_t launch_gemm_pipe(const GemmLaunch& g, const char* timer_name, hipStream_t st);
+bool gemm_ranges_ok(int M, int N, int K);
+size_t gemm_ranges_ws_bytes(int M, int N, int K);
+hipError_t launch_gemm_ranges(const GemmLaunch& g, const char* timer_name, hipStream_t st);
+
 // Up to kGemmMaxGroupJobs GEMMs of one shape and layout in one launch (no K
 // split; each job's C bitwise equal to launch_gemm of that job).  With
 // sum_jobs, C = sum over jobs of A_j B_j, written to job[0].c through fp32

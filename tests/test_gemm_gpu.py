@@ -150,3 +150,66 @@ def test_shared_input_linear_matches_separate_layers(dev):
     with torch.no_grad():
         outs = shared_input_linear(x, layers)
     assert all(o.grad_fn is None for o in outs)
+
+
+def _sum_bound(a, b, ref):
+    """A bf16 result of an fp32 sum of n products: one bf16 rounding (2^-8
+    relative) and sqrt(n) fp32 roundings of the terms' magnitudes, eight fold."""
+    n = a.shape[1]
+    return 2.0 ** -8 * ref.abs() + 8 * n ** 0.5 * 2.0 ** -24 * (a.abs() @ b.abs())
+
+
+@pytest.mark.parametrize("N,D_in,D_out", [
+    (16384, 1000, 1032),   # K ranges, last tiles of 104 columns and 8 rows
+    (9952, 1024, 1024),    # 311 steps a tile, listed as 312: empty last steps
+    (12288, 128, 3064),    # one column of tiles
+    (16384, 2816, 264),    # one band of two columns left over, 8 rows past a tile
+    (2048, 5632, 2048),    # whole K per tile, 256 x 256 tiles
+    (1024, 4104, 2056),    # the same with edges in both directions
+])
+def test_linear_wgrad_pipelined_shapes(N, D_in, D_out, dev):
+    g = torch.Generator(device=dev).manual_seed(D_in)
+    x = torch.randn(N, D_in, generator=g, device=dev).bfloat16()
+    dy = torch.randn(N, D_out, generator=g, device=dev).bfloat16()
+    got = wgrad(x, dy, torch.bfloat16).double()
+    a, b = dy.double().t(), x.double()
+    ref = a @ b
+    assert bool(((got - ref).abs() <= _sum_bound(a, b, ref)).all())
+    assert torch.equal(got, wgrad(x, dy, torch.bfloat16).double())
+
+
+@pytest.mark.parametrize("L,D", [(4000, 1568), (2048, 2048), (3000, 2080)])
+def test_bank_kv_pipelined_shapes(L, D, dev):
+    """The bank projection's three layouts on the pipelined tiles (the two K
+    segments of d_slots included), with edge tiles."""
+    from naylis_amd.mom_kernels.hip_bank import mom_bank_kv
+    g = torch.Generator(device=dev).manual_seed(L)
+    s, dk, dv = (torch.randn(L, D, generator=g, device=dev).bfloat16() for _ in range(3))
+    wk, wv = (torch.randn(D, D, generator=g, device=dev).bfloat16() for _ in range(2))
+    s, wk, wv = (t.requires_grad_() for t in (s, wk, wv))
+    k, v = mom_bank_kv(s, wk, wv)
+    torch.autograd.backward([k, v], [dk, dv])
+    s, wk, wv, k, v, dk, dv, ds, dwk, dwv = (t.detach().double() for t in (s, wk, wv, k, v, dk, dv, s.grad, wk.grad,
+                                                                           wv.grad))
+    for got, a, b in ((k, s, wk.t()), (v, s, wv.t()), (ds, torch.cat([dk, dv], 1), torch.cat([wk, wv], 0)),
+                      (dwk, dk.t(), s), (dwv, dv.t(), s)):
+        ref = a @ b
+        assert bool(((got - ref).abs() <= _sum_bound(a, b, ref)).all())
+
+
+def test_gated_wgrad_pipelined(dev):
+    """The gate epilogue on K ranges: dW = s dW', ds = sum dW' W."""
+    from naylis_amd.mom_kernels.hip_rezero import mom_gated_linear
+    g = torch.Generator(device=dev).manual_seed(0)
+    N, D = 16384, 1024
+    x, dy = (torch.randn(N, D, generator=g, device=dev).bfloat16() for _ in range(2))
+    w = (torch.randn(D, D, generator=g, device=dev) / 32).bfloat16().requires_grad_()
+    s = torch.full((1,), 0.75, device=dev, requires_grad=True)
+    mom_gated_linear(x, w, s).backward(dy.float())
+    a, b = dy.double().t(), x.double()
+    ref = a @ b
+    assert bool(((w.grad.double() - 0.75 * ref).abs() <= _sum_bound(a, b, 0.75 * ref)).all())
+    # a million products of dW' (each within 8 sqrt(n) roundings, independent) and W
+    ds = (ref * w.detach().double()).sum()
+    var = ((8 * N ** 0.5 * 2.0 ** -24 * (a.abs() @ b.abs())) * w.detach().double()).square().sum().sqrt()
+    assert abs(float(s.grad) - float(ds)) <= float(var) + 2.0 ** -20 * float((ref * w.detach().double()).abs().sum())
