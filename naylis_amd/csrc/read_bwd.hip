@@ -637,7 +637,7 @@ __device__ __forceinline__ void tile_count_prefix(const int32_t* __restrict__ co
 // accumulators already in the B-operand layout of dV^T = dO^T P and
 // dK^T = Q^T dS, whose A operands are read transposed from the tiles.
 template <int HD, bool ALIGNED, int TK, bool SPLIT_V>
-__global__ __launch_bounds__(256, 2) void read_bwd_dkdv_kernel(
+__global__ __launch_bounds__(256, HD == 128 ? 1 : 2) void read_bwd_dkdv_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
     const int32_t* __restrict__ top_idx, const float* __restrict__ top_gates, const bf16_t* __restrict__ dout,
     const float* __restrict__ lse, const float* __restrict__ delta, const int32_t* __restrict__ tile_list,
@@ -1158,8 +1158,16 @@ hipError_t launch_read_bwd_dq(const void* q, const void* k, const void* v, const
 int read_bwd_n_ttiles(const ReadDims& d) { return (int)(((long)d.B * d.S + kDkdvTile - 1) / kDkdvTile); }
 
 // ranges of the dK/dV work split per head: the heads' ranges together fill
-// the chip's 256 CUs with two workgroups each
-int read_bwd_ranges(const ReadDims& d) { return d.H >= 512 ? 1 : 512 / d.H; }
+// the chip's 256 CUs with the workgroups that a CU holds, two, or one at
+// head_dim 128.  Its K / V rows and accumulators are 192 registers; held to
+// 256 for two workgroups the kernel spilled 541.  6000 tokens, 8 x 128 heads,
+// 16 blocks of 64: 120 -> 68 us with 512 registers, 54 with the ranges halved
+// (the reduction of their partials 13 -> 8); 16384 tokens, 8 blocks of 128:
+// 224 -> 93.
+int read_bwd_ranges(const ReadDims& d) {
+  const int wgs = d.HD == 128 ? 256 : 512;
+  return d.H >= wgs ? 1 : wgs / d.H;
+}
 int read_bwd_parts(const ReadDims& d) { return read_bwd_ranges(d) + read_lq(d.L) / 128 - 1; }
 
 hipError_t launch_read_tile_lists(const int32_t* top_idx, uint8_t* tile_flags, int32_t* list, int32_t* count,

@@ -322,3 +322,11 @@ def test_read_pair_path_edges(dev):
     assert_close(dk, kf.grad, "dk")
     assert_close(dv, vf.grad, "dv")
     assert_close(dg, gf.grad, "d_gates")
+
+
+@pytest.mark.parametrize("case", [(1, 2048, 4, 128, 8, 64, 2, "smooth"),      # 64 ranges a head, crossing groups
+                                  (2, 333, 3, 128, 5, 48, 3, "random"),       # unaligned blocks, top-3
+                                  (1, 70, 300, 128, 2, 32, 1, "random")])     # more heads than CUs: one range each
+def test_read_hd128_ranges(case, dev):
+    """The head_dim 128 dK/dV ranges (one workgroup per CU)."""
+    test_read_fwd_bwd_matches_oracle(case, dev)
