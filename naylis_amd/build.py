@@ -1,5 +1,5 @@
 """Build libnaylis_mom.so (gfx950) in-tree with hipcc, then the torch
-extension of the fused layer node over it.
+extension of its autograd nodes.
 
     python -m naylis_amd.build [--jobs N]
 
@@ -7,7 +7,7 @@ Each .hip source is compiled to an object in parallel, then linked into
 ``naylis_amd/_lib/libnaylis_mom.so``.  Flags: -O3, gfx950 only, packed fp32
 instructions disabled (``-Xclang -target-feature -Xclang -packed-fp32-ops``),
 correctly rounded fp32 division (the router's prefix mean divides in fp32
-exactly as the reference does).  ``csrc/torch_layer.cpp`` becomes
+exactly as the reference does).  ``csrc/torch_*.cpp`` become
 ``naylis_amd/_lib/ext/naylis_torch.so`` (torch.utils.cpp_extension, host
 code only); it calls the library's C ABI, whose symbols it takes from the
 library loaded first with global visibility.
@@ -52,7 +52,7 @@ def sources():
 
 
 def build_torch_ext(verbose=False):
-    """Compile csrc/torch_layer.cpp into the torch extension (every time: the
+    """Compile csrc/torch_*.cpp into the torch extension (every time: the
     previous outputs are removed first)."""
     import ctypes
 
@@ -64,7 +64,7 @@ def build_torch_ext(verbose=False):
     # cpp_extension imports the module it built: its C-ABI symbols come from
     # the library, loaded here with global visibility as naylis_amd._lib does
     ctypes.CDLL(LIB, mode=ctypes.RTLD_GLOBAL)
-    ce.load(name=EXT_NAME, sources=[os.path.join(CSRC, "torch_layer.cpp")], build_directory=EXT_DIR,
+    ce.load(name=EXT_NAME, sources=[os.path.join(CSRC, f) for f in ("torch_layer.cpp", "torch_nodes.cpp")], build_directory=EXT_DIR,
             extra_include_paths=[INCLUDE], extra_cflags=["-O2"], verbose=verbose)
     if not os.path.exists(EXT):
         raise RuntimeError(f"torch extension build produced no {EXT}")

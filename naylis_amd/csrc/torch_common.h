@@ -1,0 +1,69 @@
+// Shared by the torch extension's sources: status checks, workspaces and the
+// weight-gradient call over the C ABI of libnaylis_mom.so.
+#pragma once
+#include <torch/extension.h>
+
+#include <algorithm>
+#include <stdexcept>
+#include <string>
+#include <vector>
+
+#include "../../include/naylis_mom.h"
+
+namespace naylis_ext {
+
+constexpr int kF32 = 0, kBF16 = 1;
+
+// A non-zero status of a C-ABI call; reaches Python as naylis_amd._lib.NaylisError.
+struct StatusError : std::runtime_error {
+  int code;
+  StatusError(int c, const std::string& m) : std::runtime_error(m), code(c) {}
+};
+
+inline void check(int rc) {
+  if (rc != NAYLIS_OK) {
+    const char* msg = naylis_mom_last_error();
+    throw StatusError(rc, msg ? msg : "unknown error");
+  }
+}
+
+// A workspace query's answer (0: the shape is not supported, with a message).
+inline size_t need(size_t nbytes) {
+  if (nbytes == 0) check(NAYLIS_ERR_ARG);
+  return nbytes;
+}
+
+inline at::Tensor workspace(size_t nbytes, const at::Tensor& like) {
+  return at::empty({(int64_t)std::max<size_t>(nbytes, 1)}, like.options().dtype(at::kByte));
+}
+
+inline int dtype_code(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16 ? kBF16 : kF32; }
+
+inline void* ptr(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+inline void* stream_ptr(int64_t st) { return reinterpret_cast<void*>(st); }
+
+// dW = dy^T xin over all rows: the library's GEMM when N, D_in, D_out are
+// multiples of 8, else torch's product (the hip_linear.library_wgrad rule)
+at::Tensor library_wgrad(const at::Tensor& xin, const at::Tensor& dy, at::ScalarType dtype, void* st);
+
+// y2 = out2 (s W_o)^T in fp32 and the scaled weight; its backward (d out2, dW_o, ds)
+std::pair<at::Tensor, at::Tensor> gated_linear_forward(const at::Tensor& out2, const at::Tensor& w_o,
+                                                       const at::Tensor& s, void* st);
+struct GatedGrads {
+  at::Tensor dout2, dw_o, ds;
+};
+GatedGrads gated_linear_backward(const at::Tensor& dy2, const at::Tensor& out2, const at::Tensor& w_o,
+                                 const at::Tensor& w_os, const at::Tensor& s, void* st);
+
+// The router backward's d_probs: an fp32 gradient expanded from one row goes in
+// as that row with stride 0, anything else as a dense fp32 copy with stride E.
+struct ProbsGrad {
+  at::Tensor t;
+  int64_t stride;
+};
+ProbsGrad probs_grad(const at::Tensor& g, int64_t E);
+
+void bind_nodes(pybind11::module_& m);
+
+}  // namespace naylis_ext

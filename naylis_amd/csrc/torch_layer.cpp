@@ -15,46 +15,59 @@
 // The library's symbols are not linked here: libnaylis_mom.so is loaded with
 // global visibility before this module (naylis_amd/_lib.py), so these calls
 // bind to that one instance (its timing state and scratch arrays included).
-#include <torch/extension.h>
+#include "torch_common.h"
 
-#include <algorithm>
-#include <vector>
-
-#include "../../include/naylis_mom.h"
+using namespace naylis_ext;
 
 namespace {
 
-constexpr int kF32 = 0, kBF16 = 1;
-
-void check(int rc, const char* what) {
-  if (rc != NAYLIS_OK) {
-    const char* msg = naylis_mom_last_error();
-    TORCH_CHECK(false, "naylis_mom ", what, " failed (status ", rc, "): ", msg ? msg : "");
-  }
-}
-
-at::Tensor workspace(size_t nbytes, const at::Tensor& like) {
-  return at::empty({(int64_t)std::max<size_t>(nbytes, 1)}, like.options().dtype(at::kByte));
-}
-
-int dtype_code(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16 ? kBF16 : kF32; }
-
 void* opt_ptr(const c10::optional<at::Tensor>& t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
 
-// dW = dy^T xin over all rows: the library's split-K GEMM when N, D_in, D_out
-// are multiples of 8, else torch's product (the hip_linear.library_wgrad rule)
-at::Tensor library_wgrad(const at::Tensor& xin, const at::Tensor& dy, at::ScalarType dtype, void* st) {
-  const int64_t N = xin.size(0), D_in = xin.size(1), D_out = dy.size(1);
-  if (N % 8 || D_in % 8 || D_out % 8) {
-    if (dtype == at::kFloat) return at::mm(dy.t(), xin, at::kFloat);
-    return at::mm(dy.t(), xin).to(dtype);
+// The read's inputs and what its backward takes: bank K / V (from the caller,
+// or projected from the bank's slots), queries, token order, output, the pair
+// path's side buffer and the log-sum-exp.  A gradient-checkpointed layer runs
+// this again in its backward (no random numbers: the same bits).
+struct ReadState {
+  at::Tensor slots, k, v, q, order, out, side, lse;
+};
+
+ReadState read_part(const at::Tensor& x, const c10::optional<at::Tensor>& m_blocks, const at::Tensor& w_q,
+                    const at::Tensor& w_k, const at::Tensor& w_v, const c10::optional<at::Tensor>& k_ext,
+                    const c10::optional<at::Tensor>& v_ext, const at::Tensor& top_idx, const at::Tensor& gates,
+                    int64_t n_heads, int64_t num_blocks, int64_t block_size, int64_t top_k, void* st) {
+  const int64_t B = x.size(0), T = x.size(1), D = x.size(2), H = n_heads, HD = D / n_heads;
+  ReadState r;
+  // ---- bank K/V (model.py:253-256), unless the caller projected the bank
+  if (!k_ext.has_value()) {
+    r.slots = m_blocks->reshape({-1, D}).to(at::kBFloat16).contiguous();
+    const int64_t L = r.slots.size(0);
+    r.k = at::empty({L, D}, x.options().dtype(at::kBFloat16));
+    r.v = at::empty({L, D}, x.options().dtype(at::kBFloat16));
+    check(naylis_mom_bank_kv_fwd(r.slots.data_ptr(), w_k.data_ptr(), w_v.data_ptr(), r.k.data_ptr(), r.v.data_ptr(), L, D,
+                                 D, st));
+  } else {
+    r.k = *k_ext;
+    r.v = *v_ext;
   }
-  at::Tensor ws = workspace(naylis_mom_linear_wgrad_workspace_bytes(N, D_in, D_out), xin);
-  at::Tensor dw = at::empty({D_out, D_in}, xin.options().dtype(dtype));
-  check(naylis_mom_linear_wgrad(xin.data_ptr(), dy.data_ptr(), dw.data_ptr(), dtype == at::kBFloat16 ? kBF16 : kF32,
-                                ws.data_ptr(), ws.numel(), N, D_in, D_out, st),
-        "linear_wgrad");
-  return dw;
+  // ---- q projection, token order, gated read (model.py:251, 258-276)
+  r.q = at::linear(x, w_q);
+  const int64_t words = naylis_mom_read_order_words(B, T, num_blocks, top_k);
+  if (words <= 0) check(NAYLIS_ERR_ARG);
+  r.order = at::empty({words}, x.options().dtype(at::kInt));
+  {
+    at::Tensor ows = workspace(naylis_mom_read_order_workspace_bytes(B, T, num_blocks, top_k), x);
+    check(naylis_mom_read_order(top_idx.data_ptr<int32_t>(), r.order.data_ptr<int32_t>(), ows.data_ptr(), ows.numel(),
+                                B, T, num_blocks, top_k, st));
+  }
+  r.out = at::empty_like(r.q);
+  const size_t side_bytes = naylis_mom_read_side_bytes(B, T, H, HD, num_blocks, block_size, top_k);
+  if (side_bytes > 0) r.side = at::empty({(int64_t)side_bytes}, x.options().dtype(at::kByte));
+  r.lse = at::empty({H, B, T}, x.options().dtype(at::kFloat));
+  check(naylis_mom_read_fwd(r.q.data_ptr(), r.k.data_ptr(), r.v.data_ptr(), top_idx.data_ptr<int32_t>(),
+                            gates.data_ptr<float>(), r.order.data_ptr<int32_t>(), r.out.data_ptr(),
+                            ptr(r.side), r.lse.data_ptr<float>(), nullptr, 0, B, T, H, HD,
+                            num_blocks, block_size, top_k, st));
+  return r;
 }
 
 }  // namespace
@@ -72,7 +85,7 @@ std::vector<at::Tensor> layer_fwd(at::Tensor x, c10::optional<at::Tensor> m_bloc
   void* st = reinterpret_cast<void*>(stream);
   x = x.contiguous();
   const int64_t B = x.size(0), T = x.size(1), D = x.size(2);
-  const int64_t R = w_down.size(0), E = w_up.size(0), H = n_heads, HD = D / n_heads;
+  const int64_t R = w_down.size(0), E = w_up.size(0);
   const auto f32 = x.options().dtype(at::kFloat);
   // ---- router (model.py:169-220)
   at::Tensor logits = at::empty({B, T, E}, f32), probs = at::empty({B, T, E}, f32);
@@ -84,51 +97,15 @@ std::vector<at::Tensor> layer_fwd(at::Tensor x, c10::optional<at::Tensor> m_bloc
                                 static_cast<const float*>(opt_ptr(noise)), (int)noise_kind, (float)noise_scale,
                                 logits.data_ptr<float>(), probs.data_ptr<float>(), top_idx.data_ptr<int32_t>(),
                                 gates.data_ptr<float>(), act.data_ptr<float>(), nullptr, rws.data_ptr(), rws.numel(),
-                                B, T, D, R, E, top_k, st),
-          "router_fwd");
+                                B, T, D, R, E, top_k, st));
   }
-  // ---- bank K/V (model.py:253-256), unless the caller projected the bank
-  at::Tensor slots, k, v;
-  if (!k_ext.has_value()) {
-    slots = m_blocks->reshape({-1, D}).to(at::kBFloat16).contiguous();
-    const int64_t L = slots.size(0);
-    k = at::empty({L, D}, x.options().dtype(at::kBFloat16));
-    v = at::empty({L, D}, x.options().dtype(at::kBFloat16));
-    check(naylis_mom_bank_kv_fwd(slots.data_ptr(), w_k.data_ptr(), w_v.data_ptr(), k.data_ptr(), v.data_ptr(), L, D,
-                                 D, st),
-          "bank_kv_fwd");
-  } else {
-    k = *k_ext;
-    v = *v_ext;
-  }
-  // ---- q projection, token order, gated read (model.py:251, 258-276)
-  at::Tensor q = at::linear(x, w_q);
-  const int64_t words = naylis_mom_read_order_words(B, T, num_blocks, top_k);
-  if (words <= 0) check(NAYLIS_ERR_ARG, "read_order_words");
-  at::Tensor order = at::empty({words}, x.options().dtype(at::kInt));
-  {
-    at::Tensor ows = workspace(naylis_mom_read_order_workspace_bytes(B, T, num_blocks, top_k), x);
-    check(naylis_mom_read_order(top_idx.data_ptr<int32_t>(), order.data_ptr<int32_t>(), ows.data_ptr(), ows.numel(),
-                                B, T, num_blocks, top_k, st),
-          "read_order");
-  }
-  at::Tensor out = at::empty_like(q);
-  at::Tensor side;
-  const size_t side_bytes = naylis_mom_read_side_bytes(B, T, H, HD, num_blocks, block_size, top_k);
-  if (side_bytes > 0) side = at::empty({(int64_t)side_bytes}, x.options().dtype(at::kByte));
-  at::Tensor lse = at::empty({H, B, T}, f32);
-  check(naylis_mom_read_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), top_idx.data_ptr<int32_t>(),
-                            gates.data_ptr<float>(), order.data_ptr<int32_t>(), out.data_ptr(),
-                            side.defined() ? side.data_ptr() : nullptr, lse.data_ptr<float>(), nullptr, 0, B, T, H, HD,
-                            num_blocks, block_size, top_k, st),
-        "read_fwd");
+  // ---- bank K/V, q projection, token order, gated read
+  const ReadState rd = read_part(x, m_blocks, w_q, w_k, w_v, k_ext, v_ext, top_idx, gates, n_heads, num_blocks,
+                                 block_size, top_k, st);
   // ---- o projection with the ReZero gate folded into the weight (model.py:251, 239)
-  at::Tensor w_os = at::empty_like(w_o);
-  check(naylis_mom_rezero_scale(w_o.data_ptr(), dtype_code(w_o), scale.data_ptr<float>(), w_os.data_ptr(),
-                                dtype_code(w_os), w_o.numel(), st),
-        "rezero_scale");
-  at::Tensor y = at::mm(out.view({B * T, D}), w_os.t(), at::kFloat).view({B, T, D});
-  return {y, probs, top_idx, act, gates, slots, k, v, q, order, out, side, lse, w_os};
+  const auto [y, w_os] = gated_linear_forward(rd.out.view({B * T, D}), w_o, scale, st);
+  return {y.view({B, T, D}), probs, top_idx, act, gates, rd.slots, rd.k, rd.v, rd.q, rd.order, rd.out, rd.side, rd.lse,
+          w_os};
 }
 
 // Returns [dx, d_m, dw_down, dw_up, dw_q, dw_k, dw_v, dw_o, ds, dk_ext,
@@ -149,39 +126,20 @@ std::vector<at::Tensor> layer_bwd(c10::optional<at::Tensor> dy, c10::optional<at
   const auto f32 = x.options().dtype(at::kFloat);
   // ---- o projection with the folded gate: d out, dW_o, ds
   at::Tensor dy_t = dy.has_value() && dy->defined() ? *dy : at::zeros({B, T, D}, x.options().dtype(at::kBFloat16));
-  at::Tensor dy2 = dy_t.reshape({N, D}).to(at::kBFloat16).contiguous();
-  at::Tensor out2 = out.view({N, D});
-  at::Tensor dout2 = at::mm(dy2, w_os);
-  const int64_t D_in = out2.size(1), D_out = dy2.size(1);
-  at::Tensor dw_o = at::empty_like(w_o), ds = at::empty({1}, f32);
-  if (out2.scalar_type() == at::kBFloat16 && w_o.scalar_type() == at::kBFloat16 && w_o.is_contiguous() &&
-      out2.is_contiguous() && N % 8 == 0 && D_in % 8 == 0 && D_out % 8 == 0) {
-    at::Tensor ws = workspace(naylis_mom_gated_wgrad_workspace_bytes(N, D_in, D_out), x);
-    check(naylis_mom_gated_wgrad(out2.data_ptr(), dy2.data_ptr(), w_o.data_ptr(), scale.data_ptr<float>(),
-                                 dw_o.data_ptr(), ds.data_ptr<float>(), ws.data_ptr(), ws.numel(), N, D_in, D_out, st),
-          "gated_wgrad");
-  } else {
-    at::Tensor dw_s = library_wgrad(out2, dy2, at::kFloat, st);
-    at::Tensor ws = workspace(naylis_mom_rezero_workspace_bytes(w_o.numel()), x);
-    check(naylis_mom_rezero_bwd(dw_s.data_ptr(), dtype_code(dw_s), w_o.data_ptr(), dtype_code(w_o),
-                                scale.data_ptr<float>(), dw_o.data_ptr(), ds.data_ptr<float>(), ws.data_ptr(),
-                                ws.numel(), w_o.numel(), st),
-          "rezero_bwd");
-  }
+  GatedGrads go = gated_linear_backward(dy_t.reshape({N, D}), out.view({N, D}), w_o, w_os, scale, st);
   // ---- gated read
   at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), dgates = at::empty_like(gates);
   {
     const size_t nbytes = naylis_mom_read_workspace_bytes(B, T, H, HD, num_blocks, block_size, top_k);
-    if (nbytes == 0) check(NAYLIS_ERR_ARG, "read_workspace_bytes");
+    if (nbytes == 0) check(NAYLIS_ERR_ARG);
     at::Tensor rws = workspace(nbytes, x);
     check(naylis_mom_read_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), top_idx.data_ptr<int32_t>(),
                               gates.data_ptr<float>(), order.data_ptr<int32_t>(), out.data_ptr(), opt_ptr(side),
-                              lse.data_ptr<float>(), dout2.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                              lse.data_ptr<float>(), go.dout2.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
                               dgates.data_ptr<float>(), rws.data_ptr(), rws.numel(), B, T, H, HD, num_blocks,
-                              block_size, top_k, st),
-          "read_bwd");
+                              block_size, top_k, st));
   }
-  dout2 = at::Tensor();
+  go.dout2 = at::Tensor();
   // ---- bank K/V (the caller's grouped node takes dK, dV when it projected the bank)
   at::Tensor d_m, dw_k, dw_v, dk_ext, dv_ext;
   if (external_bank) {
@@ -193,8 +151,7 @@ std::vector<at::Tensor> layer_bwd(c10::optional<at::Tensor> dy, c10::optional<at
     dw_v = at::empty_like(w_v);
     check(naylis_mom_bank_kv_bwd(slots->data_ptr(), w_k.data_ptr(), w_v.data_ptr(), dk.data_ptr(), dv.data_ptr(),
                                  d_slots.data_ptr(), m_bf16 ? kBF16 : kF32, dw_k.data_ptr(), dw_v.data_ptr(), kBF16,
-                                 L, D, D, st),
-          "bank_kv_bwd");
+                                 L, D, D, st));
     d_m = d_slots.view(m_shape);
   }
   // ---- q projection: dx = dq W_q (the router adds its part below), dW_q = dq^T x
@@ -203,31 +160,18 @@ std::vector<at::Tensor> layer_bwd(c10::optional<at::Tensor> dy, c10::optional<at
   at::Tensor dw_q = library_wgrad(x.view({N, D}), dq2, w_q.scalar_type(), st);
   // ---- router, accumulating into dx; d_probs as one row with stride 0 when it
   // is an expanded row, else dense (the hip_router.d_probs_arg rule)
-  at::Tensor dp;
-  int64_t dp_stride = E;
-  if (d_probs.has_value() && d_probs->defined()) {
-    const at::Tensor& g = *d_probs;
-    bool row = g.scalar_type() == at::kFloat && g.stride(-1) == 1;
-    for (int64_t i = 0; row && i + 1 < g.dim(); ++i) row = g.stride(i) == 0;
-    if (row) {
-      dp = g;
-      dp_stride = 0;
-    } else {
-      dp = g.to(at::kFloat).contiguous();
-    }
-  }
+  const ProbsGrad dp = probs_grad(d_probs.has_value() ? *d_probs : at::Tensor(), E);
   at::Tensor dw_down = at::empty({R, D}, f32), dw_up = at::empty({E, R}, f32);
   {
     at::Tensor rws = workspace(naylis_mom_router_workspace_bytes(B, T, D, R, E, top_k), x);
     check(naylis_mom_router_bwd(x.data_ptr(), kBF16, w_down.data_ptr<float>(), w_up.data_ptr<float>(),
                                 act.data_ptr<float>(), probs.data_ptr<float>(), top_idx.data_ptr<int32_t>(),
                                 gates.data_ptr<float>(), dgates.data_ptr<float>(),
-                                dp.defined() ? dp.data_ptr<float>() : nullptr, dp_stride, nullptr, dx.data_ptr(), 1,
+                                static_cast<const float*>(ptr(dp.t)), dp.stride, nullptr, dx.data_ptr(), 1,
                                 dw_down.data_ptr<float>(), dw_up.data_ptr<float>(), rws.data_ptr(), rws.numel(), B,
-                                T, D, R, E, top_k, st),
-          "router_bwd");
+                                T, D, R, E, top_k, st));
   }
-  return {dx, d_m, dw_down, dw_up, dw_q, dw_k, dw_v, dw_o, ds, dk_ext, dv_ext};
+  return {dx, d_m, dw_down, dw_up, dw_q, dw_k, dw_v, go.dw_o, go.ds, dk_ext, dv_ext};
 }
 
 namespace {
@@ -248,7 +192,8 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
                                                 at::Tensor scale, at::Tensor noise, bool has_noise,
                                                 double noise_scale, int64_t n_heads, int64_t num_blocks,
                                                 int64_t block_size, int64_t top_k, int64_t noise_kind,
-                                                at::Tensor k_ext, at::Tensor v_ext, bool external, int64_t stream) {
+                                                at::Tensor k_ext, at::Tensor v_ext, bool external, bool ckpt,
+                                                int64_t stream) {
     const at::Tensor none;
     x = x.contiguous();
     std::vector<at::Tensor> r =
@@ -256,8 +201,14 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
                   has_noise ? opt(noise) : c10::nullopt, noise_scale, n_heads, num_blocks, block_size, top_k,
                   noise_kind, external ? opt(k_ext) : c10::nullopt, external ? opt(v_ext) : c10::nullopt, stream);
     // r: y, probs, top_idx, act, gates, slots, k, v, q, order, out, side, lse, w_os
-    ctx->save_for_backward({x, r[5], w_down, w_up, w_q, w_k, w_v, w_o, scale, r[3], r[1], r[2], r[4], r[6], r[7],
-                            r[8], r[9], r[10], r[11], r[12], r[13]});
+    if (ckpt)  // the read's inputs only: its backward runs read_part again
+      ctx->save_for_backward({x, external ? none : m_blocks, w_down, w_up, w_q, w_k, w_v, w_o, scale, r[3], r[1],
+                              r[2], r[4], external ? k_ext : none, external ? v_ext : none, none, none, none, none,
+                              none, r[13]});
+    else
+      ctx->save_for_backward({x, r[5], w_down, w_up, w_q, w_k, w_v, w_o, scale, r[3], r[1], r[2], r[4], r[6], r[7],
+                              r[8], r[9], r[10], r[11], r[12], r[13]});
+    ctx->saved_data["ckpt"] = ckpt;
     ctx->saved_data["geom"] = std::vector<int64_t>{n_heads, num_blocks, block_size, top_k, stream};
     ctx->saved_data["external"] = external;
     ctx->saved_data["m_shape"] = external ? std::vector<int64_t>{} : m_blocks.sizes().vec();
@@ -269,13 +220,26 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
 
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
-    const torch::autograd::variable_list s = ctx->get_saved_variables();
+    torch::autograd::variable_list s = ctx->get_saved_variables();
     const std::vector<int64_t> geom = ctx->saved_data["geom"].toIntVector();
     const bool external = ctx->saved_data["external"].toBool();
     std::vector<int64_t> m_shape = ctx->saved_data["m_shape"].toIntVector();
     const bool m_bf16 = ctx->saved_data["m_bf16"].toBool();
     // s: x, slots, w_down, w_up, w_q, w_k, w_v, w_o, scale, act, probs, top_idx, gates, k, v, q, order,
     // out, side, lse, w_os
+    if (ctx->saved_data["ckpt"].toBool()) {  // s[1] is the bank
+      at::DeviceGuard guard(s[0].device());
+      const ReadState rd = read_part(s[0], opt(s[1]), s[4], s[5], s[6], opt(s[13]), opt(s[14]), s[11], s[12], geom[0],
+                                     geom[1], geom[2], geom[3], stream_ptr(geom[4]));
+      s[1] = rd.slots;
+      s[13] = rd.k;
+      s[14] = rd.v;
+      s[15] = rd.q;
+      s[16] = rd.order;
+      s[17] = rd.out;
+      s[18] = rd.side;
+      s[19] = rd.lse;
+    }
     std::vector<at::Tensor> r =
         layer_bwd(opt(grads[0]), opt(grads[1]), s[0], opt(s[1]), s[2], s[3], s[4], s[5], s[6], s[7], s[8], s[9],
                   s[10], s[11], s[12], s[13], s[14], s[15], s[16], s[17], opt(s[18]), s[19], s[20], geom[0],
@@ -283,7 +247,7 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
     // r: dx, d_m, dw_down, dw_up, dw_q, dw_k, dw_v, dw_o, ds, dk_ext, dv_ext
     const at::Tensor none;
     return {r[0], r[1],  r[2], r[3], r[4], r[5], r[6], r[7], r[8].view(s[8].sizes()), none, none,
-            none, none, none, none, none, none, r[9], r[10], none, none};
+            none, none, none, none, none, none, r[9], r[10], none, none, none};
   }
 };
 
@@ -292,20 +256,21 @@ std::vector<at::Tensor> mom_layer_node(at::Tensor x, c10::optional<at::Tensor> m
                                        at::Tensor w_o, at::Tensor scale, c10::optional<at::Tensor> noise,
                                        double noise_scale, int64_t n_heads, int64_t num_blocks, int64_t block_size,
                                        int64_t top_k, int64_t noise_kind, c10::optional<at::Tensor> k_ext,
-                                       c10::optional<at::Tensor> v_ext, int64_t stream) {
+                                       c10::optional<at::Tensor> v_ext, bool ckpt, int64_t stream) {
   const bool external = k_ext.has_value() && k_ext->defined();
   const bool has_noise = noise.has_value() && noise->defined();
   TORCH_CHECK(external || (m_blocks.has_value() && m_blocks->defined()), "mom_layer: no bank and no external K / V");
   TORCH_CHECK(!external || (v_ext.has_value() && v_ext->defined()), "mom_layer: external K without V");
   return MomLayerNode::apply(x, external ? x : *m_blocks, w_down, w_up, w_q, w_k, w_v, w_o, scale,
                              has_noise ? *noise : x, has_noise, noise_scale, n_heads, num_blocks, block_size, top_k,
-                             noise_kind, external ? *k_ext : x, external ? *v_ext : x, external, stream);
+                             noise_kind, external ? *k_ext : x, external ? *v_ext : x, external, ckpt, stream);
 }
 
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.doc() = "Fused MoM layer node over the C ABI of libnaylis_mom.so";
+  m.doc() = "Autograd nodes over the C ABI of libnaylis_mom.so";
+  bind_nodes(m);
   m.def("layer_fwd", &layer_fwd, "MoM layer forward (router, bank K/V, q projection, read, o projection)");
   m.def("layer_bwd", &layer_bwd, "MoM layer backward (the forward's gradients in one fixed order)");
   m.def("mom_layer", &mom_layer_node,

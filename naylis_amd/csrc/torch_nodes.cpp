@@ -1,0 +1,531 @@
+// The library's single operations as C++ autograd functions, and the decode
+// step: what the Python modules of mom_kernels/ call.  Each node allocates its
+// outputs, makes its C-ABI calls on the stream that the caller was on and
+// saves its tensors; the autograd engine runs the backward without Python.
+// Argument checks and dispatch rules stay in the Python wrappers.
+//
+// A Python autograd function over ctypes costs 15 - 30 us of host time per
+// call and direction, a node here about 6.  Host time to enqueue a pass: one
+// decode step 15.6 -> 7 us, the checkpointed layer (3885 tokens, forward and
+// backward, its recompute in the layer's node) 960 -> 427, the decoder's MLP
+// half 410 -> 339 and attention half 620 -> 507, eight layers' evaluation
+// 3630 -> 3120.
+#include "torch_common.h"
+
+namespace naylis_ext {
+
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+
+at::Tensor library_wgrad(const at::Tensor& xin, const at::Tensor& dy, at::ScalarType dtype, void* st) {
+  const int64_t N = xin.size(0), D_in = xin.size(1), D_out = dy.size(1);
+  if (N % 8 || D_in % 8 || D_out % 8) {
+    if (dtype == at::kFloat) return at::mm(dy.t(), xin, at::kFloat);
+    return at::mm(dy.t(), xin).to(dtype);
+  }
+  at::Tensor ws = workspace(naylis_mom_linear_wgrad_workspace_bytes(N, D_in, D_out), xin);
+  at::Tensor dw = at::empty({D_out, D_in}, xin.options().dtype(dtype));
+  check(naylis_mom_linear_wgrad(xin.data_ptr(), dy.data_ptr(), dw.data_ptr(), dtype == at::kBFloat16 ? kBF16 : kF32,
+                                ws.data_ptr(), ws.numel(), N, D_in, D_out, st));
+  return dw;
+}
+
+std::pair<at::Tensor, at::Tensor> gated_linear_forward(const at::Tensor& out2, const at::Tensor& w_o,
+                                                       const at::Tensor& s, void* st) {
+  at::Tensor w_os = at::empty_like(w_o);
+  check(naylis_mom_rezero_scale(w_o.data_ptr(), dtype_code(w_o), s.data_ptr<float>(), w_os.data_ptr(),
+                                dtype_code(w_os), w_o.numel(), st));
+  return {at::mm(out2, w_os.t(), at::kFloat), w_os};
+}
+
+GatedGrads gated_linear_backward(const at::Tensor& dy, const at::Tensor& out2, const at::Tensor& w_o,
+                                 const at::Tensor& w_os, const at::Tensor& s, void* st) {
+  const at::Tensor dy2 = dy.to(at::kBFloat16).contiguous();
+  GatedGrads g;
+  g.dout2 = at::mm(dy2, w_os);
+  const int64_t N = out2.size(0), D_in = out2.size(1), D_out = dy2.size(1);
+  g.dw_o = at::empty_like(w_o);
+  g.ds = at::empty({1}, out2.options().dtype(at::kFloat));
+  if (out2.scalar_type() == at::kBFloat16 && w_o.scalar_type() == at::kBFloat16 && w_o.is_contiguous() &&
+      out2.is_contiguous() && N % 8 == 0 && D_in % 8 == 0 && D_out % 8 == 0) {
+    // dW' = dy^T out stays inside the split-K reduction, whose epilogue writes
+    // dW_o = s dW' and the partials of ds = sum(dW' W_o)
+    at::Tensor ws = workspace(naylis_mom_gated_wgrad_workspace_bytes(N, D_in, D_out), out2);
+    check(naylis_mom_gated_wgrad(out2.data_ptr(), dy2.data_ptr(), w_o.data_ptr(), s.data_ptr<float>(),
+                                 g.dw_o.data_ptr(), g.ds.data_ptr<float>(), ws.data_ptr(), ws.numel(), N, D_in, D_out,
+                                 st));
+    return g;
+  }
+  at::Tensor dw_s = library_wgrad(out2, dy2, at::kFloat, st);
+  at::Tensor ws = workspace(naylis_mom_rezero_workspace_bytes(w_o.numel()), out2);
+  check(naylis_mom_rezero_bwd(dw_s.data_ptr(), dtype_code(dw_s), w_o.data_ptr(), dtype_code(w_o), s.data_ptr<float>(),
+                              g.dw_o.data_ptr(), g.ds.data_ptr<float>(), ws.data_ptr(), ws.numel(), w_o.numel(), st));
+  return g;
+}
+
+ProbsGrad probs_grad(const at::Tensor& g, int64_t E) {
+  if (!g.defined()) return {g, E};
+  bool row = g.scalar_type() == at::kFloat && g.stride(-1) == 1;
+  for (int64_t i = 0; row && i + 1 < g.dim(); ++i) row = g.stride(i) == 0;
+  if (row) return {g, 0};
+  return {g.to(at::kFloat).contiguous(), E};
+}
+
+namespace {
+
+at::Tensor f32_or_none(const at::Tensor& t) { return t.defined() ? t.to(at::kFloat).contiguous() : t; }
+
+at::TensorOptions f32_of(const at::Tensor& t) { return t.options().dtype(at::kFloat); }
+
+// ---- RMSNorm, with and without the residual add in front --------------------
+
+struct RmsNorm : public Function<RmsNorm> {
+  static at::Tensor forward(AutogradContext* ctx, at::Tensor x, at::Tensor w, double eps, int64_t st) {
+    at::DeviceGuard guard(x.device());
+    const int64_t D = x.size(-1);
+    const at::Tensor x2 = x.contiguous().view({-1, D});
+    const int64_t N = x2.size(0);
+    at::Tensor y = at::empty_like(x2), rstd = at::empty({N}, f32_of(x));
+    check(naylis_mom_rmsnorm_fwd(x2.data_ptr(), dtype_code(x), w.data_ptr(), y.data_ptr(), rstd.data_ptr<float>(), N,
+                                 D, (float)eps, stream_ptr(st)));
+    ctx->save_for_backward({x2, w, rstd});
+    ctx->saved_data["shape"] = x.sizes().vec();
+    ctx->saved_data["st"] = st;
+    return y.view(x.sizes());
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &x2 = s[0], &w = s[1], &rstd = s[2];
+    at::DeviceGuard guard(x2.device());
+    const int64_t N = x2.size(0), D = x2.size(1);
+    const at::Tensor dy = grads[0].to(x2.scalar_type()).contiguous();
+    at::Tensor dx = at::empty_like(x2), dw = at::empty_like(w);
+    at::Tensor ws = workspace(naylis_mom_rmsnorm_workspace_bytes(N, D), x2);
+    check(naylis_mom_rmsnorm_bwd(x2.data_ptr(), dtype_code(x2), w.data_ptr(), rstd.data_ptr<float>(), dy.data_ptr(),
+                                 dx.data_ptr(), dw.data_ptr(), ws.data_ptr(), ws.numel(), N, D,
+                                 stream_ptr(ctx->saved_data["st"].toInt())));
+    return {dx.view(ctx->saved_data["shape"].toIntVector()), dw, at::Tensor(), at::Tensor()};
+  }
+};
+
+struct AddRmsNorm : public Function<AddRmsNorm> {
+  static variable_list forward(AutogradContext* ctx, at::Tensor x, at::Tensor a, at::Tensor w, double eps,
+                               int64_t st) {
+    at::DeviceGuard guard(x.device());
+    const int64_t D = x.size(-1);
+    const at::Tensor x2 = x.contiguous().view({-1, D}), a2 = a.contiguous().view({-1, D});
+    const int64_t N = x2.size(0);
+    at::Tensor s = at::empty_like(x2), y = at::empty_like(x2), rstd = at::empty({N}, f32_of(x));
+    check(naylis_mom_add_rmsnorm_fwd(x2.data_ptr(), a2.data_ptr(), dtype_code(a2), w.data_ptr(), s.data_ptr(),
+                                     y.data_ptr(), rstd.data_ptr<float>(), dtype_code(x2), N, D, (float)eps,
+                                     stream_ptr(st)));
+    ctx->save_for_backward({s, w, rstd});
+    ctx->saved_data["shape"] = x.sizes().vec();
+    ctx->saved_data["st"] = st;
+    ctx->set_materialize_grads(false);
+    return {s.view(x.sizes()), y.view(x.sizes())};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list v = ctx->get_saved_variables();
+    const at::Tensor &s = v[0], &w = v[1], &rstd = v[2];
+    at::DeviceGuard guard(s.device());
+    const int64_t N = s.size(0), D = s.size(1);
+    const at::Tensor dy = grads[1].defined() ? grads[1].to(s.scalar_type()).contiguous() : at::zeros_like(s);
+    const at::Tensor dres = grads[0].defined() ? grads[0].to(s.scalar_type()).contiguous() : grads[0];
+    at::Tensor ds = at::empty_like(s), dw = at::empty_like(w);
+    at::Tensor ws = workspace(naylis_mom_rmsnorm_workspace_bytes(N, D), s);
+    check(naylis_mom_add_rmsnorm_bwd(s.data_ptr(), w.data_ptr(), rstd.data_ptr<float>(), dy.data_ptr(), ptr(dres),
+                                     ds.data_ptr(), dw.data_ptr(), ws.data_ptr(), ws.numel(), dtype_code(s), N, D,
+                                     stream_ptr(ctx->saved_data["st"].toInt())));
+    ds = ds.view(ctx->saved_data["shape"].toIntVector());
+    return {ds, ds, dw, at::Tensor(), at::Tensor()};
+  }
+};
+
+// ---- rotary embedding, causal attention, SwiGLU -----------------------------
+
+variable_list rope_call(const at::Tensor& q_in, const at::Tensor& k_in, const at::Tensor& cs, const at::Tensor& sn,
+                        bool backward, int64_t st) {
+  at::DeviceGuard guard(q_in.device());
+  const at::Tensor q = q_in.contiguous(), k = k_in.contiguous(), c = cs.contiguous(), s = sn.contiguous();
+  at::Tensor qo = at::empty_like(q), ko = at::empty_like(k);
+  check(naylis_mom_rope(q.data_ptr(), k.data_ptr(), c.data_ptr(), s.data_ptr(), qo.data_ptr(), ko.data_ptr(),
+                        dtype_code(q), backward, q.size(0), q.size(1), q.size(2), q.size(3), c.size(0),
+                        stream_ptr(st)));
+  return {qo, ko};
+}
+
+struct Rope : public Function<Rope> {
+  static variable_list forward(AutogradContext* ctx, at::Tensor q, at::Tensor k, at::Tensor cs, at::Tensor sn,
+                               int64_t st) {
+    ctx->save_for_backward({cs, sn});
+    ctx->saved_data["st"] = st;
+    return rope_call(q, k, cs, sn, false, st);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const variable_list g = rope_call(grads[0], grads[1], s[0], s[1], true, ctx->saved_data["st"].toInt());
+    return {g[0], g[1], at::Tensor(), at::Tensor(), at::Tensor()};
+  }
+};
+
+struct CausalAttention : public Function<CausalAttention> {
+  static at::Tensor forward(AutogradContext* ctx, at::Tensor q, at::Tensor k, at::Tensor v, double scale,
+                            int64_t st) {
+    at::DeviceGuard guard(q.device());
+    const int64_t B = q.size(0), S = q.size(1), H = q.size(2), hd = q.size(3);
+    q = q.contiguous();
+    k = k.contiguous();
+    v = v.contiguous();
+    at::Tensor out = at::empty_like(q), lse = at::empty({B, H, S}, f32_of(q));
+    check(naylis_mom_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
+                              (float)scale, B, S, H, hd, stream_ptr(st)));
+    ctx->save_for_backward({q, k, v, out, lse});
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["st"] = st;
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &q = s[0], &k = s[1], &v = s[2], &out = s[3], &lse = s[4];
+    at::DeviceGuard guard(q.device());
+    const at::Tensor dout = grads[0].to(q.scalar_type()).contiguous();
+    at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(lse);
+    check(naylis_mom_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
+                              dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr<float>(),
+                              (float)ctx->saved_data["scale"].toDouble(), q.size(0), q.size(1), q.size(2), q.size(3),
+                              stream_ptr(ctx->saved_data["st"].toInt())));
+    return {dq, dk, dv, at::Tensor(), at::Tensor()};
+  }
+};
+
+struct SwiGLU : public Function<SwiGLU> {
+  static at::Tensor forward(AutogradContext* ctx, at::Tensor g, at::Tensor u, int64_t st) {
+    at::DeviceGuard guard(g.device());
+    g = g.contiguous();
+    u = u.contiguous();
+    at::Tensor h = at::empty_like(g);
+    check(naylis_mom_swiglu_fwd(g.data_ptr(), u.data_ptr(), h.data_ptr(), dtype_code(g), g.numel(), stream_ptr(st)));
+    ctx->save_for_backward({g, u});
+    ctx->saved_data["st"] = st;
+    return h;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &g = s[0], &u = s[1];
+    at::DeviceGuard guard(g.device());
+    const at::Tensor dh = grads[0].to(g.scalar_type()).contiguous();
+    at::Tensor dg = at::empty_like(g), du = at::empty_like(u);
+    check(naylis_mom_swiglu_bwd(g.data_ptr(), u.data_ptr(), dh.data_ptr(), dg.data_ptr(), du.data_ptr(),
+                                dtype_code(g), g.numel(), stream_ptr(ctx->saved_data["st"].toInt())));
+    return {dg, du, at::Tensor()};
+  }
+};
+
+// ---- bias-free projections of one input -------------------------------------
+
+// y_i = x W_i^T for n <= 3 weights (w_i past n repeat w_0 and get no gradient);
+// the input gradients accumulate in the products' epilogues.
+struct SharedLinear : public Function<SharedLinear> {
+  static variable_list forward(AutogradContext* ctx, at::Tensor x, at::Tensor w0, at::Tensor w1, at::Tensor w2,
+                               int64_t n, int64_t st) {
+    const at::Tensor w[3] = {w0, w1, w2};
+    variable_list saved = {x}, y;
+    for (int64_t i = 0; i < n; ++i) {
+      saved.push_back(w[i]);
+      y.push_back(at::linear(x, w[i]));
+    }
+    ctx->save_for_backward(saved);
+    ctx->saved_data["st"] = st;
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor& x = s[0];
+    at::DeviceGuard guard(x.device());
+    void* st = stream_ptr(ctx->saved_data["st"].toInt());
+    const size_t n = s.size() - 1;
+    const at::Tensor x2 = x.reshape({-1, x.size(-1)}).contiguous();
+    variable_list r(6);
+    for (size_t i = 0; i < n; ++i) {
+      const at::Tensor& w = s[1 + i];
+      const at::Tensor dy = grads[i].reshape({-1, w.size(0)}).contiguous();
+      if (ctx->needs_input_grad(0)) {
+        if (i == 0)
+          r[0] = at::mm(dy, w);
+        else
+          r[0].addmm_(dy, w);
+      }
+      if (ctx->needs_input_grad(1 + i)) r[1 + i] = library_wgrad(x2, dy, w.scalar_type(), st);
+    }
+    if (r[0].defined()) r[0] = r[0].view(x.sizes());
+    return r;
+  }
+};
+
+// ---- the MoM layer's parts --------------------------------------------------
+
+struct Route : public Function<Route> {
+  static variable_list forward(AutogradContext* ctx, at::Tensor x, at::Tensor w_down, at::Tensor w_up,
+                               at::Tensor noise, bool has_noise, double noise_scale, int64_t top_k, bool want_h,
+                               int64_t noise_kind, int64_t st) {
+    at::DeviceGuard guard(x.device());
+    const int64_t B = x.size(0), T = x.size(1), D = x.size(2), R = w_down.size(0), E = w_up.size(0);
+    const auto f32 = f32_of(x);
+    at::Tensor logits = at::empty({B, T, E}, f32), probs = at::empty({B, T, E}, f32);
+    at::Tensor idx = at::empty({B, T, top_k}, x.options().dtype(at::kInt)), gates = at::empty({B, T, top_k}, f32);
+    at::Tensor act = at::empty({B, T, R}, f32), h;
+    if (want_h) h = at::empty({B, T, D}, f32);
+    at::Tensor ws = workspace(need(naylis_mom_router_workspace_bytes(B, T, D, R, E, top_k)), x);
+    check(naylis_mom_router_fwd(x.data_ptr(), dtype_code(x), w_down.data_ptr<float>(), w_up.data_ptr<float>(),
+                                has_noise ? noise.data_ptr<float>() : nullptr, (int)noise_kind, (float)noise_scale,
+                                logits.data_ptr<float>(), probs.data_ptr<float>(), idx.data_ptr<int32_t>(),
+                                gates.data_ptr<float>(), act.data_ptr<float>(),
+                                want_h ? h.data_ptr<float>() : nullptr, ws.data_ptr(), ws.numel(), B, T, D, R, E,
+                                top_k, stream_ptr(st)));
+    ctx->save_for_backward({x, w_down, w_up, act, probs, idx, gates});
+    ctx->saved_data["st"] = st;
+    ctx->set_materialize_grads(false);
+    if (want_h) {
+      ctx->mark_non_differentiable({idx, h});
+      return {logits, probs, idx, gates, h};
+    }
+    ctx->mark_non_differentiable({idx});
+    return {logits, probs, idx, gates};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &x = s[0], &w_down = s[1], &w_up = s[2], &act = s[3], &probs = s[4], &idx = s[5], &gates = s[6];
+    at::DeviceGuard guard(x.device());
+    const int64_t B = x.size(0), T = x.size(1), D = x.size(2), R = w_down.size(0), E = w_up.size(0),
+                  k = idx.size(2);
+    const at::Tensor d_logits = f32_or_none(grads[0]), d_gates = f32_or_none(grads[3]);
+    const ProbsGrad dp = probs_grad(grads[1], E);
+    at::Tensor dx = at::empty_like(x), dw_down = at::empty({R, D}, f32_of(x)), dw_up = at::empty({E, R}, f32_of(x));
+    at::Tensor ws = workspace(naylis_mom_router_workspace_bytes(B, T, D, R, E, k), x);
+    check(naylis_mom_router_bwd(x.data_ptr(), dtype_code(x), w_down.data_ptr<float>(), w_up.data_ptr<float>(),
+                                act.data_ptr<float>(), probs.data_ptr<float>(), idx.data_ptr<int32_t>(),
+                                gates.data_ptr<float>(), static_cast<const float*>(ptr(d_gates)),
+                                static_cast<const float*>(ptr(dp.t)), dp.stride,
+                                static_cast<const float*>(ptr(d_logits)), dx.data_ptr(), 0, dw_down.data_ptr<float>(),
+                                dw_up.data_ptr<float>(), ws.data_ptr(), ws.numel(), B, T, D, R, E, k,
+                                stream_ptr(ctx->saved_data["st"].toInt())));
+    variable_list r(10);
+    r[0] = dx;
+    r[1] = dw_down;
+    r[2] = dw_up;
+    return r;
+  }
+};
+
+struct RouterStats : public Function<RouterStats> {
+  static at::Tensor forward(AutogradContext* ctx, at::Tensor probs, at::Tensor idx, int64_t st) {
+    at::DeviceGuard guard(probs.device());
+    const int64_t E = probs.size(-1), N = probs.numel() / E;
+    at::Tensor stats = at::empty({2 * E + 3}, probs.options());
+    at::Tensor ws = workspace(need(naylis_mom_router_stats_workspace_bytes(N, E)), probs);
+    check(naylis_mom_router_stats(probs.data_ptr<float>(), idx.data_ptr<int32_t>(), stats.data_ptr<float>(),
+                                  ws.data_ptr(), ws.numel(), N, E, idx.size(-1), stream_ptr(st)));
+    ctx->save_for_backward({stats});
+    ctx->saved_data["shape"] = probs.sizes().vec();
+    return stats;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const at::Tensor stats = ctx->get_saved_variables()[0];
+    const std::vector<int64_t> shape = ctx->saved_data["shape"].toIntVector();
+    const int64_t E = shape.back();
+    int64_t N = 1;
+    for (size_t i = 0; i + 1 < shape.size(); ++i) N *= shape[i];
+    // d mean_prob_e = d_stats[e] + d_aux E frac_e; every token gets 1 / N of it
+    const at::Tensor& d = grads[0];
+    const at::Tensor row = (d.narrow(0, 0, E) + d.select(0, 2 * E) * E * stats.narrow(0, E, E)) / N;
+    return {row.expand(shape), at::Tensor(), at::Tensor()};
+  }
+};
+
+struct Read : public Function<Read> {
+  static at::Tensor forward(AutogradContext* ctx, at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor idx,
+                            at::Tensor gates, int64_t num_blocks, int64_t block_size, int64_t st) {
+    at::DeviceGuard guard(q.device());
+    const int64_t B = q.size(0), S = q.size(1), H = q.size(2), HD = q.size(3), top_k = idx.size(-1);
+    at::Tensor out = at::empty_like(q), side;
+    const size_t side_bytes = naylis_mom_read_side_bytes(B, S, H, HD, num_blocks, block_size, top_k);
+    if (side_bytes > 0) side = workspace(side_bytes, q);
+    at::Tensor lse = at::empty({H, B, S}, f32_of(q));
+    const int64_t words = naylis_mom_read_order_words(B, S, num_blocks, top_k);
+    if (words <= 0) check(NAYLIS_ERR_ARG);
+    at::Tensor order = at::empty({words}, idx.options());
+    at::Tensor ows = workspace(naylis_mom_read_order_workspace_bytes(B, S, num_blocks, top_k), q);
+    check(naylis_mom_read_order(idx.data_ptr<int32_t>(), order.data_ptr<int32_t>(), ows.data_ptr(), ows.numel(), B, S,
+                                num_blocks, top_k, stream_ptr(st)));
+    check(naylis_mom_read_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), idx.data_ptr<int32_t>(),
+                              gates.data_ptr<float>(), order.data_ptr<int32_t>(), out.data_ptr(), ptr(side),
+                              lse.data_ptr<float>(), nullptr, 0, B, S, H, HD, num_blocks, block_size, top_k,
+                              stream_ptr(st)));
+    ctx->save_for_backward({q, k, v, idx, gates, order, out, side, lse});
+    ctx->saved_data["geom"] = std::vector<int64_t>{num_blocks, block_size, st};
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &q = s[0], &k = s[1], &v = s[2], &idx = s[3], &gates = s[4], &order = s[5], &out = s[6],
+                     &side = s[7], &lse = s[8];
+    const std::vector<int64_t> geom = ctx->saved_data["geom"].toIntVector();
+    at::DeviceGuard guard(q.device());
+    const int64_t B = q.size(0), S = q.size(1), H = q.size(2), HD = q.size(3), top_k = idx.size(-1);
+    const at::Tensor dout = grads[0].contiguous().to(q.scalar_type());
+    at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), dg = at::empty_like(gates);
+    at::Tensor ws = workspace(need(naylis_mom_read_workspace_bytes(B, S, H, HD, geom[0], geom[1], top_k)), q);
+    check(naylis_mom_read_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), idx.data_ptr<int32_t>(),
+                              gates.data_ptr<float>(), order.data_ptr<int32_t>(), out.data_ptr(), ptr(side),
+                              lse.data_ptr<float>(), dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                              dg.data_ptr<float>(), ws.data_ptr(), ws.numel(), B, S, H, HD, geom[0], geom[1], top_k,
+                              stream_ptr(geom[2])));
+    return {dq, dk, dv, at::Tensor(), dg, at::Tensor(), at::Tensor(), at::Tensor()};
+  }
+};
+
+struct GatedLinear : public Function<GatedLinear> {
+  static at::Tensor forward(AutogradContext* ctx, at::Tensor out, at::Tensor w_o, at::Tensor s, int64_t st) {
+    at::DeviceGuard guard(out.device());
+    const auto [y2, w_os] = gated_linear_forward(out.reshape({-1, w_o.size(1)}), w_o, s, stream_ptr(st));
+    ctx->save_for_backward({out, w_o, w_os, s});
+    ctx->saved_data["st"] = st;
+    std::vector<int64_t> shape = out.sizes().vec();
+    shape.back() = w_o.size(0);
+    return y2.view(shape);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list v = ctx->get_saved_variables();
+    const at::Tensor &out = v[0], &w_o = v[1], &w_os = v[2], &s = v[3];
+    at::DeviceGuard guard(out.device());
+    const GatedGrads g = gated_linear_backward(grads[0].reshape({-1, w_o.size(0)}), out.reshape({-1, w_o.size(1)}),
+                                               w_o, w_os, s, stream_ptr(ctx->saved_data["st"].toInt()));
+    return {g.dout2.view(out.sizes()), g.dw_o, g.ds.view(s.sizes()), at::Tensor()};
+  }
+};
+
+// ---- LM loss ----------------------------------------------------------------
+
+struct Xent : public Function<Xent> {
+  static at::Tensor forward(AutogradContext* ctx, at::Tensor logits, at::Tensor labels, int64_t ignore_index,
+                            int64_t st) {
+    at::DeviceGuard guard(logits.device());
+    logits = logits.contiguous();
+    labels = labels.to(at::kLong).contiguous();
+    const int64_t N = logits.size(0), V = logits.size(1);
+    at::Tensor loss = at::empty({N}, f32_of(logits)), lse = at::empty({N}, f32_of(logits));
+    check(naylis_mom_xent_fwd(logits.data_ptr(), labels.data_ptr<int64_t>(), loss.data_ptr<float>(),
+                              lse.data_ptr<float>(), N, V, ignore_index, stream_ptr(st)));
+    ctx->save_for_backward({logits, labels, lse});
+    ctx->saved_data["args"] = std::vector<int64_t>{ignore_index, st};
+    return loss;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const at::Tensor &logits = s[0], &labels = s[1], &lse = s[2];
+    const std::vector<int64_t> args = ctx->saved_data["args"].toIntVector();
+    at::DeviceGuard guard(logits.device());
+    const int64_t N = logits.size(0), V = logits.size(1);
+    at::Tensor g = grads[0].to(at::kFloat);
+    const bool one = g.dim() == 1 && g.stride(0) == 0;  // one gradient for every row (the sum's backward)
+    if (!one) g = g.contiguous();
+    at::Tensor dlogits = at::empty_like(logits);
+    check(naylis_mom_xent_bwd(logits.data_ptr(), labels.data_ptr<int64_t>(), lse.data_ptr<float>(),
+                              g.data_ptr<float>(), one ? 0 : 1, dlogits.data_ptr(), N, V, args[0],
+                              stream_ptr(args[1])));
+    return {dlogits, at::Tensor(), at::Tensor(), at::Tensor()};
+  }
+};
+
+// ---- decode -----------------------------------------------------------------
+
+void require(bool ok, const char* what) {
+  if (!ok) throw std::runtime_error(what);
+}
+
+std::vector<at::Tensor> decode_step(at::Tensor sum_state, at::Tensor t_prev, at::Tensor x_new, at::Tensor w_down,
+                                    at::Tensor w_up, int64_t top_k, at::Tensor q_new, const at::Tensor& k8,
+                                    const at::Tensor& v8, const at::Tensor& k_scale, const at::Tensor& v_scale,
+                                    int64_t num_blocks, int64_t block_size, c10::optional<at::Tensor> out_state,
+                                    int64_t st) {
+  require(x_new.dim() == 2 && q_new.dim() == 3, "decode_step: x_new must be (B, D) and q_new (B, H, head_dim)");
+  const int64_t B = x_new.size(0), D = x_new.size(1), H = q_new.size(1), R = w_down.size(0), E = w_up.size(0);
+  if (E != num_blocks)
+    throw std::runtime_error("decode_step: the router has " + std::to_string(E) + " experts but the bank " +
+                             std::to_string(num_blocks) + " blocks");
+  require(q_new.size(0) == B && H > 0 && q_new.size(2) == D / H && q_new.scalar_type() == at::kBFloat16,
+          "decode_step: q_new must be (B, H, D / H) bf16");
+  require(x_new.scalar_type() == at::kBFloat16 || x_new.scalar_type() == at::kFloat,
+          "decode_step: x_new must be bf16 or fp32");
+  require(k8.dim() == 2 && k8.size(0) == num_blocks * block_size && k8.size(1) == D,
+          "decode_step: the bank's shape does not match num_blocks * block_size x D");
+  sum_state = sum_state.to(at::kDouble).contiguous();
+  t_prev = t_prev.to(x_new.device(), at::kInt).contiguous();
+  at::Tensor state;
+  if (out_state.has_value()) {
+    state = *out_state;
+    require(state.data_ptr() != sum_state.data_ptr() && state.scalar_type() == at::kDouble,
+            "decode_step: out_state must be a separate fp64 buffer");
+  } else {
+    state = at::empty_like(sum_state);
+  }
+  x_new = x_new.contiguous();
+  q_new = q_new.contiguous();
+  w_down = w_down.to(at::kFloat).contiguous();
+  w_up = w_up.to(at::kFloat).contiguous();
+  at::DeviceGuard guard(x_new.device());
+  at::Tensor out = at::empty({B, H, D / H}, x_new.options().dtype(at::kBFloat16));
+  at::Tensor idx = at::empty({B, top_k}, x_new.options().dtype(at::kInt));
+  at::Tensor gates = at::empty({B, top_k}, f32_of(x_new));
+  check(naylis_mom_decode_step(sum_state.data_ptr<double>(), state.data_ptr<double>(), t_prev.data_ptr<int32_t>(),
+                               x_new.data_ptr(), dtype_code(x_new), w_down.data_ptr<float>(),
+                               w_up.data_ptr<float>(), q_new.data_ptr(), static_cast<const uint8_t*>(k8.data_ptr()),
+                               static_cast<const uint8_t*>(v8.data_ptr()), k_scale.data_ptr<float>(),
+                               v_scale.data_ptr<float>(), out.data_ptr(), idx.data_ptr<int32_t>(),
+                               gates.data_ptr<float>(), B, D, H, R, E, block_size, top_k, stream_ptr(st)));
+  return {out, state, idx, gates};
+}
+
+}  // namespace
+
+void bind_nodes(pybind11::module_& m) {
+  namespace py = pybind11;
+  py::register_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const StatusError& e) {
+      py::object type = py::module_::import("naylis_amd._lib").attr("NaylisError");
+      PyErr_SetObject(type.ptr(), type(e.code, e.what()).ptr());
+    }
+  });
+  using at::Tensor;
+  m.def("rms_norm", [](Tensor x, Tensor w, double eps, int64_t st) { return RmsNorm::apply(x, w, eps, st); });
+  m.def("add_rms_norm",
+        [](Tensor x, Tensor a, Tensor w, double eps, int64_t st) { return AddRmsNorm::apply(x, a, w, eps, st); });
+  m.def("rope", [](Tensor q, Tensor k, Tensor c, Tensor s, int64_t st) { return Rope::apply(q, k, c, s, st); });
+  m.def("causal_attention",
+        [](Tensor q, Tensor k, Tensor v, double scale, int64_t st) { return CausalAttention::apply(q, k, v, scale, st); });
+  m.def("swiglu", [](Tensor g, Tensor u, int64_t st) { return SwiGLU::apply(g, u, st); });
+  m.def("shared_linear", [](Tensor x, std::vector<Tensor> w, int64_t st) {
+    TORCH_CHECK(!w.empty() && w.size() <= 3, "shared_linear: one to three weights");
+    return SharedLinear::apply(x, w[0], w[w.size() > 1 ? 1 : 0], w[w.size() > 2 ? 2 : 0], (int64_t)w.size(), st);
+  });
+  m.def("route", [](Tensor x, Tensor wd, Tensor wu, c10::optional<Tensor> noise, double noise_scale, int64_t top_k,
+                    bool want_h, int64_t kind, int64_t st) {
+    return Route::apply(x, wd, wu, noise.has_value() ? *noise : x, noise.has_value(), noise_scale, top_k, want_h, kind,
+                        st);
+  });
+  m.def("router_stats", [](Tensor probs, Tensor idx, int64_t st) { return RouterStats::apply(probs, idx, st); });
+  m.def("read", [](Tensor q, Tensor k, Tensor v, Tensor idx, Tensor gates, int64_t nb, int64_t bs, int64_t st) {
+    return Read::apply(q, k, v, idx, gates, nb, bs, st);
+  });
+  m.def("gated_linear", [](Tensor out, Tensor w, Tensor s, int64_t st) { return GatedLinear::apply(out, w, s, st); });
+  m.def("xent", [](Tensor logits, Tensor labels, int64_t ignore, int64_t st) {
+    return Xent::apply(logits, labels, ignore, st);
+  });
+  m.def("decode_step", &decode_step);
+}
+
+}  // namespace naylis_ext

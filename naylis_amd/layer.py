@@ -13,10 +13,10 @@ between the two unchanged.  The forward is
 
 q_proj / o_proj run their forward and input gradient as torch GEMMs
 (hipBLASLt) and their weight gradient on the library's split-K GEMM.  In the
-common training case (bf16 activations and projection weights, no gradient
-checkpointing) the whole forward is one autograd node
-(``mom_kernels.hip_layer``) whose backward orders the library calls so the
-router's input gradient accumulates into the q projection's.  There is one backend: the
+common training case (bf16 activations and projection weights) the whole
+forward is one autograd node (``mom_kernels.hip_layer``) whose backward orders
+the library calls so the router's input gradient accumulates into the q
+projection's; gradient checkpointing is a mode of it.  There is one backend: the
 HIP kernels (``use_kernel`` is accepted for signature compatibility).  The
 eager SDPA path of model.py:262-275 is the parity oracle and lives in
 ``oracle/``, outside the product.
@@ -27,6 +27,7 @@ import torch
 import torch.nn as nn
 
 from . import mom_kernels
+from .mom_kernels import hip_layer
 from .mom_kernels.hip_layer import fused_layer_supported, mom_layer
 
 __all__ = ["MoMLayer", "mom_aux_loss"]
@@ -110,16 +111,17 @@ class MoMLayer(nn.Module):
             # g = -log(-log(u + 1e-9) + 1e-9) and logits + noise_scale * g
             noise = torch.rand((B, S, self.num_blocks), device=x.device, dtype=torch.float32)
         ckpt = self.mom_grad_ckpt and self.training and torch.is_grad_enabled()
-        if not ckpt and fused_layer_supported(x, M_blocks, self.router_down.weight, self.router_up.weight,
-                                              self.q_proj.weight, self.k_proj.weight, self.v_proj.weight,
-                                              self.o_proj.weight, self.mom_scale, bank_kv):
+        if (not ckpt or hip_layer.cpp_node()) and fused_layer_supported(x, M_blocks, self.router_down.weight, self.router_up.weight,
+                                                                       self.q_proj.weight, self.k_proj.weight,
+                                                                       self.v_proj.weight, self.o_proj.weight,
+                                                                       self.mom_scale, bank_kv):
             # one autograd node for router + bank + q + read + o + ReZero
             y, router_probs, top_idx = mom_layer(
                 x, M_blocks, self.router_down.weight, self.router_up.weight, self.q_proj.weight,
                 self.k_proj.weight, self.v_proj.weight, self.o_proj.weight, self.mom_scale,
                 n_heads=self.n_heads, num_blocks=self.num_blocks, block_size=self.block_size,
                 top_k=self.top_blocks, noise=noise, noise_scale=self.noise_scale, noise_is_uniform=True,
-                bank_kv=bank_kv)
+                bank_kv=bank_kv, ckpt=ckpt)
             if self.training:
                 # plain attributes (not parameters, buffers or modules): set
                 # without nn.Module.__setattr__'s registry checks

@@ -19,7 +19,12 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
+from .hip_bank import mom_bank_kv, mom_bank_kv_grouped
+from .hip_decode import decode_step, quantize_bank_fp8
+from .hip_linear import mom_linear
 from .hip_read import mom_read as _hip_mom_read
+from .hip_rezero import mom_gated_linear, mom_rezero
+from .hip_router import mom_route, mom_router_stats
 
 __all__ = ["HAS_HIP", "preflight", "resolve_mode", "mom_read", "announce", "mom_route",
            "mom_bank_kv", "mom_bank_kv_grouped", "mom_linear", "mom_rezero", "mom_gated_linear", "has_hip", "quantize_bank_fp8", "decode_step",
@@ -96,48 +101,3 @@ def announce(backend: str) -> None:
             print("[MoM] use_kernel=true -> backend 'hip': gfx950 flash read with "
                   "in-register gate bias and block skipping, fused prefix-mean router, "
                   "MFMA bank K/V; deterministic backward.")
-
-
-def mom_route(*args, **kwargs):
-    from .hip_router import mom_route as _route
-    return _route(*args, **kwargs)
-
-
-def mom_router_stats(*args, **kwargs):
-    from .hip_router import mom_router_stats as _stats
-    return _stats(*args, **kwargs)
-
-
-def mom_bank_kv(*args, **kwargs):
-    from .hip_bank import mom_bank_kv as _bank
-    return _bank(*args, **kwargs)
-
-
-def mom_bank_kv_grouped(*args, **kwargs):
-    from .hip_bank import mom_bank_kv_grouped as _grouped
-    return _grouped(*args, **kwargs)
-
-
-def mom_linear(*args, **kwargs):
-    from .hip_linear import mom_linear as _linear
-    return _linear(*args, **kwargs)
-
-
-def mom_rezero(*args, **kwargs):
-    from .hip_rezero import mom_rezero as _rezero
-    return _rezero(*args, **kwargs)
-
-
-def mom_gated_linear(*args, **kwargs):
-    from .hip_rezero import mom_gated_linear as _gated
-    return _gated(*args, **kwargs)
-
-
-def quantize_bank_fp8(*args, **kwargs):
-    from .hip_decode import quantize_bank_fp8 as _quant
-    return _quant(*args, **kwargs)
-
-
-def decode_step(*args, **kwargs):
-    from .hip_decode import decode_step as _step
-    return _step(*args, **kwargs)

@@ -16,9 +16,7 @@ from typing import NamedTuple
 
 import torch
 
-from .. import _lib
-
-_DT = {torch.float32: 0, torch.bfloat16: 1}
+from .. import _lib, _torch_ext
 
 
 class Fp8Bank(NamedTuple):
@@ -70,38 +68,7 @@ def decode_step(sum_state, t_prev, x_new, w_down, w_up, top_k, q_new, bank: Fp8B
     given (it must not be sum_state: every workgroup of a sequence reads the
     old state); the caller ping-pongs two buffers across steps.
     """
-    lib = _lib.load()
-    if x_new.dim() != 2 or q_new.dim() != 3:
-        raise RuntimeError("decode_step: x_new must be (B, D) and q_new (B, H, head_dim)")
-    B, D = x_new.shape
-    H = q_new.shape[1]
-    R, E = w_down.shape[0], w_up.shape[0]
-    if E != num_blocks:
-        raise RuntimeError(f"decode_step: the router has {E} experts but the bank {num_blocks} blocks")
-    if q_new.shape != (B, H, D // H) or q_new.dtype != torch.bfloat16:
-        raise RuntimeError("decode_step: q_new must be (B, H, D / H) bf16")
-    if x_new.dtype not in _DT:
-        raise RuntimeError(f"decode_step: x_new dtype {x_new.dtype} (bf16 or fp32 expected)")
-    if bank.k8.shape != (num_blocks * block_size, D):
-        raise RuntimeError("decode_step: the bank's shape does not match num_blocks * block_size x D")
-    dev = x_new.device
-    sum_state = sum_state.to(torch.float64).contiguous()
-    t_prev = t_prev.to(device=dev, dtype=torch.int32).contiguous()
-    if out_state is None:
-        out_state = torch.empty_like(sum_state)
-    elif out_state.data_ptr() == sum_state.data_ptr() or out_state.dtype != torch.float64:
-        raise RuntimeError("decode_step: out_state must be a separate fp64 buffer")
-    x_new = x_new.contiguous()
-    q_new = q_new.contiguous()
-    w_down = w_down.float().contiguous()
-    w_up = w_up.float().contiguous()
-    out = torch.empty((B, H, D // H), device=dev, dtype=torch.bfloat16)
-    top_idx = torch.empty((B, top_k), device=dev, dtype=torch.int32)
-    gates = torch.empty((B, top_k), device=dev, dtype=torch.float32)
-    with _lib.on_device(dev):
-        _lib.check(lib.naylis_mom_decode_step(
-            sum_state.data_ptr(), out_state.data_ptr(), t_prev.data_ptr(), x_new.data_ptr(), _DT[x_new.dtype],
-            w_down.data_ptr(), w_up.data_ptr(), q_new.data_ptr(), bank.k8.data_ptr(), bank.v8.data_ptr(),
-            bank.k_scale.data_ptr(), bank.v_scale.data_ptr(), out.data_ptr(), top_idx.data_ptr(), gates.data_ptr(),
-            B, D, H, R, E, block_size, top_k, _lib.stream_of(dev)))
-    return out, out_state, top_idx, gates
+    out, state, top_idx, gates = _torch_ext.load().decode_step(
+        sum_state, t_prev, x_new, w_down, w_up, int(top_k), q_new, bank.k8, bank.v8, bank.k_scale, bank.v_scale,
+        int(num_blocks), int(block_size), out_state, _lib.stream_of(x_new.device))
+    return out, state, top_idx, gates

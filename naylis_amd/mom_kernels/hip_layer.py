@@ -15,7 +15,7 @@ out (s W_o)^T, so the layer's fp32 output is one GEMM with an fp32 result
 in fp32 and gets dW_o = s dW' and ds = sum(dW' W_o) from one pass over the
 weight.  Results equal the modular path's to bf16 rounding (W' is rounded
 where the modular path rounds o W_o^T); the modular Functions stay the
-public drop-in API (mom_read etc.) and serve gradient checkpointing.
+public drop-in API (mom_read etc.).
 
 The node's host work -- about fifteen library and torch calls each way --
 runs in C++ (the torch extension of csrc/torch_layer.cpp, one call per
@@ -41,6 +41,11 @@ USE_TORCH_EXT = True
 # the node itself in C++ (the extension's mom_layer: a torch::autograd::Function
 # whose forward / backward make the calls of MomLayerFunction's extension path)
 USE_CPP_NODE = True
+
+
+def cpp_node():
+    """True when ``mom_layer`` runs as the C++ node (which alone checkpoints)."""
+    return USE_TORCH_EXT and USE_CPP_NODE
 
 
 def _ws(nbytes, dev):
@@ -225,21 +230,25 @@ class MomLayerFunction(torch.autograd.Function):
 
 
 def mom_layer(x, M_blocks, w_down, w_up, w_q, w_k, w_v, w_o, scale, *, n_heads, num_blocks, block_size, top_k,
-              noise=None, noise_scale=1.0, noise_is_uniform=False, bank_kv=None):
+              noise=None, noise_scale=1.0, noise_is_uniform=False, bank_kv=None, ckpt=False):
     """The fused layer node; callers check fused_layer_supported() first.
     ``noise_is_uniform``: noise is the uniform draw and the router kernel
     applies the Gumbel transform.  ``bank_kv``: the bank's (K, V) projected by
     the caller (M_blocks, w_k and w_v then get no gradient here; K and V do).
-    Returns (y fp32, router probs, top_idx int32)."""
+    ``ckpt``: gradient checkpointing -- the node keeps the read's inputs only,
+    and its backward runs the q projection, bank K/V, token order and read
+    again (the same bits).  Returns (y fp32, router probs, top_idx int32)."""
     if noise is not None:
         noise = noise.detach().float().contiguous()
     k_ext, v_ext = bank_kv if bank_kv is not None else (None, None)
-    if USE_TORCH_EXT and USE_CPP_NODE:
+    if cpp_node():
         y, probs, top_idx = _torch_ext.load().mom_layer(
             x, M_blocks if bank_kv is None else None, w_down.float().contiguous(), w_up.float().contiguous(), w_q,
             w_k, w_v, w_o, scale, noise, float(noise_scale), int(n_heads), int(num_blocks), int(block_size),
-            int(top_k), 1 if noise_is_uniform else 0, k_ext, v_ext, _lib.stream_of(x.device))
+            int(top_k), 1 if noise_is_uniform else 0, k_ext, v_ext, bool(ckpt), _lib.stream_of(x.device))
         return y, probs, top_idx
+    if ckpt:
+        raise RuntimeError("mom_layer: gradient checkpointing is a mode of the C++ node")
     return MomLayerFunction.apply(x, M_blocks if bank_kv is None else None, w_down.float().contiguous(),
                                   w_up.float().contiguous(), w_q, w_k, w_v, w_o, scale, noise, float(noise_scale),
                                   (int(n_heads), int(num_blocks), int(block_size), int(top_k),

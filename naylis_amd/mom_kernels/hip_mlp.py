@@ -11,7 +11,7 @@ from __future__ import annotations
 import torch
 from transformers.models.llama.modeling_llama import LlamaMLP
 
-from .. import _lib
+from .. import _lib, _torch_ext
 from .hip_linear import shared_input_linear
 
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -22,39 +22,12 @@ def swiglu_supported(g, u):
             and u.shape == g.shape and u.device == g.device and g.numel() % 8 == 0)
 
 
-class SwiGLUFunction(torch.autograd.Function):
-
-    @staticmethod
-    def forward(ctx, g, u):
-        lib = _lib.load()
-        g = g.contiguous()
-        u = u.contiguous()
-        h = torch.empty_like(g)
-        with _lib.on_device(g.device):
-            _lib.check(lib.naylis_mom_swiglu_fwd(g.data_ptr(), u.data_ptr(), h.data_ptr(), _DT[g.dtype], g.numel(),
-                                                 _lib.stream_of(g.device)))
-        ctx.save_for_backward(g, u)
-        return h
-
-    @staticmethod
-    def backward(ctx, dh):
-        lib = _lib.load()
-        g, u = ctx.saved_tensors
-        dh = dh.to(g.dtype).contiguous()
-        dg = torch.empty_like(g)
-        du = torch.empty_like(u)
-        with _lib.on_device(g.device):
-            _lib.check(lib.naylis_mom_swiglu_bwd(g.data_ptr(), u.data_ptr(), dh.data_ptr(), dg.data_ptr(),
-                                                 du.data_ptr(), _DT[g.dtype], g.numel(), _lib.stream_of(g.device)))
-        return dg, du
-
-
 def swiglu(g, u):
     """silu(g) * u in one pass; raises when ``swiglu_supported`` is false."""
     if not swiglu_supported(g, u):
         raise RuntimeError(f"swiglu: unsupported inputs {tuple(g.shape)} {g.dtype} / {tuple(u.shape)} {u.dtype} "
                            f"on {g.device}")
-    return SwiGLUFunction.apply(g, u)
+    return _torch_ext.load().swiglu(g, u, _lib.stream_of(g.device))
 
 
 class NaylisMLP(LlamaMLP):

@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import torch
 
-from .. import _lib
+from .. import _lib, _torch_ext
 
 
 def _workspace(nbytes, device):
@@ -37,64 +37,6 @@ def read_order(top_idx, num_blocks):
                                        B, S, num_blocks, topk, _lib.stream_of(dev))
     _lib.check(rc)
     return order
-
-
-class MomReadFunction(torch.autograd.Function):
-    """Forward computes the token order (tokens grouped by selected blocks, or
-    sequence order when that does not pay, plus the pair plan) and saves (q,
-    k, v, top_idx, top_gates, order, o, the pair path's side buffer when
-    it is used, lse); backward runs the library's backward with the same order."""
-
-    @staticmethod
-    def forward(ctx, q_sh, k, v, top_idx, top_gates, num_blocks, block_size):
-        lib = _lib.load()
-        B, S, H, HD = q_sh.shape
-        topk = top_idx.shape[-1]
-        dev = q_sh.device
-        out = torch.empty_like(q_sh)
-        side = read_side(lib, out, num_blocks, block_size, topk)
-        lse = torch.empty((H, B, S), device=dev, dtype=torch.float32)
-        order = read_order(top_idx, num_blocks)  # mode word + table (+ pair plan)
-        with _lib.on_device(dev):
-            st = _lib.stream_of(dev)
-            rc = lib.naylis_mom_read_fwd(
-                q_sh.data_ptr(), k.data_ptr(), v.data_ptr(), top_idx.data_ptr(), top_gates.data_ptr(),
-                order.data_ptr(), out.data_ptr(), _ptr(side), lse.data_ptr(), None, 0,
-                B, S, H, HD, num_blocks, block_size, topk, st)
-        _lib.check(rc)
-        ctx.save_for_backward(q_sh, k, v, top_idx, top_gates, order, out, side, lse)
-        ctx.geom = (num_blocks, block_size)
-        return out
-
-    @staticmethod
-    def backward(ctx, dout):
-        lib = _lib.load()
-        q_sh, k, v, top_idx, top_gates, order, out, side, lse = ctx.saved_tensors
-        num_blocks, block_size = ctx.geom
-        B, S, H, HD = q_sh.shape
-        topk = top_idx.shape[-1]
-        dev = q_sh.device
-        dout = dout.contiguous()
-        if dout.dtype != q_sh.dtype:
-            dout = dout.to(q_sh.dtype)
-        dq = torch.empty_like(q_sh)
-        dk = torch.empty_like(k)
-        dv = torch.empty_like(v)
-        dgates = torch.empty_like(top_gates)
-        nbytes = lib.naylis_mom_read_workspace_bytes(B, S, H, HD, num_blocks, block_size, topk)
-        if nbytes == 0:
-            _lib.check(_lib.NAYLIS_ERR_ARG)
-        ws = _workspace(nbytes, dev)
-        with _lib.on_device(dev):
-            rc = lib.naylis_mom_read_bwd(
-                q_sh.data_ptr(), k.data_ptr(), v.data_ptr(), top_idx.data_ptr(), top_gates.data_ptr(),
-                order.data_ptr(), out.data_ptr(), _ptr(side), lse.data_ptr(), dout.data_ptr(), dq.data_ptr(),
-                dk.data_ptr(),
-                dv.data_ptr(),
-                dgates.data_ptr(), ws.data_ptr(), ws.numel(),
-                B, S, H, HD, num_blocks, block_size, topk, _lib.stream_of(dev))
-        _lib.check(rc)
-        return dq, dk, dv, None, dgates, None, None
 
 
 def read_side(lib, out, num_blocks, block_size, top_k):
@@ -146,4 +88,5 @@ def mom_read(q_sh, k, v, top_idx, top_gates, *, num_blocks, block_size):
     v = v.contiguous()
     top_idx = top_idx.to(torch.int32).contiguous()
     top_gates = top_gates.float().contiguous()
-    return MomReadFunction.apply(q_sh, k, v, top_idx, top_gates, int(num_blocks), int(block_size))
+    return _torch_ext.load().read(q_sh, k, v, top_idx, top_gates, int(num_blocks), int(block_size),
+                                  _lib.stream_of(q_sh.device))

@@ -20,7 +20,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
-from .. import _lib
+from .. import _lib, _torch_ext
 from .hip_linear import library_wgrad
 
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -104,29 +104,6 @@ def mom_rezero(z, s):
     return s * z
 
 
-class MomGatedLinearFunction(torch.autograd.Function):
-    """y = s * (out W_o^T) in fp32, as out (s W_o)^T (see the module notes)."""
-
-    @staticmethod
-    def forward(ctx, out, w_o, s):
-        lib = _lib.load()
-        D = w_o.shape[1]
-        with _lib.on_device(out.device):
-            y2, w_os = gated_linear_forward(lib, out.reshape(-1, D), w_o, s, _lib.stream_of(out.device))
-        ctx.save_for_backward(out, w_o, w_os, s)
-        return y2.view(*out.shape[:-1], w_o.shape[0])
-
-    @staticmethod
-    def backward(ctx, dy):
-        lib = _lib.load()
-        out, w_o, w_os, s = ctx.saved_tensors
-        D = w_o.shape[1]
-        with _lib.on_device(out.device):
-            dout2, dw_o, ds = gated_linear_backward(lib, dy.reshape(-1, w_o.shape[0]), out.reshape(-1, D), w_o, w_os,
-                                                    s, _lib.stream_of(out.device))
-        return dout2.view(out.shape), dw_o, ds.view(s.shape)
-
-
 def mom_gated_linear(out, w_o, s):
     """s * (out W_o^T) for the layer's o projection and ReZero gate
     (model.py:251, 239): one GEMM with the gate folded into the weight, for
@@ -138,5 +115,5 @@ def mom_gated_linear(out, w_o, s):
             and w_o.dtype == torch.bfloat16 and s.dtype == torch.float32 and s.numel() == 1
             and out.device == w_o.device == s.device and out.shape[-1] == D_in and D_in % 8 == 0
             and D_out % 8 == 0 and (out.numel() // D_in) % 8 == 0):
-        return MomGatedLinearFunction.apply(out.contiguous(), w_o, s)
+        return _torch_ext.load().gated_linear(out.contiguous(), w_o, s, _lib.stream_of(out.device))
     return s * F.linear(out, w_o)

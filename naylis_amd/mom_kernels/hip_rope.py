@@ -13,7 +13,7 @@ from __future__ import annotations
 import torch
 from transformers.models.llama.modeling_llama import ALL_ATTENTION_FUNCTIONS, LlamaAttention, eager_attention_forward
 
-from .. import _lib
+from .. import _lib, _torch_ext
 from .hip_attention import causal_attention, causal_attention_supported
 from .hip_linear import shared_input_linear
 
@@ -39,47 +39,14 @@ def rope_supported(q, k, cos, sin):
     return _shape_ok(q.dtype, q.device, B, S, hd, cos, sin)
 
 
-def _launch(q, k, cos, sin, backward):
-    lib = _lib.load()
-    B, S, H, hd = q.shape
-    q = q.contiguous()
-    k = k.contiguous()
-    cos = cos.contiguous()
-    sin = sin.contiguous()
-    qo = torch.empty_like(q)
-    ko = torch.empty_like(k)
-    with _lib.on_device(q.device):
-        _lib.check(lib.naylis_mom_rope(q.data_ptr(), k.data_ptr(), cos.data_ptr(), sin.data_ptr(), qo.data_ptr(),
-                                       ko.data_ptr(), _DT[q.dtype], int(backward), B, S, H, hd, cos.shape[0],
-                                       _lib.stream_of(q.device)))
-    return qo, ko
-
-
-class RopeFunction(torch.autograd.Function):
-
-    @staticmethod
-    def forward(ctx, q, k, cos, sin):
-        ctx.save_for_backward(cos, sin)
-        return _launch(q, k, cos, sin, False)
-
-    @staticmethod
-    def backward(ctx, dq, dk):
-        cos, sin = ctx.saved_tensors
-        if dq is None:
-            dq = torch.zeros_like(dk)
-        if dk is None:
-            dk = torch.zeros_like(dq)
-        gq, gk = _launch(dq, dk, cos, sin, True)
-        return gq, gk, None, None
-
-
 def rope(q, k, cos, sin):
     """(q', k') = rotary embedding of q, k (B, S, H, hd) with cos / sin
     (1 or B, S, hd); raises when ``rope_supported`` is false."""
     if not rope_supported(q, k, cos, sin):
         raise RuntimeError(f"rope: unsupported inputs q {tuple(q.shape)} {q.dtype} on {q.device}, cos "
                            f"{tuple(cos.shape)} {cos.dtype}")
-    return RopeFunction.apply(q, k, cos.detach(), sin.detach())
+    q, k = _torch_ext.load().rope(q, k, cos.detach(), sin.detach(), _lib.stream_of(q.device))
+    return q, k
 
 
 class NaylisAttention(LlamaAttention):

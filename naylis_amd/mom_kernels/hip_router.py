@@ -16,7 +16,7 @@ from __future__ import annotations
 
 import torch
 
-from .. import _lib
+from .. import _lib, _torch_ext
 
 _DT = {torch.float32: 0, torch.bfloat16: 1}
 NOISE_ADDITIVE, NOISE_GUMBEL_UNIFORM = 0, 1
@@ -34,72 +34,6 @@ def d_probs_arg(d_probs, E):
         return d_probs, d_probs.data_ptr(), 0
     dense = d_probs.float().contiguous()
     return dense, dense.data_ptr(), E
-
-
-class MomRouteFunction(torch.autograd.Function):
-
-    @staticmethod
-    def forward(ctx, x, w_down, w_up, noise, noise_scale, top_k, want_h, noise_kind=NOISE_ADDITIVE):
-        lib = _lib.load()
-        B, T, D = x.shape
-        R, E = w_down.shape[0], w_up.shape[0]
-        dev = x.device
-        f32 = dict(device=dev, dtype=torch.float32)
-        logits = torch.empty((B, T, E), **f32)
-        probs = torch.empty((B, T, E), **f32)
-        top_idx = torch.empty((B, T, top_k), device=dev, dtype=torch.int32)
-        top_gates = torch.empty((B, T, top_k), **f32)
-        act = torch.empty((B, T, R), **f32)
-        h = torch.empty((B, T, D), **f32) if want_h else None
-        nbytes = lib.naylis_mom_router_workspace_bytes(B, T, D, R, E, top_k)
-        if nbytes == 0:
-            _lib.check(_lib.NAYLIS_ERR_ARG)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-        with _lib.on_device(dev):
-            rc = lib.naylis_mom_router_fwd(
-                x.data_ptr(), _DT[x.dtype], w_down.data_ptr(), w_up.data_ptr(),
-                noise.data_ptr() if noise is not None else None, int(noise_kind), float(noise_scale),
-                logits.data_ptr(), probs.data_ptr(), top_idx.data_ptr(), top_gates.data_ptr(), act.data_ptr(),
-                h.data_ptr() if h is not None else None, ws.data_ptr(), ws.numel(),
-                B, T, D, R, E, top_k, _lib.stream_of(dev))
-        _lib.check(rc)
-        ctx.save_for_backward(x, w_down, w_up, act, probs, top_idx, top_gates)
-        ctx.mark_non_differentiable(top_idx)
-        if h is not None:
-            ctx.mark_non_differentiable(h)
-            return logits, probs, top_idx, top_gates, h
-        return logits, probs, top_idx, top_gates
-
-    @staticmethod
-    def backward(ctx, d_logits, d_probs, _d_idx, d_gates, *_rest):
-        lib = _lib.load()
-        x, w_down, w_up, act, probs, top_idx, top_gates = ctx.saved_tensors
-        B, T, D = x.shape
-        R, E = w_down.shape[0], w_up.shape[0]
-        top_k = top_idx.shape[-1]
-        dev = x.device
-
-        def opt(t):
-            return t.float().contiguous() if t is not None else None
-
-        d_logits, d_gates = opt(d_logits), opt(d_gates)
-        d_probs, dp_ptr, dp_stride = d_probs_arg(d_probs, E)
-        dx = torch.empty_like(x)
-        dw_down = torch.empty((R, D), device=dev, dtype=torch.float32)
-        dw_up = torch.empty((E, R), device=dev, dtype=torch.float32)
-        nbytes = lib.naylis_mom_router_workspace_bytes(B, T, D, R, E, top_k)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-        with _lib.on_device(dev):
-            rc = lib.naylis_mom_router_bwd(
-                x.data_ptr(), _DT[x.dtype], w_down.data_ptr(), w_up.data_ptr(), act.data_ptr(),
-                probs.data_ptr(), top_idx.data_ptr(), top_gates.data_ptr(),
-                d_gates.data_ptr() if d_gates is not None else None,
-                dp_ptr, dp_stride,
-                d_logits.data_ptr() if d_logits is not None else None,
-                dx.data_ptr(), 0, dw_down.data_ptr(), dw_up.data_ptr(), ws.data_ptr(), ws.numel(),
-                B, T, D, R, E, top_k, _lib.stream_of(dev))
-        _lib.check(rc)
-        return dx, dw_down, dw_up, None, None, None, None, None
 
 
 def mom_route(x, w_down, w_up, top_k, noise=None, noise_scale=1.0, return_h=False, noise_is_uniform=False):
@@ -133,44 +67,9 @@ def mom_route(x, w_down, w_up, top_k, noise=None, noise_scale=1.0, return_h=Fals
     x = x.contiguous()
     w_down = w_down.float().contiguous()
     w_up = w_up.float().contiguous()
-    return MomRouteFunction.apply(x, w_down, w_up, noise, float(noise_scale), int(top_k), bool(return_h),
-                                  NOISE_GUMBEL_UNIFORM if noise_is_uniform else NOISE_ADDITIVE)
-
-
-class RouterStatsFunction(torch.autograd.Function):
-    """stats = [mean_prob (E), frac (E), aux, entropy, dead] of a routing.
-    Only mean_prob and aux carry gradient (frac comes from the selection mask;
-    the reference logs entropy and dead fraction detached)."""
-
-    @staticmethod
-    def forward(ctx, probs, top_idx):
-        lib = _lib.load()
-        E = probs.shape[-1]
-        N = probs.numel() // E
-        k = top_idx.shape[-1]
-        dev = probs.device
-        stats = torch.empty(2 * E + 3, device=dev, dtype=torch.float32)
-        nbytes = lib.naylis_mom_router_stats_workspace_bytes(N, E)
-        if nbytes == 0:
-            _lib.check(_lib.NAYLIS_ERR_ARG)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-        with _lib.on_device(dev):
-            _lib.check(lib.naylis_mom_router_stats(probs.data_ptr(), top_idx.data_ptr(), stats.data_ptr(),
-                                                   ws.data_ptr(), ws.numel(), N, E, k, _lib.stream_of(dev)))
-        ctx.save_for_backward(stats)
-        ctx.shape = tuple(probs.shape)
-        return stats
-
-    @staticmethod
-    def backward(ctx, d_stats):
-        (stats,) = ctx.saved_tensors
-        E = ctx.shape[-1]
-        N = 1
-        for s in ctx.shape[:-1]:
-            N *= s
-        # d mean_prob_e = d_stats[e] + d_aux * E * frac_e; every token gets 1/N of it
-        row = (d_stats[:E] + d_stats[2 * E] * E * stats[E:2 * E]) / N
-        return row.expand(ctx.shape), None
+    return tuple(_torch_ext.load().route(x, w_down, w_up, noise, float(noise_scale), int(top_k), bool(return_h),
+                                         NOISE_GUMBEL_UNIFORM if noise_is_uniform else NOISE_ADDITIVE,
+                                         _lib.stream_of(x.device)))
 
 
 def mom_router_stats(probs, top_idx):
@@ -178,7 +77,9 @@ def mom_router_stats(probs, top_idx):
     softmax, top_idx (..., k) int.  Returns a (2E + 3,) fp32 tensor:
     [0:E] mean prob per block, [E:2E] fraction of tokens selecting it, [2E]
     the aux term E * sum(frac * mean_prob) (model.py:500-503), [2E+1] mean
-    router entropy, [2E+2] dead-block fraction (model.py:505-507)."""
+    router entropy, [2E+2] dead-block fraction (model.py:505-507).  Only
+    mean_prob and aux carry gradient (frac comes from the selection mask; the
+    reference logs entropy and dead fraction detached)."""
     if probs.dtype != torch.float32:
         probs = probs.float()
     if probs.device.type != "cuda" or torch.version.hip is None:
@@ -187,4 +88,5 @@ def mom_router_stats(probs, top_idx):
     if top_idx.shape[:-1] != probs.shape[:-1]:
         raise RuntimeError(f"mom_router_stats: top_idx {tuple(top_idx.shape)} does not match probs "
                            f"{tuple(probs.shape)}")
-    return RouterStatsFunction.apply(probs.contiguous(), top_idx.to(torch.int32).contiguous())
+    return _torch_ext.load().router_stats(probs.contiguous(), top_idx.to(torch.int32).contiguous(),
+                                          _lib.stream_of(probs.device))

@@ -307,3 +307,36 @@ def test_layer_external_bank_matches_own_projection(fused, dev, monkeypatch):
     assert torch.equal(m0, m1)
     for n in g0:
         assert torch.equal(g0[n], g1[n]), n
+
+
+@pytest.mark.parametrize("case", EXT_CASES, ids=[f"case{i}" for i in range(len(EXT_CASES))])
+def test_layer_ckpt_node_is_exact(case, dev):
+    """The node's gradient checkpointing (the read's inputs kept, the read run
+    again in the backward): output and every gradient bitwise those of the node
+    that keeps everything, twice through one graph, and less memory held."""
+    import naylis_amd.layer as layer_mod
+    from naylis_amd import mom_kernels
+    B, S, D, H, NB, BS, K, R, m_dtype, external, noise = case
+    res, held = [], []
+    for ckpt in (False, True):
+        layer, _, M = build_pair(D, H, NB, BS, K, R, seed=31)
+        ld = layer_mod.cast_mom_layer(layer.to(dev), torch.bfloat16).train()
+        ld.mom_grad_ckpt = ckpt
+        ld.noise_scale = 1.0 if noise else 0.0
+        g = torch.Generator().manual_seed(6)
+        x = torch.randn(B, S, D, generator=g).bfloat16().to(dev).requires_grad_(True)
+        dy = torch.randn(B, S, D, generator=g).to(dev)
+        Md = M.to(m_dtype).to(dev).requires_grad_(True)
+        torch.cuda.manual_seed(77)
+        kv = mom_kernels.mom_bank_kv_grouped(Md, [ld.k_proj.weight], [ld.v_proj.weight])[0] if external else None
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        y = ld(x, Md, kv)
+        held.append(torch.cuda.memory_allocated() - before)
+        loss = (y * dy).sum().add(layer_mod.mom_aux_loss([ld]))
+        loss.backward(retain_graph=True)
+        loss.backward()
+        res.append([y.detach(), x.grad, Md.grad] + [p.grad for p in ld.parameters() if p.grad is not None])
+    assert len(res[0]) == len(res[1])
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+    assert held[1] < held[0]
