@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define NAYLIS_MOM_ABI_VERSION 18
+#define NAYLIS_MOM_ABI_VERSION 19
 
 #define NAYLIS_OK 0
 #define NAYLIS_ERR_ARG 1       /* invalid shape / argument (the reference raises RuntimeError) */
@@ -369,6 +369,17 @@ int naylis_mom_bank_kv_bwd_grouped(const void* slots, const void* const* w_k, co
                                    void* const* dw_k, void* const* dw_v, int w_grad_dtype, void* workspace,
                                    size_t workspace_bytes, int64_t n_layers, int64_t L, int64_t D_in, int64_t D_out,
                                    void* stream);
+
+/* Forward and input gradient of bias-free projections (nn.Linear, model.py:239,
+ * 251, 253-256 and the Llama trunk's), bf16 operands, fp32 sums:
+ *   y_i = x W_i^T for n = 1 .. 3 weights W_i (D_out, D_in) of one input x
+ *         (N, D_in), in y_dtype;      dx = dy W, bf16, dy (N, D_out).
+ * w and y are host arrays of n device pointers.  D_in and D_out multiples of 8,
+ * any N; all pointers 16-byte aligned. */
+int naylis_mom_linear_fwd(const void* x, const void* const* w, void* const* y, int n, int y_dtype, int64_t N,
+                          int64_t D_in, int64_t D_out, void* stream);
+int naylis_mom_linear_dgrad(const void* dy, const void* w, void* dx, int64_t N, int64_t D_in, int64_t D_out,
+                            void* stream);
 
 /* ------------------------------------------------- projection weight grad ---
  * Weight gradient of the layer's bias-free query / output projections

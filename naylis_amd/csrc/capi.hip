@@ -898,6 +898,46 @@ int naylis_mom_linear_wgrad(const void* x, const void* dy, void* dw, int dw_dtyp
   return hip_status(launch_wgrad(g, (hipStream_t)stream), "linear_wgrad");
 }
 
+static int check_linear(int64_t N, int64_t D_in, int64_t D_out, const char* who) {
+  if (N < 0 || D_in <= 0 || D_out <= 0 || N > ((int64_t)1 << 30) || D_in > 65536 || D_out > 65536)
+    return fail(NAYLIS_ERR_ARG, "%s: bad shape N=%lld D_in=%lld D_out=%lld", who, (long long)N, (long long)D_in,
+                (long long)D_out);
+  if (D_in % 8 || D_out % 8)
+    return fail(NAYLIS_ERR_ARG, "%s: D_in (%lld) and D_out (%lld) must be multiples of 8", who, (long long)D_in,
+                (long long)D_out);
+  return NAYLIS_OK;
+}
+
+static int linear_status(hipError_t e, const char* who) {
+  if (e == hipErrorInvalidValue)
+    return fail(NAYLIS_ERR_ARG, "%s: needs 16-byte aligned pointers and N * max(D_in, D_out) < 2^30", who);
+  return hip_status(e, who);
+}
+
+int naylis_mom_linear_fwd(const void* x, const void* const* w, void* const* y, int n, int y_dtype, int64_t N,
+                          int64_t D_in, int64_t D_out, void* stream) {
+  int rc = check_linear(N, D_in, D_out, "linear_fwd");
+  if (rc) return rc;
+  if ((rc = check_dtype(y_dtype, "linear_fwd"))) return rc;
+  if (n < 1 || n > kGemmMaxJobs || !w || !y)
+    return fail(NAYLIS_ERR_ARG, "linear_fwd: %d weights (1 to %d expected)", n, kGemmMaxJobs);
+  if (N == 0) return NAYLIS_OK;
+  for (int i = 0; i < n; ++i)
+    if (!x || !w[i] || !y[i]) return fail(NAYLIS_ERR_ARG, "linear_fwd: null pointer argument");
+  return linear_status(launch_linear_fwd(x, w, y, n, y_dtype == NAYLIS_DTYPE_F32, (int)N, (int)D_in, (int)D_out,
+                                         (hipStream_t)stream),
+                       "linear_fwd");
+}
+
+int naylis_mom_linear_dgrad(const void* dy, const void* w, void* dx, int64_t N, int64_t D_in, int64_t D_out,
+                            void* stream) {
+  int rc = check_linear(N, D_in, D_out, "linear_dgrad");
+  if (rc || N == 0) return rc;
+  if (!dy || !w || !dx) return fail(NAYLIS_ERR_ARG, "linear_dgrad: null pointer argument");
+  return linear_status(launch_linear_dgrad(dy, w, dx, (int)N, (int)D_in, (int)D_out, (hipStream_t)stream),
+                       "linear_dgrad");
+}
+
 // The gated weight gradient: at least two K splits, so the gate epilogue of
 // the split-K reduction always runs.
 static int gated_wgrad_splits(int64_t N, int64_t D_in, int64_t D_out) {

@@ -38,7 +38,7 @@ struct DevJob {
   long ldc;
 };
 struct DevJobs {
-  DevJob j[2];
+  DevJob j[kGemmMaxJobs];
 };
 // the job table of a grouped launch (every job of one shape and layout)
 struct DevJobsGrouped {
@@ -387,7 +387,7 @@ hipError_t launch_zero(void* p, size_t bytes, hipStream_t st) {
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 bool gemm_supported(const GemmLaunch& g) {
-  if (g.njobs < 1 || g.njobs > 2 || g.M <= 0 || g.N <= 0 || g.K <= 0) return false;
+  if (g.njobs < 1 || g.njobs > kGemmMaxJobs || g.M <= 0 || g.N <= 0 || g.K <= 0) return false;
   if (g.M % 8 || g.N % 8 || g.K % 8) return false;
   if (g.K1 < g.K && g.K1 % kGK) return false;
   for (int j = 0; j < g.njobs; ++j) {
@@ -497,6 +497,48 @@ static void gemm_layouts(const DevJobs& dj, const GemmLaunch& g, int kper, int s
     gemm_dispatch<C, false, true>(dj, g, kper, splits, name, st);
   else
     gemm_dispatch<C, false, false>(dj, g, kper, splits, name, st);
+}
+
+// ---------------------------------------------------------------------------
+// The forward and input-gradient products of bias-free projections:
+//   y_i = x W_i^T (i < n),   dx = dy W
+static GemmLaunch linear_launch(int n, int M, int N, int K, GemmOut out) {
+  GemmLaunch g{};
+  g.njobs = n;
+  g.M = M;
+  g.N = N;
+  g.K = g.K1 = K;
+  g.out = out;
+  g.splits = 1;
+  return g;
+}
+
+// Row counts need not be multiples of 8: x and dy are K-contiguous, so a tile's
+// rows past their end read the last one and are not stored.
+static bool linear_supported(GemmLaunch g) {
+  g.M = (g.M + 7) / 8 * 8;
+  return gemm_supported(g);
+}
+
+hipError_t launch_linear_fwd(const void* x, const void* const* w, void* const* y, int n, bool f32, int N, int D_in,
+                             int D_out, hipStream_t st) {
+  GemmLaunch g = linear_launch(n, N, D_out, D_in, f32 ? kGemmOutF32 : kGemmOutBF16);
+  for (int i = 0; i < n; ++i) {
+    g.job[i].a = GemmOp{x, nullptr, D_in, true};
+    g.job[i].b = GemmOp{w[i], nullptr, D_in, true};
+    g.job[i].c = y[i];
+    g.job[i].ldc = D_out;
+  }
+  return linear_supported(g) ? launch_gemm(g, "linear_fwd", st) : hipErrorInvalidValue;
+}
+
+hipError_t launch_linear_dgrad(const void* dy, const void* w, void* dx, int N, int D_in, int D_out, hipStream_t st) {
+  GemmLaunch g = linear_launch(1, N, D_in, D_out, kGemmOutBF16);
+  g.job[0].a = GemmOp{dy, nullptr, D_out, true};   // A(t, o) = dy[t][o]
+  g.job[0].b = GemmOp{w, nullptr, D_in, false};    // B(o, i) = W[o][i]
+  g.job[0].c = dx;
+  g.job[0].ldc = D_in;
+  return linear_supported(g) ? launch_gemm(g, "linear_dgrad", st) : hipErrorInvalidValue;
 }
 
 hipError_t launch_gemm(const GemmLaunch& g, const char* name, hipStream_t st) {

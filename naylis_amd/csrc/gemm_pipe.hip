@@ -82,7 +82,7 @@ struct PipeJob {
   long ldc;
 };
 struct PipeJobs {
-  PipeJob j[2];
+  PipeJob j[kGemmMaxJobs];
 };
 
 // One operand's tile of a stage (ROWS rows, 32 k).

@@ -25,11 +25,12 @@ struct GemmJob {
   long ldc;
 };
 
-// Up to two GEMMs of the same shape and layouts in one launch.  splits > 1
+// Up to kGemmMaxJobs GEMMs of the same shape and layouts in one launch.  splits > 1
 // splits K over workgroups: fp32 partials go to `ws` (gemm_ws_bytes) and a
 // fixed-order reduction writes C, so results do not depend on the split.
+constexpr int kGemmMaxJobs = 3;
 struct GemmLaunch {
-  GemmJob job[2];
+  GemmJob job[kGemmMaxJobs];
   int njobs;
   int M, N, K, K1;
   GemmOut out;
@@ -81,6 +82,14 @@ struct GemmGroupedLaunch {
 bool gemm_grouped_supported(const GemmGroupedLaunch& g);
 size_t gemm_grouped_ws_bytes(int njobs, int M, int N, bool sum_jobs);
 hipError_t launch_gemm_grouped(const GemmGroupedLaunch& g, const char* timer_name, hipStream_t st);
+
+// Projections (bias-free linear layers) of N tokens: y_i = x W_i^T for n <=
+// kGemmMaxJobs weights, and dx = dy W.  hipErrorInvalidValue when the widths
+// are not multiples of 8, a pointer is not 16-byte aligned or a span exceeds
+// 31 bits.
+hipError_t launch_linear_fwd(const void* x, const void* const* w, void* const* y, int n, bool f32, int N, int D_in,
+                             int D_out, hipStream_t st);
+hipError_t launch_linear_dgrad(const void* dy, const void* w, void* dx, int N, int D_in, int D_out, hipStream_t st);
 
 // Zero `bytes` bytes at p with a kernel (safe inside captured HIP graphs).
 hipError_t launch_zero(void* p, size_t bytes, hipStream_t st);

@@ -43,6 +43,13 @@ inline void* ptr(const at::Tensor& t) { return t.defined() ? t.data_ptr() : null
 
 inline void* stream_ptr(int64_t st) { return reinterpret_cast<void*>(st); }
 
+// y_i = x W_i^T for one to three weights (x (..., D_in), y_i (..., D_out) in
+// `dtype`), and dx = dy W (dy (N, D_out)): the library's GEMM where the rules
+// in torch_nodes.cpp say so, else torch's (hipBLASLt).
+std::vector<at::Tensor> linear_fwd(const at::Tensor& x, const std::vector<at::Tensor>& w, at::ScalarType dtype,
+                                   void* st);
+at::Tensor linear_dgrad(const at::Tensor& dy, const at::Tensor& w, void* st);
+
 // dW = dy^T xin over all rows: the library's GEMM when N, D_in, D_out are
 // multiples of 8, else torch's product (the hip_linear.library_wgrad rule)
 at::Tensor library_wgrad(const at::Tensor& xin, const at::Tensor& dy, at::ScalarType dtype, void* st);

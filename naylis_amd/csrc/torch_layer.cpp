@@ -50,7 +50,7 @@ ReadState read_part(const at::Tensor& x, const c10::optional<at::Tensor>& m_bloc
     r.v = *v_ext;
   }
   // ---- q projection, token order, gated read (model.py:251, 258-276)
-  r.q = at::linear(x, w_q);
+  r.q = linear_fwd(x, {w_q}, at::kBFloat16, st)[0];
   const int64_t words = naylis_mom_read_order_words(B, T, num_blocks, top_k);
   if (words <= 0) check(NAYLIS_ERR_ARG);
   r.order = at::empty({words}, x.options().dtype(at::kInt));
@@ -156,7 +156,7 @@ std::vector<at::Tensor> layer_bwd(c10::optional<at::Tensor> dy, c10::optional<at
   }
   // ---- q projection: dx = dq W_q (the router adds its part below), dW_q = dq^T x
   at::Tensor dq2 = dq.view({N, D});
-  at::Tensor dx = at::mm(dq2, w_q).view({B, T, D});
+  at::Tensor dx = linear_dgrad(dq2, w_q, st).view({B, T, D});
   at::Tensor dw_q = library_wgrad(x.view({N, D}), dq2, w_q.scalar_type(), st);
   // ---- router, accumulating into dx; d_probs as one row with stride 0 when it
   // is an expanded row, else dense (the hip_router.d_probs_arg rule)

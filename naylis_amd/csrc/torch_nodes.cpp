@@ -10,6 +10,8 @@
 // backward, its recompute in the layer's node) 960 -> 427, the decoder's MLP
 // half 410 -> 339 and attention half 620 -> 507, eight layers' evaluation
 // 3630 -> 3120.
+#include <ATen/autocast_mode.h>
+
 #include "torch_common.h"
 
 namespace naylis_ext {
@@ -17,6 +19,76 @@ namespace naylis_ext {
 using torch::autograd::AutogradContext;
 using torch::autograd::Function;
 using torch::autograd::variable_list;
+
+namespace {
+
+bool plain_bf16(const at::Tensor& t) {
+  return t.scalar_type() == at::kBFloat16 && t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0;
+}
+
+// Autocast to another type than bf16 makes torch's products cast their operands.
+bool bf16_products() {
+  return !at::autocast::is_autocast_enabled(at::kCUDA) ||
+         at::autocast::get_autocast_dtype(at::kCUDA) == at::kBFloat16;
+}
+
+// Where the library's GEMM takes a forward product (whole 128-column tiles):
+// one product up to 2048 x 1024 outputs, where its kernel is within a few us of
+// hipBLASLt's (10.6 against 11.1 us at 2042 x 1024 x 1024, 17.3 against 14.9 at
+// 1021 x 2816 -> 1024) and its host call 6 us against 20; two or three of one
+// input up to 768 tiles of 128 x 128, in one launch (q/k/v of 2042 tokens at d
+// 1024: 20 us against 33; gate/up 1024 -> 2816: 29 against 42; three at 3885
+// tokens: 30 against 41).  Past that hipBLASLt's tiles win (two of 3885 x 1024
+// -> 2816, 1335 tiles: 58 against 48).
+bool own_fwd(int64_t n, int64_t N, int64_t D_in, int64_t D_out) {
+  return N > 0 && D_in % 64 == 0 && D_out % 128 == 0 && D_in <= 2816 &&
+         (n == 1 ? N * D_out <= 2 << 20 : n * N * D_out <= 12 << 20);
+}
+
+// ... and an input gradient: level with hipBLASLt's kernel or ahead of it from
+// 64 rows to 3 M outputs (2042 x 1024 x 1024: 10.2 against 12.2 us; 2042 x 2048
+// x 2048: 27.8 against 23.7).
+bool own_dgrad(int64_t N, int64_t D_in, int64_t D_out) {
+  return N >= 64 && D_in % 128 == 0 && D_out % 64 == 0 && D_out <= 2816 && N * D_in <= 3 << 20;
+}
+
+}  // namespace
+
+std::vector<at::Tensor> linear_fwd(const at::Tensor& x, const std::vector<at::Tensor>& w, at::ScalarType dtype,
+                                   void* st) {
+  const int64_t D_out = w[0].size(0), D_in = w[0].size(1), N = x.numel() / std::max<int64_t>(D_in, 1), n = w.size();
+  bool own = x.size(-1) == D_in && own_fwd(n, N, D_in, D_out) && x.scalar_type() == at::kBFloat16 && bf16_products();
+  for (const at::Tensor& t : w) own = own && plain_bf16(t) && t.sizes() == w[0].sizes();
+  std::vector<at::Tensor> y;
+  const at::Tensor xc = own ? x.contiguous() : x;
+  if (!own || !plain_bf16(xc)) {
+    for (const at::Tensor& t : w)
+      y.push_back(dtype == at::kFloat ? at::mm(x.reshape({-1, D_in}), t.t(), at::kFloat) : at::linear(x, t));
+    return y;
+  }
+  std::vector<int64_t> shape = x.sizes().vec();
+  if (dtype == at::kFloat)
+    shape = {N, D_out};
+  else
+    shape.back() = D_out;
+  const void* wp[3];
+  void* yp[3];
+  for (int64_t i = 0; i < n; ++i) {
+    y.push_back(at::empty(shape, x.options().dtype(dtype)));
+    wp[i] = w[i].data_ptr();
+    yp[i] = y[i].data_ptr();
+  }
+  check(naylis_mom_linear_fwd(xc.data_ptr(), wp, yp, (int)n, dtype == at::kFloat ? kF32 : kBF16, N, D_in, D_out, st));
+  return y;
+}
+
+at::Tensor linear_dgrad(const at::Tensor& dy, const at::Tensor& w, void* st) {
+  const int64_t N = dy.size(0), D_out = w.size(0), D_in = w.size(1);
+  if (!own_dgrad(N, D_in, D_out) || !plain_bf16(dy) || !plain_bf16(w) || !bf16_products()) return at::mm(dy, w);
+  at::Tensor dx = at::empty({N, D_in}, dy.options());
+  check(naylis_mom_linear_dgrad(dy.data_ptr(), w.data_ptr(), dx.data_ptr(), N, D_in, D_out, st));
+  return dx;
+}
 
 at::Tensor library_wgrad(const at::Tensor& xin, const at::Tensor& dy, at::ScalarType dtype, void* st) {
   const int64_t N = xin.size(0), D_in = xin.size(1), D_out = dy.size(1);
@@ -36,14 +108,14 @@ std::pair<at::Tensor, at::Tensor> gated_linear_forward(const at::Tensor& out2, c
   at::Tensor w_os = at::empty_like(w_o);
   check(naylis_mom_rezero_scale(w_o.data_ptr(), dtype_code(w_o), s.data_ptr<float>(), w_os.data_ptr(),
                                 dtype_code(w_os), w_o.numel(), st));
-  return {at::mm(out2, w_os.t(), at::kFloat), w_os};
+  return {linear_fwd(out2, {w_os}, at::kFloat, st)[0], w_os};
 }
 
 GatedGrads gated_linear_backward(const at::Tensor& dy, const at::Tensor& out2, const at::Tensor& w_o,
                                  const at::Tensor& w_os, const at::Tensor& s, void* st) {
   const at::Tensor dy2 = dy.to(at::kBFloat16).contiguous();
   GatedGrads g;
-  g.dout2 = at::mm(dy2, w_os);
+  g.dout2 = linear_dgrad(dy2, w_os, st);
   const int64_t N = out2.size(0), D_in = out2.size(1), D_out = dy2.size(1);
   g.dw_o = at::empty_like(w_o);
   g.ds = at::empty({1}, out2.options().dtype(at::kFloat));
@@ -230,30 +302,29 @@ struct SwiGLU : public Function<SwiGLU> {
 struct SharedLinear : public Function<SharedLinear> {
   static variable_list forward(AutogradContext* ctx, at::Tensor x, at::Tensor w0, at::Tensor w1, at::Tensor w2,
                                int64_t n, int64_t st) {
-    const at::Tensor w[3] = {w0, w1, w2};
-    variable_list saved = {x}, y;
-    for (int64_t i = 0; i < n; ++i) {
-      saved.push_back(w[i]);
-      y.push_back(at::linear(x, w[i]));
-    }
+    at::DeviceGuard guard(x.device());
+    std::vector<at::Tensor> w = {w0, w1, w2};
+    w.resize(n);
+    variable_list saved = w;
+    saved.push_back(x);
     ctx->save_for_backward(saved);
     ctx->saved_data["st"] = st;
-    return y;
+    return linear_fwd(x, w, x.scalar_type(), stream_ptr(st));
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
-    const at::Tensor& x = s[0];
+    const at::Tensor& x = s.back();
     at::DeviceGuard guard(x.device());
     void* st = stream_ptr(ctx->saved_data["st"].toInt());
     const size_t n = s.size() - 1;
     const at::Tensor x2 = x.reshape({-1, x.size(-1)}).contiguous();
     variable_list r(6);
     for (size_t i = 0; i < n; ++i) {
-      const at::Tensor& w = s[1 + i];
+      const at::Tensor& w = s[i];
       const at::Tensor dy = grads[i].reshape({-1, w.size(0)}).contiguous();
       if (ctx->needs_input_grad(0)) {
         if (i == 0)
-          r[0] = at::mm(dy, w);
+          r[0] = linear_dgrad(dy, w, st);
         else
           r[0].addmm_(dy, w);
       }
@@ -511,6 +582,16 @@ void bind_nodes(pybind11::module_& m) {
   m.def("shared_linear", [](Tensor x, std::vector<Tensor> w, int64_t st) {
     TORCH_CHECK(!w.empty() && w.size() <= 3, "shared_linear: one to three weights");
     return SharedLinear::apply(x, w[0], w[w.size() > 1 ? 1 : 0], w[w.size() > 2 ? 2 : 0], (int64_t)w.size(), st);
+  });
+  m.def("linear", [](Tensor x, std::vector<Tensor> w, bool f32, int64_t st) {  // the products alone, no graph
+    at::NoGradGuard no_grad;
+    at::DeviceGuard guard(x.device());
+    return linear_fwd(x, w, f32 ? at::kFloat : x.scalar_type(), stream_ptr(st));
+  });
+  m.def("linear_dgrad", [](Tensor dy, Tensor w, int64_t st) {
+    at::NoGradGuard no_grad;
+    at::DeviceGuard guard(dy.device());
+    return linear_dgrad(dy, w, stream_ptr(st));
   });
   m.def("route", [](Tensor x, Tensor wd, Tensor wu, c10::optional<Tensor> noise, double noise_scale, int64_t top_k,
                     bool want_h, int64_t kind, int64_t st) {

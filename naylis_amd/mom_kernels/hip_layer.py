@@ -26,7 +26,6 @@ tests that compare the two bitwise.
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 
 from .. import _lib, _torch_ext
 from .hip_linear import library_wgrad as _wgrad
@@ -85,7 +84,7 @@ class MomLayerFunction(torch.autograd.Function):
     def forward(ctx, x, M_blocks, w_down, w_up, w_q, w_k, w_v, w_o, scale, noise, noise_scale, geom, k_ext=None,
                 v_ext=None):
         n_heads, num_blocks, block_size, top_k, noise_kind = geom
-        lib = _lib.load()
+        lib, ext = _lib.load(), _torch_ext.load()
         B, T, D = x.shape
         R, E = w_down.shape[0], w_up.shape[0]
         H, HD = n_heads, D // n_heads
@@ -133,7 +132,7 @@ class MomLayerFunction(torch.autograd.Function):
             else:
                 slots, m_dtype, k, v = None, None, k_ext, v_ext
             # ---- q projection, gated read, o projection (model.py:251, 258-276)
-            q = F.linear(x, w_q)
+            q = ext.linear(x, [w_q], False, st)[0]
             order = read_order(top_idx, num_blocks)
             out = torch.empty_like(q)
             side = read_side(lib, out.view(B, T, H, HD), num_blocks, block_size, top_k)
@@ -213,7 +212,7 @@ class MomLayerFunction(torch.autograd.Function):
                 d_m, dk_ext, dv_ext = d_slots.view(m_shape), None, None
             # ---- q projection: dx = dq W_q (the router adds its part below), dW_q = dq^T x
             dq2 = dq.view(N, D)
-            dx = torch.mm(dq2, w_q).view(B, T, D)
+            dx = _torch_ext.load().linear_dgrad(dq2, w_q, st).view(B, T, D)
             dw_q = _wgrad(lib, x.view(N, D), dq2, w_q.dtype, dev, st)
             # ---- router, accumulating into dx
             d_probs, dp_ptr, dp_stride = d_probs_arg(d_probs, E)

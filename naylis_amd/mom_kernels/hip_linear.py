@@ -19,6 +19,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.autograd import forward_ad
 
 from .. import _lib, _torch_ext
 
@@ -44,23 +45,35 @@ def library_wgrad(lib, xin, dy, dtype, dev, st):
     return dw
 
 
-def mom_linear(x, weight):
-    """y = x W^T (no bias).  For bf16 activations and weights on a ROCm device
-    with dimensions that are multiples of 8 the weight gradient runs on the
-    library's GEMM; any other combination is the plain torch linear."""
-    D_out, D_in = weight.shape
-    if (x.is_cuda and torch.version.hip is not None and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
-            and D_in % 8 == 0 and D_out % 8 == 0 and (x.numel() // D_in) % 8 == 0 and torch.is_grad_enabled()
-            and weight.requires_grad):
-        return _torch_ext.load().shared_linear(x, [weight], _lib.stream_of(x.device))[0]
-    return F.linear(x, weight)
-
-
-def _library_ok(x, weight):
+def _library_ok(x, weight, rows=8):
+    """bf16 x and weight on one ROCm device, widths multiples of 8 and the
+    token count a multiple of ``rows``."""
     D_out, D_in = weight.shape
     return (x.is_cuda and torch.version.hip is not None and x.dtype == torch.bfloat16
             and weight.dtype == torch.bfloat16 and weight.device == x.device and D_in % 8 == 0 and D_out % 8 == 0
-            and x.shape[-1] == D_in and (x.numel() // D_in) % 8 == 0)
+            and x.shape[-1] == D_in and (x.numel() // D_in) % rows == 0)
+
+
+def _untransformed(x, *weights):
+    """Plain tensors outside functorch transforms, forward-mode AD and tracing:
+    what may go to a kernel by its pointer where torch's own product, which
+    knows about those, ran before."""
+    return (type(x) is torch.Tensor and all(type(w) in (torch.Tensor, nn.Parameter) for w in weights)
+            and not torch._C._are_functorch_transforms_active() and forward_ad._current_level < 0
+            and torch._C._get_tracing_state() is None)
+
+
+def mom_linear(x, weight):
+    """y = x W^T (no bias).  For bf16 activations and weights on a ROCm device
+    with dimensions that are multiples of 8 the weight gradient runs on the
+    library's GEMM, and so do the forward and the input gradient at the sizes
+    where it is faster; any other combination is the plain torch linear."""
+    if not torch.is_grad_enabled():
+        if _untransformed(x, weight) and _library_ok(x, weight, 1):
+            return _torch_ext.load().linear(x, [weight], False, _lib.stream_of(x.device))[0]
+    elif weight.requires_grad and _library_ok(x, weight):
+        return _torch_ext.load().shared_linear(x, [weight], _lib.stream_of(x.device))[0]
+    return F.linear(x, weight)
 
 
 def shared_input_linear(x, linears):
@@ -70,10 +83,17 @@ def shared_input_linear(x, linears):
     with dimensions that are multiples of 8: autograd would sum their input
     gradients with separate elementwise adds, the node accumulates each
     further product into the first in the GEMM's epilogue (one rounding of the
-    sum).  Otherwise each layer applied in turn."""
-    if (torch.is_grad_enabled() and len(linears) <= 3 and all(m.bias is None and _library_ok(x, m.weight) for m in linears)
-            and any(m.weight.requires_grad for m in linears)):
-        return tuple(_torch_ext.load().shared_linear(x, [m.weight for m in linears], _lib.stream_of(x.device)))
+    sum).  Where the library's GEMM is faster it takes all forward products in
+    one launch, in evaluation too.  Otherwise each layer applied in turn."""
+    if len(linears) <= 3 and all(m.bias is None for m in linears):
+        ws = [m.weight for m in linears]
+        if not torch.is_grad_enabled():
+            if _untransformed(x, *ws) and all(type(m) is NaylisLinear and not m._forward_hooks
+                                              and not m._forward_pre_hooks and _library_ok(x, w, 1)
+                                              for m, w in zip(linears, ws)):
+                return tuple(_torch_ext.load().linear(x, ws, False, _lib.stream_of(x.device)))
+        elif all(_library_ok(x, w) for w in ws) and any(w.requires_grad for w in ws):
+            return tuple(_torch_ext.load().shared_linear(x, ws, _lib.stream_of(x.device)))
     return tuple(m(x) for m in linears)
 
 

@@ -31,7 +31,7 @@ def gated_linear_forward(lib, out2, w_o, s, st):
     w_os = torch.empty_like(w_o)
     _lib.check(lib.naylis_mom_rezero_scale(w_o.data_ptr(), _DT[w_o.dtype], s.data_ptr(), w_os.data_ptr(),
                                            _DT[w_os.dtype], w_o.numel(), st))
-    return torch.mm(out2, w_os.t(), out_dtype=torch.float32), w_os
+    return _torch_ext.load().linear(out2, [w_os], True, st)[0], w_os
 
 
 def gated_linear_backward(lib, dy2, out2, w_o, w_os, s, st):
@@ -39,7 +39,7 @@ def gated_linear_backward(lib, dy2, out2, w_o, w_os, s, st):
     (rows = tokens, rounded to bf16 for the two GEMMs)."""
     dev = out2.device
     dy2 = dy2.to(torch.bfloat16).contiguous()
-    dout2 = torch.mm(dy2, w_os)
+    dout2 = _torch_ext.load().linear_dgrad(dy2, w_os, st)
     N, D_in = out2.shape
     D_out = dy2.shape[1]
     if (out2.dtype == torch.bfloat16 and w_o.dtype == torch.bfloat16 and w_o.is_contiguous() and out2.is_contiguous()

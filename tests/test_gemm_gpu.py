@@ -213,3 +213,63 @@ def test_gated_wgrad_pipelined(dev):
     ds = (ref * w.detach().double()).sum()
     var = ((8 * N ** 0.5 * 2.0 ** -24 * (a.abs() @ b.abs())) * w.detach().double()).square().sum().sqrt()
     assert abs(float(s.grad) - float(ds)) <= float(var) + 2.0 ** -20 * float((ref * w.detach().double()).abs().sum())
+
+
+@pytest.mark.parametrize("N", [1, 63, 64, 131, 1021, 2048, 2050])
+@pytest.mark.parametrize("D_in,D_out,n", [(64, 128, 3), (1024, 1024, 3), (1024, 2816, 2), (2816, 1024, 1),
+                                          (256, 640, 2)])
+def test_linear_fwd_and_dgrad_match_fp64(N, D_in, D_out, n, dev):
+    """naylis_mom_linear_fwd (one to three weights, bf16 and fp32 results) and
+    naylis_mom_linear_dgrad at row counts around the tiles, odd ones among them."""
+    import ctypes
+
+    from naylis_amd import _lib
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev).manual_seed(N + D_in)
+    x = torch.randn(N, D_in, generator=g, device=dev).bfloat16()
+    dy = torch.randn(N, D_out, generator=g, device=dev).bfloat16()
+    ws = [torch.randn(D_out, D_in, generator=g, device=dev).bfloat16() for _ in range(n)]
+    ptrs = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])  # noqa: E731
+    for code, dtype in ((0, torch.float32), (1, torch.bfloat16)):
+        ys = [torch.full((N + 1, D_out), 7.0, device=dev, dtype=dtype) for _ in range(n)]
+        _lib.check(lib.naylis_mom_linear_fwd(x.data_ptr(), ptrs(ws), ptrs(ys), n, code, N, D_in, D_out, st))
+        for y, w in zip(ys, ws):
+            a, b = x.double(), w.double().t()
+            ref = a @ b
+            bound = _sum_bound(a, b, ref)
+            assert bool(((y[:N].double() - ref).abs() <= bound).all())
+            assert bool((y[N] == 7).all())      # nothing past the last row
+    dx = torch.full((N + 1, D_in), 7.0, device=dev, dtype=torch.bfloat16)
+    _lib.check(lib.naylis_mom_linear_dgrad(dy.data_ptr(), ws[0].data_ptr(), dx.data_ptr(), N, D_in, D_out, st))
+    a, b = dy.double(), ws[0].double()
+    ref = a @ b
+    assert bool(((dx[:N].double() - ref).abs() <= _sum_bound(a, b, ref)).all()) and bool((dx[N] == 7).all())
+
+
+def test_linear_routes(dev):
+    """Evaluation and training take the same product (bit for bit); transforms,
+    tracing and module hooks keep torch's."""
+    from naylis_amd.mom_kernels.hip_linear import NaylisLinear, shared_input_linear
+    g = torch.Generator(device=dev).manual_seed(1)
+    mods = [NaylisLinear(256, 384, bias=False).to(dev, torch.bfloat16) for _ in range(3)]
+    x = torch.randn(3, 80, 256, generator=g, device=dev).bfloat16()
+    train = shared_input_linear(x, mods)
+    want = [torch.nn.functional.linear(x.double(), m.weight.double()) for m in mods]
+    with torch.no_grad():
+        ev = shared_input_linear(x, mods)
+        assert all(torch.equal(a, b) for a, b in zip(train, ev))
+        for y, r, m in zip(ev, want, mods):
+            a, b = x.double().view(-1, 256), m.weight.double().t()
+            assert bool(((y.double() - r).abs() <= _sum_bound(a, b, r.view(-1, 384)).view_as(r)).all())
+        mapped = torch.func.vmap(mods[0])(x)
+        assert mapped.shape == ev[0].shape
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+            assert torch.autograd.forward_ad.unpack_dual(mods[0](dual)).tangent is not None
+        seen = []
+        h = mods[1].register_forward_hook(lambda m, i, o: seen.append(1))
+        shared_input_linear(x, mods)
+        h.remove()
+        assert seen == [1]
+        traced = torch.jit.trace(mods[0], (x,), check_trace=False)
+        assert not torch.equal(traced(x), traced(2 * x))
