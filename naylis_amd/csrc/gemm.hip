@@ -556,6 +556,7 @@ hipError_t launch_gemm(const GemmLaunch& g, const char* name, hipStream_t st) {
   GemmLaunch gl = g;
   gl.K1 = g.K1 < g.K ? g.K1 : g.K;
   if (splits == 1 && g.gate_w == nullptr && gemm_pipe_ok(gl)) return launch_gemm_pipe(gl, name, st);
+  if (splits == 1 && g.gate_w == nullptr && gemm_small_ok(gl)) return launch_gemm_small(gl, name, st);
   // the largest tile that still gives at least one workgroup per CU
   auto wgs = [&](int bm, int bn) {
     return (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * splits * g.njobs;

@@ -1,15 +1,19 @@
-// Pipelined bf16 GEMM for large shapes (gfx950, v_mfma_f32_32x32x16_bf16, fp32
-// sums): the products of gemm.hip whose grid fills the chip with 256 x 128
-// tiles, and the weight gradients, whose K (all tokens) is cut into equal
-// ranges of the (tile, K step) list so that every CU works to the end.
+// Pipelined bf16 GEMM (gfx950, v_mfma_f32_32x32x16_bf16, fp32 sums): the
+// products of gemm.hip whose grid fills the chip with 256 x 128 tiles, those
+// that fit it once with smaller ones, and the weight gradients, whose K (all
+// tokens) is cut into equal ranges of the (tile, K step) list so that every CU
+// works to the end.
 //
-// 8 waves (4 x 2) of 64 x 64 per 256 x 128 tile, K steps of 32.  Stages go from
+// 8 waves (4 x 2) of 64 x 64 per 256 x 128 tile, K steps of 64.  Stages go from
 // memory to LDS directly (buffer loads with an LDS destination, no staging
-// registers), through a ring of 6 x 24 KB: at step s the loads of stage s + 5
-// are issued while stages s + 1 .. s + 4 are in flight.  One barrier a step,
-// between its two 16-wide halves: the fragments of the second half are read
-// before it, those of the next stage's first half after it, so LDS latency
-// lies under the products of the other half.
+// registers), through a ring of 3 x 48 KB: at step s the loads of stage s + 2
+// are issued while stage s + 1 is in flight.  One barrier a step, before its
+// last 16-wide slice: fragments are read a slice ahead, the last slice's before
+// the barrier and those of the next stage's first slice after it, so LDS
+// latency lies under the products of the slice before.  Steps of 32 in a ring
+// of 6 hold as many bytes in flight but pay twice the barriers: 2042 x 2816 over
+// K 1024 19.1 us against 17.0, 4096 x 1536 over 1536 27.1 against 22.6; weight
+// gradients over 16384 tokens 3 - 5 % slower.
 //
 // Direct loads write LDS in lane order, so the tiles cannot be padded; 64-byte
 // groups (row-contiguous operands, [k][row]) or 16-byte chunks (K-contiguous
@@ -17,11 +21,11 @@
 // leaves both fragment reads (ds_read_b64_tr_b16, ds_read_b128) free of bank
 // conflicts.
 //
-// The K loop is bound by the matrix units at the clock that the card holds
+// Large products are bound by the matrix units at the clock that the card holds
 // under them: operands of zeros run 15 - 20 % faster, and without any load or
-// LDS read it takes 53 us of the 66 below.  Against gemm.hip (kernel and
-// reduction, 16384 tokens): 1024 x 1024 51.5 -> 45.5 us, 2048 x 1024 80 -> 72,
-// 1024 x 2816 135 -> 104 (0.91 PFLOP/s), 1536 x 1536 107 -> 84; whole tiles,
+// LDS read the K loop takes 53 us of the 62 below.  Against gemm.hip (kernel
+// and reduction, 16384 tokens): 1024 x 1024 51.5 -> 42.8 us, 2048 x 1024 80 ->
+// 72, 1024 x 2816 135 -> 99 (0.96 PFLOP/s), 1536 x 1536 107 -> 84; whole tiles,
 // 5632 x 2048 over 4096: 116 -> 85 (1.11 PFLOP/s).
 #include "common.h"
 #include "launch_gemm.h"
@@ -34,20 +38,28 @@ namespace naylis {
 
 namespace {
 
-constexpr int kBK = 32, kNT = 512;
-
-// Workgroup tile BM x BN of 8 waves, WM of them along M, each with TM x TN
-// tiles of 32 x 32; RING stages of LDS.
-template <int BN_, int WM_, int TM_, int TN_, int RING_>
+// WAVES waves, WM of them along M, each with TM x TN tiles of 32 x 32; K steps
+// of BK, RING stages of them in LDS.
+template <int WAVES_, int WM_, int TM_, int TN_, int BK_, int RING_>
 struct PipeCfg {
-  static constexpr int BM = 256, BN = BN_, WM = WM_, TM = TM_, TN = TN_, RING = RING_;
-  static constexpr int ABYTES = BM * kBK * 2, STAGE = ABYTES + BN * kBK * 2;
-  static constexpr int NA = BM / 128, NB = BN / 128;  // 1 KB pieces of A and B that a wave loads of each stage
+  static constexpr int WAVES = WAVES_, WM = WM_, TM = TM_, TN = TN_, BK = BK_, RING = RING_, NT = 64 * WAVES;
+  static constexpr int BM = WM * TM * 32, BN = WAVES / WM * TN * 32;
+  static constexpr int ABYTES = BM * BK * 2, STAGE = ABYTES + BN * BK * 2;
+  // 1 KB pieces of A and B that a wave loads of each stage
+  static constexpr int NA = ABYTES / 1024 / WAVES, NB = (STAGE - ABYTES) / 1024 / WAVES;
   static constexpr int FLIGHT = (RING - 2) * (NA + NB);  // loads in flight past the stage waited for
-  static_assert(WM * TM * 32 == BM && 8 / WM * TN * 32 == BN);
+  static_assert(NA * WAVES * 1024 == ABYTES && NB * WAVES * 1024 == STAGE - ABYTES && RING * STAGE <= 160 * 1024);
 };
-using Cfg128 = PipeCfg<128, 4, 2, 2, 6>;
-using Cfg256 = PipeCfg<256, 2, 4, 2, 5>;
+using Cfg128 = PipeCfg<8, 4, 2, 2, 64, 3>;     // 256 x 128
+using Cfg128K32 = PipeCfg<8, 4, 2, 2, 32, 6>;  // ... for an odd number of 32s of K
+using Cfg256 = PipeCfg<8, 2, 4, 2, 32, 5>;     // 256 x 256
+// Products of at most one of these per CU.  They are bound by latency (one
+// step: a barrier, an LDS read and 4 dependent products) and by what one CU
+// draws from L2, so stages are deep (6 - 8 of 16 - 24 KB) and 128 x 128 and 64 x
+// 128 take 8 waves, two per SIMD: with 4 waves the former is 10 - 15 % slower.
+using CfgS128 = PipeCfg<8, 4, 1, 2, 64, 4>;  // 128 x 128
+using CfgS64 = PipeCfg<8, 2, 1, 1, 64, 6>;   // 64 x 128
+using CfgS32 = PipeCfg<4, 2, 1, 1, 64, 8>;   // 64 x 64
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
@@ -85,11 +97,17 @@ struct PipeJobs {
   PipeJob j[kGemmMaxJobs];
 };
 
-// One operand's tile of a stage (ROWS rows, 32 k).
-template <bool KC, int ROWS>
+// One operand's tile of a stage (ROWS rows, BK k).
+template <bool KC, int ROWS, int BK>
 struct Operand {
-  static constexpr int RB = KC ? kBK * 2 : ROWS * 2;  // bytes of an LDS row
-  static constexpr int CPR = RB / 16;                 // its 16-byte chunks
+  static constexpr int RB = KC ? BK * 2 : ROWS * 2;  // bytes of an LDS row
+  static constexpr int CPR = RB / 16;                // its 16-byte chunks
+  // XOR applied to the chunk index of LDS row i: 16 rows' equal chunks (KC) or
+  // four rows' 64-byte groups then cover 256 bytes
+  static __device__ __forceinline__ int swz(int i) {
+    if constexpr (KC) return RB == 64 ? (i >> 2) & 3 : (i >> 1) & 7;
+    return RB == 128 ? (i & 2) << 1 : (i & 3) << 2;
+  }
   i32x4 r1, r2;
   long ld;
 
@@ -109,30 +127,31 @@ struct Operand {
     const int i = u * (64 / CPR) + lane / CPR, c = lane % CPR;  // LDS row, chunk
     if constexpr (KC) {
       const int r = min(row0 + i, nrows - 1) - row0;
-      return (int)((long)r * ld * 2) + ((c ^ ((i >> 2) & 3)) << 4);
+      return (int)((long)r * ld * 2) + ((c ^ swz(i)) << 4);
     } else {
-      const int r = min(row0 + ((c ^ ((i & 3) << 2)) << 3), nrows - 8) - row0;
+      const int r = min(row0 + ((c ^ swz(i)) << 3), nrows - 8) - row0;
       return (int)(((long)i * ld + r) * 2);
     }
   }
   __device__ __forceinline__ int soff(int k) const { return (int)(KC ? (long)k * 2 : (long)k * ld * 2); }
 };
 
-// Fragments (A layout of common.h) of rows m0 + 32 i, i < T, K half h.
-template <bool KC, int ROWS, int T>
+// Fragments (A layout of common.h) of rows m0 + 32 i, i < T, K slice h of 16.
+template <bool KC, int ROWS, int T, int BK>
 struct Frags {
-  static constexpr int RB = Operand<KC, ROWS>::RB;
-  int off[2 * T];
+  using Op = Operand<KC, ROWS, BK>;
+  static constexpr int RB = Op::RB;
+  int off[KC ? BK / 16 : T];
   __device__ __forceinline__ Frags(int m0, int lane) {
     if constexpr (KC) {
       const int r = lane & 31, g = lane >> 5;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) off[h] = (m0 + r) * RB + (((2 * h + g) ^ ((r >> 2) & 3)) << 4);
+      for (int h = 0; h < BK / 16; ++h) off[h] = (m0 + r) * RB + (((2 * h + g) ^ Op::swz(r)) << 4);
     } else {  // lds_frag_T<false, false> of common.h
       const int q = lane >> 4, j = lane & 15, x = j >> 2;
 #pragma unroll
       for (int i = 0; i < T; ++i)
-        off[i] = (8 * (q >> 1) + x) * RB + (((m0 / 32 + i) ^ x) << 6) + 32 * (q & 1) + 8 * (j & 3);
+        off[i] = (8 * (q >> 1) + x) * RB + (((m0 / 32 + i) ^ (Op::swz(x) >> 2)) << 6) + 32 * (q & 1) + 8 * (j & 3);
     }
   }
   __device__ __forceinline__ void get(bf16x8 (&f)[T], const uint8_t* tile, int h) const {
@@ -195,16 +214,18 @@ struct Ranges {
 // goes to partial w + t (unique: a later workgroup never holds an earlier
 // tile).
 template <class C, bool AKC, bool BKC, int OUT>
-__global__ __launch_bounds__(kNT, 2) void gemm_pipe_kernel(PipeJobs jobs, int M, int N, int K, int K1, int tiles_m,
+__global__ __launch_bounds__(C::NT, C::WAVES == 8 ? 2 : 1) void gemm_pipe_kernel(PipeJobs jobs, int M, int N, int K, int K1, int tiles_m,
                                                            int tiles_n, Ranges rg, float* __restrict__ ws) {
   __shared__ __align__(1024) uint8_t ring[C::RING * C::STAGE];
   const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)ring;  // LDS byte address
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % C::WM * (32 * C::TM), wn = wave / C::WM * (32 * C::TN);
-  const int nk = K / kBK, tiles = tiles_m * tiles_n;
-  const Frags<AKC, C::BM, C::TM> fa(wm, lane);
-  const Frags<BKC, C::BN, C::TN> fb(wn, lane);
+  constexpr int BK = C::BK;
+  // OUT == 2: rows of K past the last one are out of the operands' resources and read as zeros
+  const int nk = (K + BK - 1) / BK, tiles = tiles_m * tiles_n;
+  const Frags<AKC, C::BM, C::TM, BK> fa(wm, lane);
+  const Frags<BKC, C::BN, C::TN, BK> fb(wn, lane);
 
   int w = blockIdx.x, pos, end;  // this workgroup's steps: pos .. end
   const PipeJob* job = &jobs.j[0];
@@ -224,15 +245,15 @@ __global__ __launch_bounds__(kNT, 2) void gemm_pipe_kernel(PipeJobs jobs, int M,
     int tm, tn;
     TileGrid{tiles_m, tiles_n}.tile_of(OUT == 2 ? rg.rank_of(t, tiles) : t, tm, tn);
     const int m0 = tm * C::BM, n0 = tn * C::BN;
-    Operand<AKC, C::BM> A;
-    Operand<BKC, C::BN> B;
+    Operand<AKC, C::BM, BK> A;
+    Operand<BKC, C::BN, BK> B;
     A.init(job->a, m0, M, K1, K);
     B.init(job->b, n0, N, K1, K);
     int va[C::NA], vb[C::NB];
 #pragma unroll
-    for (int i = 0; i < C::NA; ++i) va[i] = A.voff(wave + 8 * i, m0, M, lane);
+    for (int i = 0; i < C::NA; ++i) va[i] = A.voff(wave + C::WAVES * i, m0, M, lane);
 #pragma unroll
-    for (int i = 0; i < C::NB; ++i) vb[i] = B.voff(wave + 8 * i, n0, N, lane);
+    for (int i = 0; i < C::NB; ++i) vb[i] = B.voff(wave + C::WAVES * i, n0, N, lane);
     const i32x4 none = rsrc_words(jobs.j[0].a.p1, 0);
     f32x16 acc[C::TM][C::TN];
 #pragma unroll
@@ -243,15 +264,15 @@ __global__ __launch_bounds__(kNT, 2) void gemm_pipe_kernel(PipeJobs jobs, int M,
     // stage s of this part into ring slot `slot`; past the last one an empty
     // resource keeps the number of loads in flight the same
     auto load = [&](int s, int slot) {
-      const int k = (kb + s) * kBK;
+      const int k = (kb + s) * BK;
       const bool live = s < n, second = k >= K1;
       const i32x4 ra = live ? (second ? A.r2 : A.r1) : none, rb = live ? (second ? B.r2 : B.r1) : none;
       const int ks = live ? (second ? k - K1 : k) : 0;
       const uint32_t p = ring0 + slot * C::STAGE + wave * 1024;
 #pragma unroll
-      for (int i = 0; i < C::NA; ++i) load_to_lds(ra, va[i], A.soff(ks), p + i * 8192);
+      for (int i = 0; i < C::NA; ++i) load_to_lds(ra, va[i], A.soff(ks), p + i * C::WAVES * 1024);
 #pragma unroll
-      for (int i = 0; i < C::NB; ++i) load_to_lds(rb, vb[i], B.soff(ks), p + C::ABYTES + i * 8192);
+      for (int i = 0; i < C::NB; ++i) load_to_lds(rb, vb[i], B.soff(ks), p + C::ABYTES + i * C::WAVES * 1024);
     };
     auto products = [&](const bf16x8 (&a)[C::TM], const bf16x8 (&b)[C::TN]) {
 #pragma unroll
@@ -274,6 +295,18 @@ __global__ __launch_bounds__(kNT, 2) void gemm_pipe_kernel(PipeJobs jobs, int M,
       __builtin_amdgcn_sched_barrier(0);
       products(a0, b0);
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (BK == 64) {
+        fa.get(a0, cur, 2);
+        fb.get(b0, cur + C::ABYTES, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        products(a1, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        fa.get(a1, cur, 3);
+        fb.get(b1, cur + C::ABYTES, 3);
+        __builtin_amdgcn_sched_barrier(0);
+        products(a0, b0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       // stage s + 1 is in LDS, and every wave has read stage s (its slot is loaded from the next step on)
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::FLIGHT) : "memory");
       slot = slot == C::RING - 1 ? 0 : slot + 1;
@@ -283,6 +316,9 @@ __global__ __launch_bounds__(kNT, 2) void gemm_pipe_kernel(PipeJobs jobs, int M,
       products(a1, b1);
       __builtin_amdgcn_sched_barrier(0);
     }
+
+    // the late loads (zeros, past the last stage) are in LDS before its next user's
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     // acc[i][j][v] = C(m0 + wm + 32 i + acc_row(lane / 32, v), n0 + wn + 32 j + lane % 32)
     const int g = lane >> 5, col = lane & 31;
@@ -317,8 +353,8 @@ __global__ __launch_bounds__(kNT, 2) void gemm_pipe_kernel(PipeJobs jobs, int M,
       }
     }
     pos += share;
-    // no wave loads the next part's stages over this one's reads or late loads
-    if (pos < end) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // no wave loads the next part's stages over this one's reads
+    if (pos < end) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
 }
 
@@ -414,11 +450,10 @@ static PipeJobs pipe_jobs(const GemmLaunch& g) {
 }
 
 // Whole tiles, one per workgroup: K in whole steps, and 256 x 128 tiles for
-// more than half of the CUs (128 tiles, one round at half the chip: the bank's
-// K / V of 1024 slots at d 2048 take 31 us against 27 with the 128 x 128 tiles
-// of gemm.hip; 144 tiles, its weight gradients at d 1536: 55 against 71).
+// more than half of the CUs; below that the small tiles also fit the chip once
+// (2042 x 1024 over 1024, 64 against 128 tiles: 9.2 us with the latter).
 bool gemm_pipe_ok(const GemmLaunch& g) {
-  return g.K % kBK == 0 && g.K1 % kBK == 0 && g.M >= 256 && g.N >= 128 && pipe_tiles<Cfg128>(g.M, g.N) * g.njobs >= 144;
+  return g.K % 32 == 0 && g.K1 % 32 == 0 && g.M >= 256 && g.N >= 128 && pipe_tiles<Cfg128>(g.M, g.N) * g.njobs >= 144;
 }
 
 template <class C>
@@ -427,7 +462,7 @@ static hipError_t pipe_direct(const GemmLaunch& g, const char* name, hipStream_t
   const dim3 grid((unsigned)(tiles_m * tiles_n * g.njobs));
   const PipeJobs pj = pipe_jobs(g);
   auto run = [&](auto kernel) {
-    NAYLIS_TIMED(name, st, hipLaunchKernelGGL(kernel, grid, dim3(kNT), 0, st, pj, g.M, g.N, g.K, std::min(g.K1, g.K),
+    NAYLIS_TIMED(name, st, hipLaunchKernelGGL(kernel, grid, dim3(C::NT), 0, st, pj, g.M, g.N, g.K, std::min(g.K1, g.K),
                                               tiles_m, tiles_n, Ranges{}, (float*)nullptr));
   };
   const bool ak = g.job[0].a.kcontig, bk = g.job[0].b.kcontig, f32 = g.out == kGemmOutF32;
@@ -444,11 +479,29 @@ static hipError_t pipe_direct(const GemmLaunch& g, const char* name, hipStream_t
 
 hipError_t launch_gemm_pipe(const GemmLaunch& g, const char* name, hipStream_t st) {
   // 256 x 256 tiles do a step's work at 0.87 of the time of two 256 x 128 ones:
-  // taken unless the smaller tiles save a round (384 tiles, the bank's K / V of
-  // 4096 slots at d 1536: 41 against 54 us; 192 tiles, its d_slots: 62 against 44)
+  // taken unless the smaller tiles save a round (2042 x 5632 over 2048, 352 tiles
+  // against 176: 59 and 52 us; 4096 x 1536 over 1536, 192 against 96: 23 and 42)
   const int r128 = (pipe_tiles<Cfg128>(g.M, g.N) * g.njobs + 255) / 256;
   const int r256 = (pipe_tiles<Cfg256>(g.M, g.N) * g.njobs + 255) / 256;
-  return 2 * r256 * 0.87 < r128 ? pipe_direct<Cfg256>(g, name, st) : pipe_direct<Cfg128>(g, name, st);
+  if (2 * r256 * 0.87 < r128) return pipe_direct<Cfg256>(g, name, st);
+  return g.K % 64 || g.K1 % 64 ? pipe_direct<Cfg128K32>(g, name, st) : pipe_direct<Cfg128>(g, name, st);
+}
+
+// The smallest of the small tiles that needs at most one workgroup per CU: the
+// LDS of one holds a CU, and a second round costs as much as the first (512 x
+// 2816 over 1024: 176 tiles of 64 x 128 take 9.5 us, 352 of 64 x 64 14.5).
+// Against gemm.hip, 2 - 3 workgroups per CU with padded tiles and one stage
+// ahead: 512 x 1024 over 2816 14.7 against 16.4 us, 1021 x 1536 over 1536 11.8
+// against 15.6, 2042 x 2048 over 2048 20.8 against 25.9; at K 512 level (2042 x
+// 512: 5.9 against 6.3), there launch and first loads are all.
+bool gemm_small_ok(const GemmLaunch& g) {
+  return g.K % 64 == 0 && g.K1 % 64 == 0 && g.M >= 8 && g.N >= 8 && pipe_tiles<CfgS128>(g.M, g.N) * g.njobs <= 256;
+}
+
+hipError_t launch_gemm_small(const GemmLaunch& g, const char* name, hipStream_t st) {
+  if (pipe_tiles<CfgS32>(g.M, g.N) * g.njobs <= 256) return pipe_direct<CfgS32>(g, name, st);
+  if (pipe_tiles<CfgS64>(g.M, g.N) * g.njobs <= 256) return pipe_direct<CfgS64>(g, name, st);
+  return pipe_direct<CfgS128>(g, name, st);
 }
 
 // K ranges over one workgroup per CU.
@@ -459,21 +512,21 @@ constexpr int kRangeWgs = 256;
 static Ranges ranges_of(int M, int N, int K) {
   const int tiles = pipe_tiles<Cfg128>(M, N), unit = kRangeWgs / std::gcd(tiles, kRangeWgs);
   Ranges r;
-  r.nk = (K / kBK + unit - 1) / unit * unit;
+  r.nk = ((K + Cfg128::BK - 1) / Cfg128::BK + unit - 1) / unit * unit;
   r.per = (int)((long)tiles * r.nk / kRangeWgs);
   r.stride = r.per / std::gcd(r.per, r.nk);
   return r;
 }
 
-// At least 32 steps a workgroup (at 16 - 22 the fixed costs, 128 KB of partials
+// At least 1024 rows of K a workgroup (at 512 - 704 the fixed costs, 128 KB of partials
 // per workgroup above all, leave it level with gemm.hip's splits or 10 - 20 %
 // behind), few enough tiles that K has to be cut at all, and at most 4 % of the
 // steps empty (unaligned ranges of 10016 tokens, 1024 x 1024: 47 us against 35
 // with gemm.hip's splits).
 bool gemm_ranges_ok(int M, int N, int K) {
-  if (K <= 0 || K % kBK || M < 256 || N < 128 || M % 8 || N % 8 || pipe_tiles<Cfg128>(M, N) >= 144) return false;
+  if (K <= 0 || K % 32 || M < 256 || N < 128 || M % 8 || N % 8 || pipe_tiles<Cfg128>(M, N) >= 144) return false;
   const Ranges r = ranges_of(M, N, K);
-  return r.per >= 32 && (long)(r.nk - K / kBK) * 25 <= K / kBK;
+  return r.per >= 16 && ((long)r.nk * Cfg128::BK - K) * 25 <= K;
 }
 
 size_t gemm_ranges_ws_bytes(int M, int N, int K) {
@@ -485,7 +538,7 @@ hipError_t launch_gemm_ranges(const GemmLaunch& g, const char* name, hipStream_t
   const TileGrid tg{(g.M + C::BM - 1) / C::BM, (g.N + C::BN - 1) / C::BN};
   const Ranges rg = ranges_of(g.M, g.N, g.K);
   NAYLIS_TIMED(name, st,
-               hipLaunchKernelGGL((gemm_pipe_kernel<C, false, false, 2>), dim3(kRangeWgs), dim3(kNT), 0, st,
+               hipLaunchKernelGGL((gemm_pipe_kernel<C, false, false, 2>), dim3(kRangeWgs), dim3(C::NT), 0, st,
                                   pipe_jobs(g), g.M, g.N, g.K, g.K, tg.tiles_m, tg.tiles_n, rg, (float*)g.ws));
   const RangeSum<C> rs{(const float*)g.ws, tg, rg};
   const dim3 grid((unsigned)(((long)g.M * g.N / 4 + 255) / 256));

@@ -33,23 +33,24 @@ bool bf16_products() {
 }
 
 // Where the library's GEMM takes a forward product (whole 128-column tiles):
-// one product up to 2048 x 1024 outputs, where its kernel is within a few us of
-// hipBLASLt's (10.6 against 11.1 us at 2042 x 1024 x 1024, 17.3 against 14.9 at
-// 1021 x 2816 -> 1024) and its host call 6 us against 20; two or three of one
-// input up to 768 tiles of 128 x 128, in one launch (q/k/v of 2042 tokens at d
-// 1024: 20 us against 33; gate/up 1024 -> 2816: 29 against 42; three at 3885
-// tokens: 30 against 41).  Past that hipBLASLt's tiles win (two of 3885 x 1024
-// -> 2816, 1335 tiles: 58 against 48).
+// one product up to 6 M outputs, where its kernel is level with hipBLASLt's or
+// ahead from 1024 rows on (8.6 against 11.2 us at 2042 x 1024 x 1024, 17.0
+// against 22.0 at 2042 x 1024 -> 2816, 22.6 against 22.9 at 4096 x 1536 x 1536;
+// below, up to 6 us behind) and its host call takes 6 us against 20; two or
+// three of one input up to 768 tiles of 128 x 128, in one launch (q/k/v of 2042
+// tokens at d 1024: 17.2 us against 34; gate/up 1024 -> 2816: 29 against 44;
+// three at 3885 tokens: 30 against 41).  Past that hipBLASLt's tiles win (two of
+// 3885 x 1024 -> 2816, 1335 tiles: 50 against 47).
 bool own_fwd(int64_t n, int64_t N, int64_t D_in, int64_t D_out) {
   return N > 0 && D_in % 64 == 0 && D_out % 128 == 0 && D_in <= 2816 &&
-         (n == 1 ? N * D_out <= 2 << 20 : n * N * D_out <= 12 << 20);
+         (n == 1 ? N * D_out <= 6 << 20 : n * N * D_out <= 12 << 20);
 }
 
-// ... and an input gradient: level with hipBLASLt's kernel or ahead of it from
-// 64 rows to 3 M outputs (2042 x 1024 x 1024: 10.2 against 12.2 us; 2042 x 2048
-// x 2048: 27.8 against 23.7).
+// ... and an input gradient: ahead of hipBLASLt's kernel from 64 rows to 6 M
+// outputs (2042 x 1024 x 1024: 9.2 against 12.6 us; 4096 x 1536 x 1536: 23.0
+// against 26.6; past it level, 4096 x 2048 x 2048 33.2 against 34.1).
 bool own_dgrad(int64_t N, int64_t D_in, int64_t D_out) {
-  return N >= 64 && D_in % 128 == 0 && D_out % 64 == 0 && D_out <= 2816 && N * D_in <= 3 << 20;
+  return N >= 64 && D_in % 128 == 0 && D_out % 64 == 0 && D_out <= 2816 && N * D_in <= 6 << 20;
 }
 
 }  // namespace

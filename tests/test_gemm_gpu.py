@@ -273,3 +273,29 @@ def test_linear_routes(dev):
         assert seen == [1]
         traced = torch.jit.trace(mods[0], (x,), check_trace=False)
         assert not torch.equal(traced(x), traced(2 * x))
+
+
+@pytest.mark.parametrize("rows,cols", [(500, 1000), (500, 2824), (1000, 2824)])  # 64 x 64, 64 x 128, 128 x 128 tiles
+@pytest.mark.parametrize("K", [64, 576])                                           # one step; more than any ring holds
+def test_small_tiles(rows, cols, K, dev):
+    """One-round products on the small pipelined tiles, ragged in both directions,
+    in the three operand layouts: weight gradient, forward and input gradient."""
+    import ctypes
+
+    from naylis_amd import _lib
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev).manual_seed(rows + cols + K)
+    r8 = rows // 8 * 8
+    a = torch.randn(rows, K, generator=g, device=dev).bfloat16()
+    w = torch.randn(cols, K, generator=g, device=dev).bfloat16()
+    ref = a.double() @ w.double().t()
+    bound = _sum_bound(a.double(), w.double().t(), ref)
+    got = wgrad(w.t().contiguous(), a[:r8].t().contiguous(), torch.bfloat16).double()
+    assert bool(((got - ref[:r8]).abs() <= bound[:r8]).all())
+    y, dx = (torch.full((rows + 1, cols), 7.0, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    _lib.check(lib.naylis_mom_linear_fwd(a.data_ptr(), (ctypes.c_void_p * 1)(w.data_ptr()),
+                                         (ctypes.c_void_p * 1)(y.data_ptr()), 1, 1, rows, K, cols, st))
+    wt = w.t().contiguous()
+    _lib.check(lib.naylis_mom_linear_dgrad(a.data_ptr(), wt.data_ptr(), dx.data_ptr(), rows, cols, K, st))
+    for out in (y, dx):
+        assert bool(((out[:rows].double() - ref).abs() <= bound).all()) and bool((out[rows] == 7).all())
