@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define NAYLIS_MOM_ABI_VERSION 19
+#define NAYLIS_MOM_ABI_VERSION 20
 
 #define NAYLIS_OK 0
 #define NAYLIS_ERR_ARG 1       /* invalid shape / argument (the reference raises RuntimeError) */
@@ -396,6 +396,10 @@ int naylis_mom_linear_dgrad(const void* dy, const void* w, void* dx, int64_t N, 
 size_t naylis_mom_linear_wgrad_workspace_bytes(int64_t N, int64_t D_in, int64_t D_out);
 int naylis_mom_linear_wgrad(const void* x, const void* dy, void* dw, int dw_dtype, void* workspace,
                             size_t workspace_bytes, int64_t N, int64_t D_in, int64_t D_out, void* stream);
+/* The same for any N (D_in and D_out multiples of 8); its own workspace size. */
+size_t naylis_mom_linear_wgrad_rows_workspace_bytes(int64_t N, int64_t D_in, int64_t D_out);
+int naylis_mom_linear_wgrad_rows(const void* x, const void* dy, void* dw, int dw_dtype, void* workspace,
+                                 size_t workspace_bytes, int64_t N, int64_t D_in, int64_t D_out, void* stream);
 
 /* ------------------------------------------------------------- ReZero ---
  * The layer's output gate (model.py:151 `mom_scale`, applied at model.py:239

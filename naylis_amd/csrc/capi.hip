@@ -850,10 +850,26 @@ static hipError_t launch_wgrad(const GemmLaunch& g, hipStream_t st) {
                                        : launch_gemm(g, "linear_wgrad", st);
 }
 
-static int check_wgrad_dims(int64_t N, int64_t D_in, int64_t D_out) {
+static int check_linear(int64_t N, int64_t D_in, int64_t D_out, const char* who) {
+  if (N < 0 || D_in <= 0 || D_out <= 0 || N > ((int64_t)1 << 30) || D_in > 65536 || D_out > 65536)
+    return fail(NAYLIS_ERR_ARG, "%s: bad shape N=%lld D_in=%lld D_out=%lld", who, (long long)N, (long long)D_in,
+                (long long)D_out);
+  if (D_in % 8 || D_out % 8)
+    return fail(NAYLIS_ERR_ARG, "%s: D_in (%lld) and D_out (%lld) must be multiples of 8", who, (long long)D_in,
+                (long long)D_out);
+  return NAYLIS_OK;
+}
+
+static int check_wgrad_shape(int64_t N, int64_t D_in, int64_t D_out) {
   if (N < 0 || D_in <= 0 || D_out <= 0 || N > ((int64_t)1 << 30) || D_in > 65536 || D_out > 65536)
     return fail(NAYLIS_ERR_ARG, "linear_wgrad: bad shape N=%lld D_in=%lld D_out=%lld", (long long)N, (long long)D_in,
                 (long long)D_out);
+  return NAYLIS_OK;
+}
+
+static int check_wgrad_dims(int64_t N, int64_t D_in, int64_t D_out) {
+  const int rc = check_wgrad_shape(N, D_in, D_out);
+  if (rc) return rc;
   if (N % 8 || D_in % 8 || D_out % 8)
     return fail(NAYLIS_ERR_ARG, "linear_wgrad: N (%lld), D_in (%lld) and D_out (%lld) must be multiples of 8",
                 (long long)N, (long long)D_in, (long long)D_out);
@@ -866,13 +882,11 @@ size_t naylis_mom_linear_wgrad_workspace_bytes(int64_t N, int64_t D_in, int64_t 
   return b ? b : 256;
 }
 
-int naylis_mom_linear_wgrad(const void* x, const void* dy, void* dw, int dw_dtype, void* workspace,
-                            size_t workspace_bytes, int64_t N, int64_t D_in, int64_t D_out, void* stream) {
-  int rc = check_wgrad_dims(N, D_in, D_out);
+static int run_wgrad(const void* x, const void* dy, void* dw, int dw_dtype, void* workspace, size_t workspace_bytes,
+                     int64_t N, int64_t D_in, int64_t D_out, int splits, void* stream) {
+  const int rc = check_dtype(dw_dtype, "linear_wgrad");
   if (rc) return rc;
-  if ((rc = check_dtype(dw_dtype, "linear_wgrad"))) return rc;
   if (!dw || (N > 0 && (!x || !dy))) return fail(NAYLIS_ERR_ARG, "linear_wgrad: null pointer argument");
-  const int splits = wgrad_splits(N, D_in, D_out);
   const size_t need = wgrad_partial_bytes(N, D_in, D_out, splits);
   if (need && (!workspace || workspace_bytes < need))
     return fail(NAYLIS_ERR_WORKSPACE, "linear_wgrad: workspace of %zu bytes is smaller than the %zu required",
@@ -893,19 +907,39 @@ int naylis_mom_linear_wgrad(const void* x, const void* dy, void* dw, int dw_dtyp
   g.job[0].b = GemmOp{x, nullptr, D_in, false};    // B(t, i) = x[t][i]
   g.job[0].c = dw;
   g.job[0].ldc = D_in;
-  if (!gemm_supported(g))
+  GemmLaunch whole = g;  // K (rows here) may be any count: the GEMMs read rows past the last one as zeros
+  whole.K = whole.K1 = (g.K + 7) & ~7;
+  if (!gemm_supported(whole))
     return fail(NAYLIS_ERR_ARG, "linear_wgrad: needs 16-byte aligned pointers and N * max(D_in, D_out) < 2^30");
   return hip_status(launch_wgrad(g, (hipStream_t)stream), "linear_wgrad");
 }
 
-static int check_linear(int64_t N, int64_t D_in, int64_t D_out, const char* who) {
-  if (N < 0 || D_in <= 0 || D_out <= 0 || N > ((int64_t)1 << 30) || D_in > 65536 || D_out > 65536)
-    return fail(NAYLIS_ERR_ARG, "%s: bad shape N=%lld D_in=%lld D_out=%lld", who, (long long)N, (long long)D_in,
-                (long long)D_out);
-  if (D_in % 8 || D_out % 8)
-    return fail(NAYLIS_ERR_ARG, "%s: D_in (%lld) and D_out (%lld) must be multiples of 8", who, (long long)D_in,
-                (long long)D_out);
-  return NAYLIS_OK;
+int naylis_mom_linear_wgrad(const void* x, const void* dy, void* dw, int dw_dtype, void* workspace,
+                            size_t workspace_bytes, int64_t N, int64_t D_in, int64_t D_out, void* stream) {
+  const int rc = check_wgrad_dims(N, D_in, D_out);
+  return rc ? rc : run_wgrad(x, dy, dw, dw_dtype, workspace, workspace_bytes, N, D_in, D_out,
+                             wgrad_splits(N, D_in, D_out), stream);
+}
+
+// Row counts that are no multiple of 8: one tile per workgroup over all rows
+// where that occupies half of the CUs and is not long (hipBLASLt, whose place
+// it takes, sums them in one chain, too), else the splits or ranges of whole
+// counts.  3885 rows, 1024 x 1024: @@ us against 37 with hipBLASLt.
+static int wgrad_rows_splits(int64_t N, int64_t D_in, int64_t D_out) {
+  return N <= 8192 && gemm_small_fills((int)D_out, (int)D_in) ? 1 : wgrad_splits(N, D_in, D_out);
+}
+
+size_t naylis_mom_linear_wgrad_rows_workspace_bytes(int64_t N, int64_t D_in, int64_t D_out) {
+  if (check_wgrad_shape(N, D_in, D_out) || D_in % 8 || D_out % 8) return 0;
+  const size_t b = wgrad_partial_bytes(N, D_in, D_out, wgrad_rows_splits(N, D_in, D_out));
+  return b ? b : 256;
+}
+
+int naylis_mom_linear_wgrad_rows(const void* x, const void* dy, void* dw, int dw_dtype, void* workspace,
+                                 size_t workspace_bytes, int64_t N, int64_t D_in, int64_t D_out, void* stream) {
+  const int rc = check_linear(N, D_in, D_out, "linear_wgrad_rows");
+  return rc ? rc : run_wgrad(x, dy, dw, dw_dtype, workspace, workspace_bytes, N, D_in, D_out,
+                             wgrad_rows_splits(N, D_in, D_out), stream);
 }
 
 static int linear_status(hipError_t e, const char* who) {

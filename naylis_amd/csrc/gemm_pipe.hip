@@ -222,7 +222,7 @@ __global__ __launch_bounds__(C::NT, C::WAVES == 8 ? 2 : 1) void gemm_pipe_kernel
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % C::WM * (32 * C::TM), wn = wave / C::WM * (32 * C::TN);
   constexpr int BK = C::BK;
-  // OUT == 2: rows of K past the last one are out of the operands' resources and read as zeros
+  // where both operands are row-contiguous, rows of K past the last one are out of their resources and read as zeros
   const int nk = (K + BK - 1) / BK, tiles = tiles_m * tiles_n;
   const Frags<AKC, C::BM, C::TM, BK> fa(wm, lane);
   const Frags<BKC, C::BN, C::TN, BK> fb(wn, lane);
@@ -495,7 +495,15 @@ hipError_t launch_gemm_pipe(const GemmLaunch& g, const char* name, hipStream_t s
 // against 15.6, 2042 x 2048 over 2048 20.8 against 25.9; at K 512 level (2042 x
 // 512: 5.9 against 6.3), there launch and first loads are all.
 bool gemm_small_ok(const GemmLaunch& g) {
-  return g.K % 64 == 0 && g.K1 % 64 == 0 && g.M >= 8 && g.N >= 8 && pipe_tiles<CfgS128>(g.M, g.N) * g.njobs <= 256;
+  const bool k_ok = g.K % 64 == 0 && g.K1 % 64 == 0;
+  const bool rows = !g.job[0].a.kcontig && !g.job[0].b.kcontig && g.K1 == g.K;
+  return (k_ok || rows) && g.M >= 8 && g.N >= 8 && pipe_tiles<CfgS128>(g.M, g.N) * g.njobs <= 256;
+}
+
+bool gemm_small_fills(int M, int N) {
+  const int s32 = pipe_tiles<CfgS32>(M, N), s64 = pipe_tiles<CfgS64>(M, N), s128 = pipe_tiles<CfgS128>(M, N);
+  const int n = s32 <= 256 ? s32 : s64 <= 256 ? s64 : s128;
+  return n >= 128 && n <= 256;
 }
 
 hipError_t launch_gemm_small(const GemmLaunch& g, const char* name, hipStream_t st) {
@@ -524,7 +532,7 @@ static Ranges ranges_of(int M, int N, int K) {
 // steps empty (unaligned ranges of 10016 tokens, 1024 x 1024: 47 us against 35
 // with gemm.hip's splits).
 bool gemm_ranges_ok(int M, int N, int K) {
-  if (K <= 0 || K % 32 || M < 256 || N < 128 || M % 8 || N % 8 || pipe_tiles<Cfg128>(M, N) >= 144) return false;
+  if (K <= 0 || M < 256 || N < 128 || M % 8 || N % 8 || pipe_tiles<Cfg128>(M, N) >= 144) return false;
   const Ranges r = ranges_of(M, N, K);
   return r.per >= 16 && ((long)r.nk * Cfg128::BK - K) * 25 <= K;
 }

@@ -62,9 +62,12 @@ hipError_t launch_gemm(const GemmLaunch& g, const char* timer_name, hipStream_t 
 // the gate epilogue included.
 bool gemm_pipe_ok(const GemmLaunch& g);
 hipError_t launch_gemm_pipe(const GemmLaunch& g, const char* timer_name, hipStream_t st);
-// The same kernel on 128 x 128, 64 x 128 and 64 x 64 tiles (K a multiple of 64).
+// The same kernel on 128 x 128, 64 x 128 and 64 x 64 tiles (K a multiple of 64,
+// or any where both operands are row-contiguous), at most one per CU.
 bool gemm_small_ok(const GemmLaunch& g);
 hipError_t launch_gemm_small(const GemmLaunch& g, const char* timer_name, hipStream_t st);
+// whether an M x N product of one job gives them to at least half of the CUs
+bool gemm_small_fills(int M, int N);
 bool gemm_ranges_ok(int M, int N, int K);
 size_t gemm_ranges_ws_bytes(int M, int N, int K);
 hipError_t launch_gemm_ranges(const GemmLaunch& g, const char* timer_name, hipStream_t st);

@@ -51,7 +51,7 @@ std::vector<at::Tensor> linear_fwd(const at::Tensor& x, const std::vector<at::Te
 at::Tensor linear_dgrad(const at::Tensor& dy, const at::Tensor& w, void* st);
 
 // dW = dy^T xin over all rows: the library's GEMM when N, D_in, D_out are
-// multiples of 8, else torch's product (the hip_linear.library_wgrad rule)
+// multiples of 8 (any row count of plain bf16 operands), else torch's product
 at::Tensor library_wgrad(const at::Tensor& xin, const at::Tensor& dy, at::ScalarType dtype, void* st);
 
 // y2 = out2 (s W_o)^T in fp32 and the scaled weight; its backward (d out2, dW_o, ds)

@@ -93,14 +93,23 @@ at::Tensor linear_dgrad(const at::Tensor& dy, const at::Tensor& w, void* st) {
 
 at::Tensor library_wgrad(const at::Tensor& xin, const at::Tensor& dy, at::ScalarType dtype, void* st) {
   const int64_t N = xin.size(0), D_in = xin.size(1), D_out = dy.size(1);
+  const auto grad = [&] { return at::empty({D_out, D_in}, xin.options().dtype(dtype)); };
+  const int code = dtype == at::kBFloat16 ? kBF16 : kF32;
   if (N % 8 || D_in % 8 || D_out % 8) {
+    if (N % 8 && D_in % 8 == 0 && D_out % 8 == 0 && N * std::max(D_in, D_out) < 1 << 29 && plain_bf16(xin) &&
+        plain_bf16(dy) && bf16_products()) {
+      at::Tensor ws = workspace(naylis_mom_linear_wgrad_rows_workspace_bytes(N, D_in, D_out), xin), dw = grad();
+      check(naylis_mom_linear_wgrad_rows(xin.data_ptr(), dy.data_ptr(), dw.data_ptr(), code, ws.data_ptr(), ws.numel(),
+                                         N, D_in, D_out, st));
+      return dw;
+    }
     if (dtype == at::kFloat) return at::mm(dy.t(), xin, at::kFloat);
     return at::mm(dy.t(), xin).to(dtype);
   }
   at::Tensor ws = workspace(naylis_mom_linear_wgrad_workspace_bytes(N, D_in, D_out), xin);
-  at::Tensor dw = at::empty({D_out, D_in}, xin.options().dtype(dtype));
-  check(naylis_mom_linear_wgrad(xin.data_ptr(), dy.data_ptr(), dw.data_ptr(), dtype == at::kBFloat16 ? kBF16 : kF32,
-                                ws.data_ptr(), ws.numel(), N, D_in, D_out, st));
+  at::Tensor dw = grad();
+  check(naylis_mom_linear_wgrad(xin.data_ptr(), dy.data_ptr(), dw.data_ptr(), code, ws.data_ptr(), ws.numel(), N, D_in,
+                                D_out, st));
   return dw;
 }
 

@@ -299,3 +299,24 @@ def test_small_tiles(rows, cols, K, dev):
     _lib.check(lib.naylis_mom_linear_dgrad(a.data_ptr(), wt.data_ptr(), dx.data_ptr(), rows, cols, K, st))
     for out in (y, dx):
         assert bool(((out[:rows].double() - ref).abs() <= bound).all()) and bool((out[rows] == 7).all())
+
+
+@pytest.mark.parametrize("N", [1, 61, 3885, 16381])
+@pytest.mark.parametrize("D_in,D_out", [(1024, 1024), (264, 520), (2824, 1000)])
+def test_linear_wgrad_rows(N, D_in, D_out, dev):
+    """Row counts that are no multiple of 8: one tile per workgroup, K splits and K ranges."""
+    from naylis_amd import _lib
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev).manual_seed(N + D_in)
+    # the next rows hold infinities: none may be read into a sum
+    x, dy = (torch.cat([torch.randn(N, d, generator=g, device=dev), torch.full((64, d), float("inf"), device=dev)])
+             .bfloat16() for d in (D_in, D_out))
+    nb = lib.naylis_mom_linear_wgrad_rows_workspace_bytes(N, D_in, D_out)
+    ws = torch.empty(nb, dtype=torch.uint8, device=dev)
+    a, b = dy[:N].double().t(), x[:N].double()
+    ref = a @ b
+    for code, dtype in ((0, torch.float32), (1, torch.bfloat16)):
+        dw = torch.empty(D_out, D_in, device=dev, dtype=dtype)
+        _lib.check(lib.naylis_mom_linear_wgrad_rows(x.data_ptr(), dy.data_ptr(), dw.data_ptr(), code, ws.data_ptr(), nb,
+                                                    N, D_in, D_out, st))
+        assert bool(((dw.double() - ref).abs() <= _sum_bound(a, b, ref)).all())
