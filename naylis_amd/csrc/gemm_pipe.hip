@@ -47,12 +47,14 @@ struct PipeCfg {
   static constexpr int ABYTES = BM * BK * 2, STAGE = ABYTES + BN * BK * 2;
   // 1 KB pieces of A and B that a wave loads of each stage
   static constexpr int NA = ABYTES / 1024 / WAVES, NB = (STAGE - ABYTES) / 1024 / WAVES;
+  static constexpr bool A_ROWS = (BM & (BM - 1)) == 0;  // the XOR of row-contiguous A needs it
   static constexpr int FLIGHT = (RING - 2) * (NA + NB);  // loads in flight past the stage waited for
   static_assert(NA * WAVES * 1024 == ABYTES && NB * WAVES * 1024 == STAGE - ABYTES && RING * STAGE <= 160 * 1024);
 };
 using Cfg128 = PipeCfg<8, 4, 2, 2, 64, 3>;     // 256 x 128
 using Cfg128K32 = PipeCfg<8, 4, 2, 2, 32, 6>;  // ... for an odd number of 32s of K
 using Cfg256 = PipeCfg<8, 2, 4, 2, 32, 5>;     // 256 x 256
+using Cfg192 = PipeCfg<8, 2, 3, 2, 64, 2>;     // 192 x 256, K-contiguous A only
 // Products of at most one of these per CU.  They are bound by latency (one
 // step: a barrier, an LDS read and 4 dependent products) and by what one CU
 // draws from L2, so stages are deep (6 - 8 of 16 - 24 KB) and 128 x 128 and 64 x
@@ -470,6 +472,8 @@ static hipError_t pipe_direct(const GemmLaunch& g, const char* name, hipStream_t
     f32 ? run(gemm_pipe_kernel<C, true, true, 0>) : run(gemm_pipe_kernel<C, true, true, 1>);
   else if (ak)
     f32 ? run(gemm_pipe_kernel<C, true, false, 0>) : run(gemm_pipe_kernel<C, true, false, 1>);
+  else if constexpr (!C::A_ROWS)
+    return hipErrorInvalidValue;
   else if (bk)
     f32 ? run(gemm_pipe_kernel<C, false, true, 0>) : run(gemm_pipe_kernel<C, false, true, 1>);
   else
@@ -483,8 +487,15 @@ hipError_t launch_gemm_pipe(const GemmLaunch& g, const char* name, hipStream_t s
   // against 176: 59 and 52 us; 4096 x 1536 over 1536, 192 against 96: 23 and 42)
   const int r128 = (pipe_tiles<Cfg128>(g.M, g.N) * g.njobs + 255) / 256;
   const int r256 = (pipe_tiles<Cfg256>(g.M, g.N) * g.njobs + 255) / 256;
+  const bool k64 = g.K % 64 == 0 && g.K1 % 64 == 0;
+  // 192 x 256 tiles, where they take fewer rounds than the small ones and no
+  // more than the large: 2 x 2042 x 2816 over 1024 (352, 242 and 176 tiles)
+  // 33.2 us with 256 x 128, 27.4 with these, 30.2 with 256 x 256; 3 x 4096 x
+  // 2816 (1056, 726, 528) 77 against 90 with 256 x 256
+  const int r192 = (pipe_tiles<Cfg192>(g.M, g.N) * g.njobs + 255) / 256;
+  if (g.job[0].a.kcontig && k64 && r192 * 1.35 < r128 && r192 <= r256) return pipe_direct<Cfg192>(g, name, st);
   if (2 * r256 * 0.87 < r128) return pipe_direct<Cfg256>(g, name, st);
-  return g.K % 64 || g.K1 % 64 ? pipe_direct<Cfg128K32>(g, name, st) : pipe_direct<Cfg128>(g, name, st);
+  return k64 ? pipe_direct<Cfg128>(g, name, st) : pipe_direct<Cfg128K32>(g, name, st);
 }
 
 // The smallest of the small tiles that needs at most one workgroup per CU: the
@@ -497,13 +508,16 @@ hipError_t launch_gemm_pipe(const GemmLaunch& g, const char* name, hipStream_t s
 bool gemm_small_ok(const GemmLaunch& g) {
   const bool k_ok = g.K % 64 == 0 && g.K1 % 64 == 0;
   const bool rows = !g.job[0].a.kcontig && !g.job[0].b.kcontig && g.K1 == g.K;
-  return (k_ok || rows) && g.M >= 8 && g.N >= 8 && pipe_tiles<CfgS128>(g.M, g.N) * g.njobs <= 256;
+  // with two row-contiguous operands a full chip of 128 x 128 tiles is bound by
+  // LDS reads: the 64 x 64 blocks per wave of gemm.hip's tile read a third less
+  // (2048 x 2048 over 2008: 27.1 against 29.3 us)
+  return (k_ok || rows) && g.M >= 8 && g.N >= 8 && pipe_tiles<CfgS128>(g.M, g.N) * g.njobs <= (rows ? 255 : 256);
 }
 
 bool gemm_small_fills(int M, int N) {
   const int s32 = pipe_tiles<CfgS32>(M, N), s64 = pipe_tiles<CfgS64>(M, N), s128 = pipe_tiles<CfgS128>(M, N);
   const int n = s32 <= 256 ? s32 : s64 <= 256 ? s64 : s128;
-  return n >= 128 && n <= 256;
+  return n >= 128 && n <= 255;
 }
 
 hipError_t launch_gemm_small(const GemmLaunch& g, const char* name, hipStream_t st) {

@@ -275,7 +275,8 @@ def test_linear_routes(dev):
         assert not torch.equal(traced(x), traced(2 * x))
 
 
-@pytest.mark.parametrize("rows,cols", [(500, 1000), (500, 2824), (1000, 2824)])  # 64 x 64, 64 x 128, 128 x 128 tiles
+@pytest.mark.parametrize("rows,cols", [(500, 1000), (500, 2824), (1000, 2824),  # 64 x 64, 64 x 128, 128 x 128 tiles
+                                       (4100, 2824)])                           # 192 x 256, 256 x 128
 @pytest.mark.parametrize("K", [64, 576])                                           # one step; more than any ring holds
 def test_small_tiles(rows, cols, K, dev):
     """One-round products on the small pipelined tiles, ragged in both directions,
