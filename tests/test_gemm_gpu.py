@@ -275,6 +275,25 @@ def test_linear_routes(dev):
         assert not torch.equal(traced(x), traced(2 * x))
 
 
+@pytest.mark.parametrize("grad", [False, True])
+def test_traced_modules_follow_their_input(grad, dev):
+    """A traced norm and projection run their kernels on the inputs of each call
+    (bit for bit the eager results, gradients among them)."""
+    from naylis_amd.mom_kernels.hip_linear import NaylisLinear
+    from naylis_amd.mom_kernels.hip_norm import NaylisRMSNorm
+    block = torch.nn.Sequential(NaylisRMSNorm(512), NaylisLinear(512, 512, bias=False)).to(dev, torch.bfloat16)
+    g = torch.Generator(device=dev).manual_seed(5)
+    a, b = (torch.randn(64, 512, generator=g, device=dev).bfloat16().requires_grad_(grad) for _ in range(2))
+    with torch.set_grad_enabled(grad):
+        traced = torch.jit.trace(block, (a,), check_trace=False)
+        y, want = traced(b), block(b)
+        assert torch.equal(y, want)
+        if grad:
+            ins = (b, *block.parameters())
+            for p, q in zip(torch.autograd.grad(y, ins, y.detach()), torch.autograd.grad(want, ins, y.detach())):
+                assert torch.equal(p, q)
+
+
 @pytest.mark.parametrize("rows,cols", [(500, 1000), (500, 2824), (1000, 2824),  # 64 x 64, 64 x 128, 128 x 128 tiles
                                        (4100, 2824)])                           # 192 x 256, 256 x 128
 @pytest.mark.parametrize("K", [64, 576])                                           # one step; more than any ring holds
