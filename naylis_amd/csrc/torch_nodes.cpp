@@ -85,7 +85,9 @@ std::vector<at::Tensor> linear_fwd(const at::Tensor& x, const std::vector<at::Te
 
 at::Tensor linear_dgrad(const at::Tensor& dy, const at::Tensor& w, void* st) {
   const int64_t N = dy.size(0), D_out = w.size(0), D_in = w.size(1);
-  if (!own_dgrad(N, D_in, D_out) || !plain_bf16(dy) || !plain_bf16(w) || !bf16_products()) return at::mm(dy, w);
+  // in grad mode (a backward with create_graph) the product itself is differentiated
+  if (!own_dgrad(N, D_in, D_out) || !plain_bf16(dy) || !plain_bf16(w) || !bf16_products() || at::GradMode::is_enabled())
+    return at::mm(dy, w);
   at::Tensor dx = at::empty({N, D_in}, dy.options());
   check(naylis_mom_linear_dgrad(dy.data_ptr(), w.data_ptr(), dx.data_ptr(), N, D_in, D_out, st));
   return dx;
@@ -97,7 +99,7 @@ at::Tensor library_wgrad(const at::Tensor& xin, const at::Tensor& dy, at::Scalar
   const int code = dtype == at::kBFloat16 ? kBF16 : kF32;
   if (N % 8 || D_in % 8 || D_out % 8) {
     if (N % 8 && D_in % 8 == 0 && D_out % 8 == 0 && N * std::max(D_in, D_out) < 1 << 29 && plain_bf16(xin) &&
-        plain_bf16(dy) && bf16_products()) {
+        plain_bf16(dy) && bf16_products() && !at::GradMode::is_enabled()) {
       at::Tensor ws = workspace(naylis_mom_linear_wgrad_rows_workspace_bytes(N, D_in, D_out), xin), dw = grad();
       check(naylis_mom_linear_wgrad_rows(xin.data_ptr(), dy.data_ptr(), dw.data_ptr(), code, ws.data_ptr(), ws.numel(),
                                          N, D_in, D_out, st));

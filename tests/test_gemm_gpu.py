@@ -275,6 +275,21 @@ def test_linear_routes(dev):
         assert not torch.equal(traced(x), traced(2 * x))
 
 
+def test_linear_second_derivative(dev):
+    """A gradient taken with create_graph: the input gradient g = dy W stays a
+    product that autograd knows, d(sum(g^2) / 2)/d dy = g W^T."""
+    from naylis_amd import mom_kernels
+    g = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn(128, 256, generator=g, device=dev).bfloat16().requires_grad_(True)
+    w = (torch.randn(384, 256, generator=g, device=dev) * 0.05).bfloat16().requires_grad_(True)
+    dy = torch.randn(128, 384, generator=g, device=dev).bfloat16().requires_grad_(True)
+    dx, = torch.autograd.grad(mom_kernels.mom_linear(x, w), x, dy, create_graph=True)
+    got, = torch.autograd.grad(dx, dy, dx.detach())
+    a, b = dx.detach().double(), w.detach().double().t()
+    ref = a @ b
+    assert bool(((got.double() - ref).abs() <= _sum_bound(a, b, ref)).all())
+
+
 @pytest.mark.parametrize("grad", [False, True])
 def test_traced_modules_follow_their_input(grad, dev):
     """A traced norm and projection run their kernels on the inputs of each call
