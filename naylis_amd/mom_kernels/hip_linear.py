@@ -20,6 +20,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 from torch.autograd import forward_ad
+from torch.nn.modules import module as _modules
 
 from .. import _lib, _torch_ext
 
@@ -63,6 +64,14 @@ def _untransformed(x, *weights):
             and torch._C._get_tracing_state() is None)
 
 
+def _plain_module(m):
+    """A NaylisLinear whose call is its forward and nothing else: no hooks, its
+    own or for all modules, and no forward put on the instance."""
+    return (type(m) is NaylisLinear and "forward" not in m.__dict__ and not m._forward_hooks
+            and not m._forward_pre_hooks and not _modules._global_forward_hooks
+            and not _modules._global_forward_pre_hooks)
+
+
 def mom_linear(x, weight):
     """y = x W^T (no bias).  For bf16 activations and weights on a ROCm device
     with dimensions that are multiples of 8 the weight gradient runs on the
@@ -88,8 +97,7 @@ def shared_input_linear(x, linears):
     if len(linears) <= 3 and all(m.bias is None for m in linears):
         ws = [m.weight for m in linears]
         if not torch.is_grad_enabled():
-            if _untransformed(x, *ws) and all(type(m) is NaylisLinear and not m._forward_hooks
-                                              and not m._forward_pre_hooks and _library_ok(x, w, 1)
+            if _untransformed(x, *ws) and all(_plain_module(m) and _library_ok(x, w, 1)
                                               for m, w in zip(linears, ws)):
                 return tuple(_torch_ext.load().linear(x, ws, False, _lib.stream_of(x.device)))
         elif all(_library_ok(x, w) for w in ws) and any(w.requires_grad for w in ws):

@@ -275,6 +275,20 @@ def test_linear_routes(dev):
         assert not torch.equal(traced(x), traced(2 * x))
 
 
+def test_linear_keeps_global_hooks_and_replaced_forwards(dev):
+    from naylis_amd.mom_kernels.hip_linear import NaylisLinear, shared_input_linear
+    mods = [NaylisLinear(256, 384, bias=False).to(dev, torch.bfloat16) for _ in range(2)]
+    x = torch.randn(16, 256, device=dev).bfloat16()
+    with torch.no_grad():
+        seen = []
+        h = torch.nn.modules.module.register_module_forward_hook(lambda m, i, o: seen.append(m))
+        shared_input_linear(x, mods)
+        h.remove()
+        assert seen == mods
+        mods[1].forward = lambda x: torch.zeros(1)
+        assert shared_input_linear(x, mods)[1].numel() == 1
+
+
 def test_linear_second_derivative(dev):
     """A gradient taken with create_graph: the input gradient g = dy W stays a
     product that autograd knows, d(sum(g^2) / 2)/d dy = g W^T."""
