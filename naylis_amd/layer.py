@@ -111,10 +111,9 @@ class MoMLayer(nn.Module):
             # g = -log(-log(u + 1e-9) + 1e-9) and logits + noise_scale * g
             noise = torch.rand((B, S, self.num_blocks), device=x.device, dtype=torch.float32)
         ckpt = self.mom_grad_ckpt and self.training and torch.is_grad_enabled()
-        if (not ckpt or hip_layer.cpp_node()) and fused_layer_supported(x, M_blocks, self.router_down.weight, self.router_up.weight,
-                                                                       self.q_proj.weight, self.k_proj.weight,
-                                                                       self.v_proj.weight, self.o_proj.weight,
-                                                                       self.mom_scale, bank_kv):
+        if (not ckpt or hip_layer.ckpt_node()) and fused_layer_supported(
+                x, M_blocks, self.router_down.weight, self.router_up.weight, self.q_proj.weight, self.k_proj.weight,
+                self.v_proj.weight, self.o_proj.weight, self.mom_scale, bank_kv):
             # one autograd node for router + bank + q + read + o + ReZero
             y, router_probs, top_idx = mom_layer(
                 x, M_blocks, self.router_down.weight, self.router_up.weight, self.q_proj.weight,

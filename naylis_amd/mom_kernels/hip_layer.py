@@ -47,6 +47,14 @@ def cpp_node():
     return USE_TORCH_EXT and USE_CPP_NODE
 
 
+def ckpt_node():
+    """True where the node takes a gradient-checkpointed layer too: the C++ node,
+    outside autocast to another type than bf16 (torch.utils.checkpoint then
+    runs the projection in that type both times)."""
+    return cpp_node() and (not torch.is_autocast_enabled("cuda")
+                           or torch.get_autocast_dtype("cuda") == torch.bfloat16)
+
+
 def _ws(nbytes, dev):
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=dev)
 

@@ -309,6 +309,15 @@ def test_layer_external_bank_matches_own_projection(fused, dev, monkeypatch):
         assert torch.equal(g0[n], g1[n]), n
 
 
+def test_ckpt_node_leaves_other_autocast_types(dev):
+    from naylis_amd.mom_kernels import hip_layer
+    assert hip_layer.ckpt_node()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert hip_layer.ckpt_node()
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert not hip_layer.ckpt_node()
+
+
 @pytest.mark.parametrize("case", EXT_CASES, ids=[f"case{i}" for i in range(len(EXT_CASES))])
 def test_layer_ckpt_node_is_exact(case, dev):
     """The node's gradient checkpointing (the read's inputs kept, the read run
