@@ -4,9 +4,10 @@
 // router, bank K/V, q projection, token order, gated read, o projection with
 // the folded ReZero gate, and their gradients -- as one call each from
 // Python instead of about fifteen ctypes and torch calls.  They make the same
-// library calls in the same order, with the same allocations and torch GEMMs
-// (hipBLASLt through at::mm / at::linear on torch's current stream), so their
-// results are bitwise those of the Python node.
+// library calls in the same order, with the same allocations and products
+// (linear_fwd / linear_dgrad: the library's GEMM, or hipBLASLt through at::mm /
+// at::linear on torch's current stream), so their results are bitwise those of
+// the Python node.
 //
 // MomLayerNode is the same node as a C++ autograd function: its forward
 // calls layer_fwd and saves what the Python node saves, its backward calls

@@ -11,8 +11,8 @@ between the two unchanged.  The forward is
     out   = mom_read(q_proj(x), K, V, idx, gates)       # gated flash read
     y     = mom_scale * o_proj(out)
 
-q_proj / o_proj run their forward and input gradient as torch GEMMs
-(hipBLASLt) and their weight gradient on the library's split-K GEMM.  In the
+q_proj / o_proj run their weight gradient on the library's GEMM, forward and
+input gradient on it or as torch GEMMs (hipBLASLt), by size.  In the
 common training case (bf16 activations and projection weights) the whole
 forward is one autograd node (``mom_kernels.hip_layer``) whose backward orders
 the library calls so the router's input gradient accumulates into the q

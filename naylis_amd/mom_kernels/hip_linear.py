@@ -3,16 +3,18 @@ gradient on the library's split-K MFMA GEMM (C ABI: naylis_mom_linear_wgrad).
 
 model.py:239 (`q_proj`) and model.py:251 (`o_proj`) are nn.Linear(d, d,
 bias=False); the reference takes their weight gradient from autograd, a
-dy^T x reduction over all B*T tokens.  Here the forward product and the input
-gradient stay torch GEMMs (hipBLASLt); the weight gradient is
-naylis_mom_linear_wgrad, deterministic (fixed-order split-K reduction).
+dy^T x reduction over all B*T tokens.  Here the weight gradient is
+naylis_mom_linear_wgrad, deterministic (fixed-order reduction over K ranges or
+splits).  The forward product and the input gradient run on the library's GEMM
+at the sizes where it is ahead (csrc/torch_nodes.cpp: own_fwd, own_dgrad), as
+torch GEMMs (hipBLASLt) otherwise.
 
 The decoder trunk's projections (the Llama attention's q/k/v/o and the MLP's
 gate/up/down inside every Naylis decoder layer, model.py:279-345) are the same
 bias-free nn.Linear; ``NaylisLinear`` / ``use_library_wgrad`` give them this
 weight gradient too.  At the config-3 shapes (16384 tokens) hipBLASLt's
 weight-gradient GEMM runs d x d at about 340 TFLOP/s and d x 2816 at about
-620, the library's split-K kernel at about 680 and 750.
+620, the library's at about 800 and 950.
 """
 from __future__ import annotations
 
