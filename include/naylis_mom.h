@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define NAYLIS_MOM_ABI_VERSION 20
+#define NAYLIS_MOM_ABI_VERSION 21
 
 #define NAYLIS_OK 0
 #define NAYLIS_ERR_ARG 1       /* invalid shape / argument (the reference raises RuntimeError) */
@@ -419,6 +419,10 @@ int naylis_mom_rezero_bwd(const void* dy, int dy_dtype, const void* z, int z_dty
  * s then follow from dW' (the gradient of W') by naylis_mom_rezero_bwd over
  * the weight's elements: dW_o = s * dW', ds = sum(dW' * W_o). */
 int naylis_mom_rezero_scale(const void* x, int x_dtype, const float* s, void* y, int y_dtype, int64_t n, void* stream);
+/* a = bf16(dy) and b = bf16(s * dy) in one pass over n elements of dy (a may
+ * be NULL): the o projection's backward where naylis_mom_gated_wgrad does not
+ * apply takes dW' from a and the gradient of its input, b W_o, from b. */
+int naylis_mom_rezero_round(const void* dy, int dy_dtype, const float* s, void* a, void* b, int64_t n, void* stream);
 /* The two steps above in one call for the layer's backward (the o projection's
  * weight gradient, model.py:251, with the gate of model.py:239 folded in):
  *   dW'[o][i] = sum_t dy[t][o] * x[t][i]   (fp32, as naylis_mom_linear_wgrad)

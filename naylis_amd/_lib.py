@@ -14,7 +14,7 @@ import threading
 
 LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libnaylis_mom.so")
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 NAYLIS_OK = 0
 NAYLIS_ERR_ARG = 1
@@ -68,6 +68,7 @@ SIGNATURES = {
     "naylis_mom_rezero_fwd": (_int, [_c_void_p, _int, _c_void_p, _c_void_p, _i64, _c_void_p]),
     "naylis_mom_rezero_bwd": (_int, [_c_void_p, _int, _c_void_p, _int] + [_c_void_p] * 4 + [_size_t, _i64, _c_void_p]),
     "naylis_mom_rezero_scale": (_int, [_c_void_p, _int, _c_void_p, _c_void_p, _int, _i64, _c_void_p]),
+    "naylis_mom_rezero_round": (_int, [_c_void_p, _int, _c_void_p, _c_void_p, _c_void_p, _i64, _c_void_p]),
     "naylis_mom_linear_fwd": (_int, [_c_void_p, _pp, _pp, _int, _int] + [_i64] * 3 + [_c_void_p]),
     "naylis_mom_linear_dgrad": (_int, [_c_void_p] * 3 + [_i64] * 3 + [_c_void_p]),
     "naylis_mom_linear_wgrad_rows_workspace_bytes": (_size_t, [_i64] * 3),

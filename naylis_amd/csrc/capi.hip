@@ -1057,6 +1057,16 @@ int naylis_mom_rezero_scale(const void* x, int x_dtype, const float* s, void* y,
                     "rezero_scale");
 }
 
+int naylis_mom_rezero_round(const void* dy, int dy_dtype, const float* s, void* a, void* b, int64_t n, void* stream) {
+  int rc;
+  if (n < 0) return fail(NAYLIS_ERR_ARG, "rezero_round: negative size %lld", (long long)n);
+  if ((rc = check_dtype(dy_dtype, "rezero_round"))) return rc;
+  if (n == 0) return NAYLIS_OK;
+  if (!dy || !s || !b) return fail(NAYLIS_ERR_ARG, "rezero_round: null pointer argument");
+  return hip_status(launch_rezero_round(dy, dy_dtype == NAYLIS_DTYPE_BF16, s, a, b, (long)n, (hipStream_t)stream),
+                    "rezero_round");
+}
+
 int naylis_mom_rezero_bwd(const void* dy, int dy_dtype, const void* z, int z_dtype, const float* s, void* dz, float* ds,
                           void* workspace, size_t workspace_bytes, int64_t n, void* stream) {
   int rc;

@@ -12,6 +12,8 @@
 // layer then gets y straight from one GEMM with an fp32 result, and the
 // backward's dW = s * dW' and ds = sum(W * dW'), dW' the gradient of the
 // scaled weight, are this file's backward run over the weight's elements.
+// d out = (s dy) W for the latter's rows that have no gate epilogue takes both
+// roundings of dy from rezero_round.
 #include "common.h"
 #include "launch_rezero.h"
 #include "timing.h"
@@ -98,6 +100,43 @@ __global__ __launch_bounds__(kRzThreads) void rezero_fwd_kernel(const ZT* __rest
     const long i = base + ((long)st * kRzThreads + threadIdx.x) * kRzVec;
     for (int e = 0; e < kRzVec; ++e)
       if (i + e < n) st1<YT>(y + i + e, sc * ld1<ZT>(z + i + e));
+  }
+}
+
+// a = bf16(dy) and b = bf16(s dy) in one pass (a may be NULL): the operands of
+// the o projection's backward at row counts whose weight gradient has no gate
+// epilogue.  d out = b W_o then reads the weight itself; through bf16(s W_o) it
+// would carry a third rounding (2.4e-3 against 2.2e-3 in the bank's gradient
+// at s 0.37, 3885 tokens, d 1024).  Bound by HBM: 2 bytes a value more than
+// the cast of dy that it takes the place of.
+template <typename DT>
+__global__ __launch_bounds__(kRzThreads) void rezero_round_kernel(const DT* __restrict__ dy, const float* __restrict__ s,
+                                                                  bf16_t* __restrict__ a, bf16_t* __restrict__ b, long n,
+                                                                  int vec) {
+  const float sc = *s;
+  const long base = (long)blockIdx.x * kRzChunk;
+  if (vec && base + kRzChunk <= n) {  // whole chunk: every load issued before the first store
+    float v[kRzSteps][8];
+#pragma unroll
+    for (int st = 0; st < kRzSteps; ++st) ld8<DT>(dy + base + ((long)st * kRzThreads + threadIdx.x) * kRzVec, v[st]);
+#pragma unroll
+    for (int st = 0; st < kRzSteps; ++st) {
+      const long i = base + ((long)st * kRzThreads + threadIdx.x) * kRzVec;
+      if (a) st8<bf16_t>(a + i, v[st]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[st][e] *= sc;
+      st8<bf16_t>(b + i, v[st]);
+    }
+    return;
+  }
+  for (int st = 0; st < kRzSteps; ++st) {
+    const long i = base + ((long)st * kRzThreads + threadIdx.x) * kRzVec;
+    for (int e = 0; e < kRzVec; ++e)
+      if (i + e < n) {
+        const float g = ld1<DT>(dy + i + e);
+        if (a) st1<bf16_t>(a + i + e, g);
+        st1<bf16_t>(b + i + e, sc * g);
+      }
   }
 }
 
@@ -198,6 +237,20 @@ hipError_t launch_rezero_scale(const void* z, bool z_bf16, const float* s, void*
 
 hipError_t launch_rezero_fwd(const void* z, bool z_bf16, const float* s, float* y, long n, hipStream_t st) {
   return launch_rezero_scale(z, z_bf16, s, y, false, n, st);
+}
+
+hipError_t launch_rezero_round(const void* dy, bool dy_bf16, const float* s, void* a, void* b, long n, hipStream_t st) {
+  if (n == 0) return hipSuccess;
+  const int vec = ((uintptr_t)dy & 15) == 0 && ((uintptr_t)a & 15) == 0 && ((uintptr_t)b & 15) == 0;
+  if (dy_bf16)
+    NAYLIS_TIMED("rezero_bwd", st,
+                 hipLaunchKernelGGL(rezero_round_kernel<bf16_t>, dim3(n_chunks(n)), dim3(kRzThreads), 0, st,
+                                    (const bf16_t*)dy, s, (bf16_t*)a, (bf16_t*)b, n, vec));
+  else
+    NAYLIS_TIMED("rezero_bwd", st,
+                 hipLaunchKernelGGL(rezero_round_kernel<float>, dim3(n_chunks(n)), dim3(kRzThreads), 0, st,
+                                    (const float*)dy, s, (bf16_t*)a, (bf16_t*)b, n, vec));
+  return hipGetLastError();
 }
 
 template <typename ZT, typename DT>

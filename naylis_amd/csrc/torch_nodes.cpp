@@ -125,10 +125,21 @@ std::pair<at::Tensor, at::Tensor> gated_linear_forward(const at::Tensor& out2, c
 
 GatedGrads gated_linear_backward(const at::Tensor& dy, const at::Tensor& out2, const at::Tensor& w_o,
                                  const at::Tensor& w_os, const at::Tensor& s, void* st) {
-  const at::Tensor dy2 = dy.to(at::kBFloat16).contiguous();
+  const int64_t N = out2.size(0), D_in = out2.size(1), D_out = dy.size(1);
   GatedGrads g;
-  g.dout2 = linear_dgrad(dy2, w_os, st);
-  const int64_t N = out2.size(0), D_in = out2.size(1), D_out = dy2.size(1);
+  at::Tensor dy2;
+  if (N % 8 == 0) {
+    dy2 = dy.to(at::kBFloat16).contiguous();
+    g.dout2 = linear_dgrad(dy2, w_os, st);
+  } else {  // d out from bf16(s dy) and W_o, one rounding less than from bf16(dy) and bf16(s W_o)
+    const at::Tensor d = dy.contiguous();
+    at::Tensor dz = at::empty({N, D_out}, d.options().dtype(at::kBFloat16));
+    const bool cast = d.scalar_type() != at::kBFloat16;
+    dy2 = cast ? at::empty_like(dz) : d;
+    check(naylis_mom_rezero_round(d.data_ptr(), dtype_code(d), s.data_ptr<float>(), cast ? dy2.data_ptr() : nullptr,
+                                  dz.data_ptr(), d.numel(), st));
+    g.dout2 = linear_dgrad(dz, w_o, st);
+  }
   g.dw_o = at::empty_like(w_o);
   g.ds = at::empty({1}, out2.options().dtype(at::kFloat));
   if (out2.scalar_type() == at::kBFloat16 && w_o.scalar_type() == at::kBFloat16 && w_o.is_contiguous() &&

@@ -11,7 +11,8 @@ folds into the projection's weight: s * (out W_o^T) = out (s W_o)^T.  The
 layer's fp32 output is then one GEMM with an fp32 result instead of a bf16
 GEMM result that is scaled, stored and read back; backward, d out = dy W',
 dW' = dy^T out in fp32, and dW_o = s dW', ds = sum(dW' W_o) come from the
-ReZero backward kernel run over the weight's elements
+ReZero backward kernel run over the weight's elements.  Row counts that are no
+multiple of 8 take d out = (s dy) W_o, which rounds one operand less
 (``gated_linear_forward`` / ``gated_linear_backward``, shared by the fused
 layer node and ``mom_gated_linear``).
 """
@@ -38,10 +39,20 @@ def gated_linear_backward(lib, dy2, out2, w_o, w_os, s, st):
     """(d out2, dW_o, ds) of y2 = out2 (s W_o)^T for the upstream gradient dy2
     (rows = tokens, rounded to bf16 for the two GEMMs)."""
     dev = out2.device
-    dy2 = dy2.to(torch.bfloat16).contiguous()
-    dout2 = _torch_ext.load().linear_dgrad(dy2, w_os, st)
     N, D_in = out2.shape
     D_out = dy2.shape[1]
+    if N % 8 == 0:
+        dy2 = dy2.to(torch.bfloat16).contiguous()
+        dout2 = _torch_ext.load().linear_dgrad(dy2, w_os, st)
+    else:
+        # d out from bf16(s dy) and W_o, one rounding less than from bf16(dy) and bf16(s W_o)
+        d = dy2.contiguous()
+        dz = torch.empty((N, D_out), device=dev, dtype=torch.bfloat16)
+        cast = d.dtype != torch.bfloat16
+        dy2 = torch.empty_like(dz) if cast else d
+        _lib.check(lib.naylis_mom_rezero_round(d.data_ptr(), _DT[d.dtype], s.data_ptr(),
+                                               dy2.data_ptr() if cast else None, dz.data_ptr(), d.numel(), st))
+        dout2 = _torch_ext.load().linear_dgrad(dz, w_o, st)
     if (out2.dtype == torch.bfloat16 and w_o.dtype == torch.bfloat16 and w_o.is_contiguous() and out2.is_contiguous()
             and N % 8 == 0 and D_in % 8 == 0 and D_out % 8 == 0):
         # dW' = dy^T out stays inside the split-K reduction, whose epilogue

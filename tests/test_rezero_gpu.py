@@ -153,3 +153,39 @@ def test_gated_wgrad_matches_two_steps(N, D_in, D_out, dev):
         assert bool((d <= 2.0 ** -7 * dw_ref.float().abs() + 1e-3).all()), f"max {float(d.max())}"
     mag = float((dwp.double() * w.double()).abs().sum())
     assert abs(float(ds) - float(ds_ref)) <= 1e-5 * mag + 1e-6
+
+
+@pytest.mark.parametrize("n,dydt", [(8192, torch.float32), (1000003, torch.float32), (4099, torch.bfloat16), (5, torch.float32)])
+@pytest.mark.parametrize("both", [False, True])
+def test_rezero_round_matches_torch(n, dydt, both, dev):
+    """naylis_mom_rezero_round: dy and s dy, each rounded once to bf16, bitwise
+    torch's; nothing written past the end."""
+    from naylis_amd import _lib
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    dy = torch.randn(n, generator=torch.Generator().manual_seed(n), dtype=torch.float32).to(dydt).to(dev)
+    s = torch.tensor([0.37], device=dev)
+    a, b = (torch.full((n + 8,), 7.0, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    _lib.check(lib.naylis_mom_rezero_round(dy.data_ptr(), 1 if dydt == torch.bfloat16 else 0, s.data_ptr(),
+                                           a.data_ptr() if both else None, b.data_ptr(), n, st))
+    assert torch.equal(b[:n], (s * dy).bfloat16()) and bool((b[n:] == 7).all())
+    assert torch.equal(a[:n], dy.bfloat16()) if both else bool((a == 7).all())
+
+
+@pytest.mark.parametrize("N", [131, 1029])
+@pytest.mark.parametrize("s", [0.37, 0.5, 1.7])
+def test_gated_linear_ragged_rounds_like_the_product(N, s, dev):
+    """The folded gate at row counts that are no multiple of 8: d out carries two
+    bf16 roundings, of s dy and of the result, as s * (out W_o^T) does, and not a
+    third one of s W_o.  A rounding's relative error r (2-norm) is measured on s dy;
+    independent ones add in squares: sqrt(2) r here, sqrt(3) r with a third."""
+    from naylis_amd import _lib, _torch_ext
+    g = torch.Generator(device=dev).manual_seed(N)
+    out = torch.randn(N, 512, generator=g, device=dev).bfloat16().requires_grad_(True)
+    w = (torch.randn(512, 512, generator=g, device=dev) / 20).bfloat16().requires_grad_(True)
+    dy = torch.randn(N, 512, generator=g, device=dev)
+    sc = torch.tensor([s], device=dev, requires_grad=True)
+    _torch_ext.load().gated_linear(out, w, sc, _lib.stream_of(dev)).backward(dy)
+    sdy = float(sc.detach()) * dy.double()
+    r = float((sdy.bfloat16().double() - sdy).norm() / sdy.norm())
+    ref = sdy @ w.detach().double()
+    assert float((out.grad.double() - ref).norm() / ref.norm()) < 1.57 * r
