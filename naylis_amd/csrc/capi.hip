@@ -924,7 +924,11 @@ int naylis_mom_linear_wgrad(const void* x, const void* dy, void* dw, int dw_dtyp
 // Row counts that are no multiple of 8: one tile per workgroup over all rows
 // where that occupies half of the CUs and is not long (hipBLASLt, whose place
 // it takes, sums them in one chain, too), else the splits or ranges of whole
-// counts.  3885 rows, 1024 x 1024: 12 us against 37 with hipBLASLt.
+// counts.  About 3885 rows, one tile / K splits / hipBLASLt: 1024 x 1024 18.1 /
+// 20.8 / 34.2 us, 1024 x 2048 24.5 / 32.3 / 39.8, 1536 x 1536 31.1 / 44.6 / 46.6,
+// 2816 x 1024 32.2 / 44.9 / 46.8; under 2048 rows the splits are one, from 6000
+// to 8184 rows one tile and splits are within 6 %.  (Multiples of 8 stay with
+// wgrad_splits, although between 2048 and 4096 rows one tile is ahead there too.)
 static int wgrad_rows_splits(int64_t N, int64_t D_in, int64_t D_out) {
   return N <= 8192 && gemm_small_fills((int)D_out, (int)D_in) ? 1 : wgrad_splits(N, D_in, D_out);
 }

@@ -516,8 +516,8 @@ bool gemm_small_ok(const GemmLaunch& g) {
 
 bool gemm_small_fills(int M, int N) {
   const int s32 = pipe_tiles<CfgS32>(M, N), s64 = pipe_tiles<CfgS64>(M, N), s128 = pipe_tiles<CfgS128>(M, N);
-  const int n = s32 <= 256 ? s32 : s64 <= 256 ? s64 : s128;
-  return n >= 128 && n <= 255;
+  if (s32 <= 256) return s32 >= 128;
+  return s64 <= 256 || s128 <= 255;  // (gemm_small_ok: not a full chip of 128 x 128)
 }
 
 hipError_t launch_gemm_small(const GemmLaunch& g, const char* name, hipStream_t st) {

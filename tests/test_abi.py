@@ -328,3 +328,14 @@ def test_bank_grouped_rejects_bad_arguments(lib):
     assert bwd(*args, None, 0, 2, 64, 32, 64, None) == _lib.NAYLIS_ERR_WORKSPACE
     assert bwd(*args, 1, 2 * 64 * 32 * 4 - 1, 2, 64, 32, 64, None) == _lib.NAYLIS_ERR_WORKSPACE
     assert bwd(*args, 1, 1 << 20, 25, 64, 32, 64, None) == _lib.NAYLIS_ERR_ARG
+
+
+@pytest.mark.parametrize("D_in,D_out,one", [(1024, 1024, True),   # 256 tiles of 64 x 64
+                                            (2048, 1024, True),   # 256 of 64 x 128
+                                            (2048, 2048, False),  # 256 of 128 x 128, bound by LDS reads: K splits
+                                            (1000, 1000, True), (512, 512, False)])
+def test_ragged_weight_gradient_one_round(lib, D_in, D_out, one):
+    """A ragged row count takes one tile per workgroup over all rows, without
+    partials in the workspace, where those tiles fill half to all of the CUs."""
+    nbytes = lib.naylis_mom_linear_wgrad_rows_workspace_bytes(3885, D_in, D_out)
+    assert nbytes == 256 if one else nbytes >= 2 * 4 * D_in * D_out
