@@ -265,6 +265,30 @@ struct Rope : public Function<Rope> {
   }
 };
 
+variable_list attention_grads(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& out,
+                              const at::Tensor& lse, const at::Tensor& grad, double scale, int64_t st) {
+  at::DeviceGuard guard(q.device());
+  const at::Tensor dout = grad.to(q.scalar_type()).contiguous();
+  at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(lse);
+  check(naylis_mom_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
+                            dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr<float>(),
+                            (float)scale, q.size(0), q.size(1), q.size(2), q.size(3), stream_ptr(st)));
+  return {dq, dk, dv};
+}
+
+// The gradients as a node of their own, for a backward with create_graph: they
+// depend on q, k, v and the incoming gradient, and a second derivative raises
+// (as torch's flash attention does) instead of leaving this part out.
+struct CausalAttentionGrad : public Function<CausalAttentionGrad> {
+  static variable_list forward(AutogradContext*, at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor out,
+                               at::Tensor lse, at::Tensor dout, double scale, int64_t st) {
+    return attention_grads(q, k, v, out, lse, dout, scale, st);
+  }
+  static variable_list backward(AutogradContext*, variable_list) {
+    TORCH_CHECK(false, "causal_attention: the derivative of its backward is not implemented");
+  }
+};
+
 struct CausalAttention : public Function<CausalAttention> {
   static at::Tensor forward(AutogradContext* ctx, at::Tensor q, at::Tensor k, at::Tensor v, double scale,
                             int64_t st) {
@@ -283,15 +307,13 @@ struct CausalAttention : public Function<CausalAttention> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
-    const at::Tensor &q = s[0], &k = s[1], &v = s[2], &out = s[3], &lse = s[4];
-    at::DeviceGuard guard(q.device());
-    const at::Tensor dout = grads[0].to(q.scalar_type()).contiguous();
-    at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(lse);
-    check(naylis_mom_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
-                              dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr<float>(),
-                              (float)ctx->saved_data["scale"].toDouble(), q.size(0), q.size(1), q.size(2), q.size(3),
-                              stream_ptr(ctx->saved_data["st"].toInt())));
-    return {dq, dk, dv, at::Tensor(), at::Tensor()};
+    const double scale = ctx->saved_data["scale"].toDouble();
+    const int64_t st = ctx->saved_data["st"].toInt();
+    variable_list g = at::GradMode::is_enabled()
+                          ? CausalAttentionGrad::apply(s[0], s[1], s[2], s[3], s[4], grads[0], scale, st)
+                          : attention_grads(s[0], s[1], s[2], s[3], s[4], grads[0], scale, st);
+    g.resize(5);
+    return g;
   }
 };
 

@@ -88,3 +88,29 @@ def test_attention_module_route(dev):
         want = attn(hidden_states=x, position_embeddings=(cos, sin), attention_mask=mask)[0]
     # bf16 P and one rounding of the attention's output each side, then the o projection
     assert float((got.float() - want.float()).norm() / want.float().norm()) < 2.0 ** -7
+
+
+def test_attention_second_derivative_raises(dev):
+    """Gradients taken with create_graph are right (bit for bit the others); a
+    second derivative through them raises, also where other paths of the graph
+    would go on without it."""
+    from naylis_amd.decoder import naylis_config
+    from naylis_amd.mom_kernels import hip_rope
+    from naylis_amd.mom_kernels.hip_attention import causal_attention
+    g = torch.Generator(device=dev).manual_seed(2)
+    q, k, v, dout = (torch.randn(1, 70, 2, 64, generator=g, device=dev).bfloat16().requires_grad_() for _ in range(4))
+    o = causal_attention(q, k, v, 0.125)
+    want = torch.autograd.grad(o, (q, k, v), dout.detach(), retain_graph=True)
+    got = torch.autograd.grad(o, (q, k, v), dout, create_graph=True)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    for x in (q, k, v, dout):
+        with pytest.raises(RuntimeError, match="not implemented"):
+            torch.autograd.grad(sum(t.float().square().sum() for t in got), x, retain_graph=True)
+    cfg = naylis_config(vocab_size=256, d_model=128, n_layers=1, n_heads=2, intermediate_size=256, seq_len=96)
+    attn = hip_rope.NaylisAttention(cfg, 0).to(dev).bfloat16()
+    x = torch.randn(1, 96, 128, generator=g, device=dev).bfloat16().requires_grad_()
+    cos, sin = (torch.rand(1, 96, 64, generator=g, device=dev).bfloat16() for _ in range(2))
+    dx, = torch.autograd.grad(attn(hidden_states=x, position_embeddings=(cos, sin))[0].float().square().sum(), x,
+                              create_graph=True)
+    with pytest.raises(RuntimeError, match="not implemented"):
+        torch.autograd.grad(dx.float().square().sum(), attn.v_proj.weight)
