@@ -22,6 +22,12 @@ using namespace naylis_ext;
 
 namespace {
 
+// The kernels read the products' results by their pointers, as bf16: a backward
+// that the caller runs under autocast must not make them another type.
+struct NoAutocast {
+  c10::impl::ExcludeDispatchKeyGuard guard{c10::autocast_dispatch_keyset};
+};
+
 void* opt_ptr(const c10::optional<at::Tensor>& t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
 
 // The read's inputs and what its backward takes: bank K / V (from the caller,
@@ -120,6 +126,7 @@ std::vector<at::Tensor> layer_bwd(c10::optional<at::Tensor> dy, c10::optional<at
                                   c10::optional<at::Tensor> side, at::Tensor lse, at::Tensor w_os, int64_t n_heads,
                                   int64_t num_blocks, int64_t block_size, int64_t top_k, bool external_bank,
                                   std::vector<int64_t> m_shape, bool m_bf16, int64_t stream) {
+  const NoAutocast no_autocast;
   at::DeviceGuard guard(x.device());
   void* st = reinterpret_cast<void*>(stream);
   const int64_t B = x.size(0), T = x.size(1), D = x.size(2);
@@ -229,6 +236,7 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
     // s: x, slots, w_down, w_up, w_q, w_k, w_v, w_o, scale, act, probs, top_idx, gates, k, v, q, order,
     // out, side, lse, w_os
     if (ctx->saved_data["ckpt"].toBool()) {  // s[1] is the bank
+      const NoAutocast no_autocast;
       at::DeviceGuard guard(s[0].device());
       const ReadState rd = read_part(s[0], opt(s[1]), s[4], s[5], s[6], opt(s[13]), opt(s[14]), s[11], s[12], geom[0],
                                      geom[1], geom[2], geom[3], stream_ptr(geom[4]));

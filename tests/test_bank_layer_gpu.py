@@ -349,3 +349,25 @@ def test_layer_ckpt_node_is_exact(case, dev):
     assert len(res[0]) == len(res[1])
     assert all(torch.equal(a, b) for a, b in zip(*res))
     assert held[1] < held[0]
+
+
+@pytest.mark.parametrize("ckpt", [False, True])
+@pytest.mark.parametrize("B,S", [(2, 200), (3, 77)])
+def test_layer_backward_under_autocast(ckpt, B, S, dev):
+    """A backward that runs under fp16 autocast gives the gradients of one that
+    does not: the node's products keep their bf16 results."""
+    import naylis_amd.layer as layer_mod
+    res = []
+    for autocast in (False, True):
+        layer, _, M = build_pair(256, 4, 8, 128, 2, 32, seed=31)
+        ld = layer_mod.cast_mom_layer(layer.to(dev), torch.bfloat16).train()
+        ld.mom_grad_ckpt, ld.noise_scale = ckpt, 0.0
+        g = torch.Generator().manual_seed(6)
+        x = torch.randn(B, S, 256, generator=g).bfloat16().to(dev).requires_grad_(True)
+        dy = torch.randn(B, S, 256, generator=g).to(dev)
+        Md = M.to(dev).requires_grad_(True)
+        y = ld(x, Md)
+        with torch.autocast("cuda", dtype=torch.float16, enabled=autocast):
+            y.backward(dy)
+        res.append([x.grad, Md.grad] + [p.grad for p in ld.parameters()])
+    assert all(torch.equal(a, b) for a, b in zip(*res))
