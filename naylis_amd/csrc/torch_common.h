@@ -43,6 +43,12 @@ inline void* ptr(const at::Tensor& t) { return t.defined() ? t.data_ptr() : null
 
 inline void* stream_ptr(int64_t st) { return reinterpret_cast<void*>(st); }
 
+// The kernels read the products' results by their pointers, as bf16: a backward
+// that the caller runs under autocast must not make them another type.
+struct NoAutocast {
+  c10::impl::ExcludeDispatchKeyGuard guard{c10::autocast_dispatch_keyset};
+};
+
 // y_i = x W_i^T for one to three weights (x (..., D_in), y_i (..., D_out) in
 // `dtype`), and dx = dy W (dy (N, D_out)): the library's GEMM where the rules
 // in torch_nodes.cpp say so, else torch's (hipBLASLt).
@@ -62,6 +68,9 @@ struct GatedGrads {
 };
 GatedGrads gated_linear_backward(const at::Tensor& dy2, const at::Tensor& out2, const at::Tensor& w_o,
                                  const at::Tensor& w_os, const at::Tensor& s, void* st);
+
+// y = out (s W_o)^T, fp32, as a node
+at::Tensor gated_linear(const at::Tensor& out, const at::Tensor& w_o, const at::Tensor& s, int64_t st);
 
 // The router backward's d_probs: an fp32 gradient expanded from one row goes in
 // as that row with stride 0, anything else as a dense fp32 copy with stride E.

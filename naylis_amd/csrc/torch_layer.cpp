@@ -22,12 +22,6 @@ using namespace naylis_ext;
 
 namespace {
 
-// The kernels read the products' results by their pointers, as bf16: a backward
-// that the caller runs under autocast must not make them another type.
-struct NoAutocast {
-  c10::impl::ExcludeDispatchKeyGuard guard{c10::autocast_dispatch_keyset};
-};
-
 void* opt_ptr(const c10::optional<at::Tensor>& t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
 
 // The read's inputs and what its backward takes: bank K / V (from the caller,
@@ -77,17 +71,14 @@ ReadState read_part(const at::Tensor& x, const c10::optional<at::Tensor>& m_bloc
   return r;
 }
 
-}  // namespace
-
-// Returns [y, probs, top_idx, act, gates, slots, k, v, q, order, out, side,
-// lse, w_os]; slots is undefined (None) with an external bank, side when the
-// read keeps no side buffer.
-std::vector<at::Tensor> layer_fwd(at::Tensor x, c10::optional<at::Tensor> m_blocks, at::Tensor w_down,
-                                  at::Tensor w_up, at::Tensor w_q, at::Tensor w_k, at::Tensor w_v, at::Tensor w_o,
-                                  at::Tensor scale, c10::optional<at::Tensor> noise, double noise_scale,
-                                  int64_t n_heads, int64_t num_blocks, int64_t block_size, int64_t top_k,
-                                  int64_t noise_kind, c10::optional<at::Tensor> k_ext,
-                                  c10::optional<at::Tensor> v_ext, int64_t stream) {
+// layer_fwd; without `gate` y and w_os stay undefined.
+std::vector<at::Tensor> forward_parts(at::Tensor x, const c10::optional<at::Tensor>& m_blocks, const at::Tensor& w_down,
+                                      const at::Tensor& w_up, const at::Tensor& w_q, const at::Tensor& w_k,
+                                      const at::Tensor& w_v, const at::Tensor& w_o, const at::Tensor& scale,
+                                      const c10::optional<at::Tensor>& noise, double noise_scale, int64_t n_heads,
+                                      int64_t num_blocks, int64_t block_size, int64_t top_k, int64_t noise_kind,
+                                      const c10::optional<at::Tensor>& k_ext, const c10::optional<at::Tensor>& v_ext,
+                                      bool gate, int64_t stream) {
   at::DeviceGuard guard(x.device());
   void* st = reinterpret_cast<void*>(stream);
   x = x.contiguous();
@@ -110,22 +101,24 @@ std::vector<at::Tensor> layer_fwd(at::Tensor x, c10::optional<at::Tensor> m_bloc
   const ReadState rd = read_part(x, m_blocks, w_q, w_k, w_v, k_ext, v_ext, top_idx, gates, n_heads, num_blocks,
                                  block_size, top_k, st);
   // ---- o projection with the ReZero gate folded into the weight (model.py:251, 239)
-  const auto [y, w_os] = gated_linear_forward(rd.out.view({B * T, D}), w_o, scale, st);
-  return {y.view({B, T, D}), probs, top_idx, act, gates, rd.slots, rd.k, rd.v, rd.q, rd.order, rd.out, rd.side, rd.lse,
-          w_os};
+  at::Tensor y, w_os;
+  if (gate) {
+    std::tie(y, w_os) = gated_linear_forward(rd.out.view({B * T, D}), w_o, scale, st);
+    y = y.view({B, T, D});
+  }
+  return {y, probs, top_idx, act, gates, rd.slots, rd.k, rd.v, rd.q, rd.order, rd.out, rd.side, rd.lse, w_os};
 }
 
-// Returns [dx, d_m, dw_down, dw_up, dw_q, dw_k, dw_v, dw_o, ds, dk_ext,
-// dv_ext]; with an external bank d_m, dw_k, dw_v are undefined and dk_ext,
-// dv_ext the bank's K / V gradients, else the reverse.
-std::vector<at::Tensor> layer_bwd(c10::optional<at::Tensor> dy, c10::optional<at::Tensor> d_probs, at::Tensor x,
-                                  c10::optional<at::Tensor> slots, at::Tensor w_down, at::Tensor w_up,
-                                  at::Tensor w_q, at::Tensor w_k, at::Tensor w_v, at::Tensor w_o, at::Tensor scale,
-                                  at::Tensor act, at::Tensor probs, at::Tensor top_idx, at::Tensor gates,
-                                  at::Tensor k, at::Tensor v, at::Tensor q, at::Tensor order, at::Tensor out,
-                                  c10::optional<at::Tensor> side, at::Tensor lse, at::Tensor w_os, int64_t n_heads,
-                                  int64_t num_blocks, int64_t block_size, int64_t top_k, bool external_bank,
-                                  std::vector<int64_t> m_shape, bool m_bf16, int64_t stream) {
+// layer_bwd; without `gate` the incoming gradient is that of the read's output.
+std::vector<at::Tensor> backward_parts(
+    const c10::optional<at::Tensor>& dy, const c10::optional<at::Tensor>& d_probs, const at::Tensor& x,
+    const c10::optional<at::Tensor>& slots, const at::Tensor& w_down, const at::Tensor& w_up, const at::Tensor& w_q,
+    const at::Tensor& w_k, const at::Tensor& w_v, const at::Tensor& w_o, const at::Tensor& scale,
+    const at::Tensor& act, const at::Tensor& probs, const at::Tensor& top_idx, const at::Tensor& gates,
+    const at::Tensor& k, const at::Tensor& v, const at::Tensor& q, const at::Tensor& order, const at::Tensor& out,
+    const c10::optional<at::Tensor>& side, const at::Tensor& lse, const at::Tensor& w_os, int64_t n_heads,
+    int64_t num_blocks, int64_t block_size, int64_t top_k, bool external_bank, const std::vector<int64_t>& m_shape,
+    bool m_bf16, bool gate, int64_t stream) {
   const NoAutocast no_autocast;
   at::DeviceGuard guard(x.device());
   void* st = reinterpret_cast<void*>(stream);
@@ -134,7 +127,11 @@ std::vector<at::Tensor> layer_bwd(c10::optional<at::Tensor> dy, c10::optional<at
   const auto f32 = x.options().dtype(at::kFloat);
   // ---- o projection with the folded gate: d out, dW_o, ds
   at::Tensor dy_t = dy.has_value() && dy->defined() ? *dy : at::zeros({B, T, D}, x.options().dtype(at::kBFloat16));
-  GatedGrads go = gated_linear_backward(dy_t.reshape({N, D}), out.view({N, D}), w_o, w_os, scale, st);
+  GatedGrads go;
+  if (gate)
+    go = gated_linear_backward(dy_t.reshape({N, D}), out.view({N, D}), w_o, w_os, scale, st);
+  else
+    go.dout2 = dy_t.to(at::kBFloat16).contiguous();
   // ---- gated read
   at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), dgates = at::empty_like(gates);
   {
@@ -182,6 +179,37 @@ std::vector<at::Tensor> layer_bwd(c10::optional<at::Tensor> dy, c10::optional<at
   return {dx, d_m, dw_down, dw_up, dw_q, dw_k, dw_v, go.dw_o, go.ds, dk_ext, dv_ext};
 }
 
+}  // namespace
+
+// Returns [y, probs, top_idx, act, gates, slots, k, v, q, order, out, side,
+// lse, w_os]; slots is undefined (None) with an external bank, side when the
+// read keeps no side buffer.
+std::vector<at::Tensor> layer_fwd(at::Tensor x, c10::optional<at::Tensor> m_blocks, at::Tensor w_down,
+                                  at::Tensor w_up, at::Tensor w_q, at::Tensor w_k, at::Tensor w_v, at::Tensor w_o,
+                                  at::Tensor scale, c10::optional<at::Tensor> noise, double noise_scale,
+                                  int64_t n_heads, int64_t num_blocks, int64_t block_size, int64_t top_k,
+                                  int64_t noise_kind, c10::optional<at::Tensor> k_ext,
+                                  c10::optional<at::Tensor> v_ext, int64_t stream) {
+  return forward_parts(x, m_blocks, w_down, w_up, w_q, w_k, w_v, w_o, scale, noise, noise_scale, n_heads, num_blocks,
+                       block_size, top_k, noise_kind, k_ext, v_ext, true, stream);
+}
+
+// Returns [dx, d_m, dw_down, dw_up, dw_q, dw_k, dw_v, dw_o, ds, dk_ext,
+// dv_ext]; with an external bank d_m, dw_k, dw_v are undefined and dk_ext,
+// dv_ext the bank's K / V gradients, else the reverse.
+std::vector<at::Tensor> layer_bwd(c10::optional<at::Tensor> dy, c10::optional<at::Tensor> d_probs, at::Tensor x,
+                                  c10::optional<at::Tensor> slots, at::Tensor w_down, at::Tensor w_up,
+                                  at::Tensor w_q, at::Tensor w_k, at::Tensor w_v, at::Tensor w_o, at::Tensor scale,
+                                  at::Tensor act, at::Tensor probs, at::Tensor top_idx, at::Tensor gates,
+                                  at::Tensor k, at::Tensor v, at::Tensor q, at::Tensor order, at::Tensor out,
+                                  c10::optional<at::Tensor> side, at::Tensor lse, at::Tensor w_os, int64_t n_heads,
+                                  int64_t num_blocks, int64_t block_size, int64_t top_k, bool external_bank,
+                                  std::vector<int64_t> m_shape, bool m_bf16, int64_t stream) {
+  return backward_parts(dy, d_probs, x, slots, w_down, w_up, w_q, w_k, w_v, w_o, scale, act, probs, top_idx, gates, k,
+                        v, q, order, out, side, lse, w_os, n_heads, num_blocks, block_size, top_k, external_bank,
+                        m_shape, m_bf16, true, stream);
+}
+
 namespace {
 
 c10::optional<at::Tensor> opt(const at::Tensor& t) {
@@ -192,7 +220,7 @@ c10::optional<at::Tensor> opt(const at::Tensor& t) {
 // only defined tensors, so an absent noise draw is passed as x with
 // has_noise false, and the bank (m_blocks) or the external K / V that the
 // call does not use likewise (external tells which); no gradient flows to
-// those placeholders.  Outputs y, probs, top_idx.
+// those placeholders.  Outputs y (without `gate` the read's output), probs, top_idx.
 struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
   static torch::autograd::variable_list forward(torch::autograd::AutogradContext* ctx, at::Tensor x,
                                                 at::Tensor m_blocks, at::Tensor w_down, at::Tensor w_up,
@@ -201,13 +229,13 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
                                                 double noise_scale, int64_t n_heads, int64_t num_blocks,
                                                 int64_t block_size, int64_t top_k, int64_t noise_kind,
                                                 at::Tensor k_ext, at::Tensor v_ext, bool external, bool ckpt,
-                                                int64_t stream) {
+                                                bool gate, int64_t stream) {
     const at::Tensor none;
     x = x.contiguous();
-    std::vector<at::Tensor> r =
-        layer_fwd(x, external ? c10::nullopt : opt(m_blocks), w_down, w_up, w_q, w_k, w_v, w_o, scale,
-                  has_noise ? opt(noise) : c10::nullopt, noise_scale, n_heads, num_blocks, block_size, top_k,
-                  noise_kind, external ? opt(k_ext) : c10::nullopt, external ? opt(v_ext) : c10::nullopt, stream);
+    std::vector<at::Tensor> r = forward_parts(
+        x, external ? c10::nullopt : opt(m_blocks), w_down, w_up, w_q, w_k, w_v, w_o, scale,
+        has_noise ? opt(noise) : c10::nullopt, noise_scale, n_heads, num_blocks, block_size, top_k, noise_kind,
+        external ? opt(k_ext) : c10::nullopt, external ? opt(v_ext) : c10::nullopt, gate, stream);
     // r: y, probs, top_idx, act, gates, slots, k, v, q, order, out, side, lse, w_os
     if (ckpt)  // the read's inputs only: its backward runs read_part again
       ctx->save_for_backward({x, external ? none : m_blocks, w_down, w_up, w_q, w_k, w_v, w_o, scale, r[3], r[1],
@@ -217,13 +245,14 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
       ctx->save_for_backward({x, r[5], w_down, w_up, w_q, w_k, w_v, w_o, scale, r[3], r[1], r[2], r[4], r[6], r[7],
                               r[8], r[9], r[10], r[11], r[12], r[13]});
     ctx->saved_data["ckpt"] = ckpt;
+    ctx->saved_data["gate"] = gate;
     ctx->saved_data["geom"] = std::vector<int64_t>{n_heads, num_blocks, block_size, top_k, stream};
     ctx->saved_data["external"] = external;
     ctx->saved_data["m_shape"] = external ? std::vector<int64_t>{} : m_blocks.sizes().vec();
     ctx->saved_data["m_bf16"] = !external && m_blocks.scalar_type() == at::kBFloat16;
     ctx->mark_non_differentiable({r[2]});
     ctx->set_materialize_grads(false);
-    return {r[0], r[1], r[2]};
+    return {gate ? r[0] : r[10], r[1], r[2]};
   }
 
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
@@ -249,14 +278,16 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
       s[18] = rd.side;
       s[19] = rd.lse;
     }
+    const bool gate = ctx->saved_data["gate"].toBool();
     std::vector<at::Tensor> r =
-        layer_bwd(opt(grads[0]), opt(grads[1]), s[0], opt(s[1]), s[2], s[3], s[4], s[5], s[6], s[7], s[8], s[9],
-                  s[10], s[11], s[12], s[13], s[14], s[15], s[16], s[17], opt(s[18]), s[19], s[20], geom[0],
-                  geom[1], geom[2], geom[3], external, m_shape, m_bf16, geom[4]);
+        backward_parts(opt(grads[0]), opt(grads[1]), s[0], opt(s[1]), s[2], s[3], s[4], s[5], s[6], s[7], s[8], s[9],
+                       s[10], s[11], s[12], s[13], s[14], s[15], s[16], s[17], opt(s[18]), s[19], s[20], geom[0],
+                       geom[1], geom[2], geom[3], external, m_shape, m_bf16, gate, geom[4]);
     // r: dx, d_m, dw_down, dw_up, dw_q, dw_k, dw_v, dw_o, ds, dk_ext, dv_ext
     const at::Tensor none;
-    return {r[0], r[1],  r[2], r[3], r[4], r[5], r[6], r[7], r[8].view(s[8].sizes()), none, none,
-            none, none, none, none, none, none, r[9], r[10], none, none, none};
+    if (gate) r[8] = r[8].view(s[8].sizes());
+    return {r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7], r[8], none, none, none,
+            none, none, none, none, none, r[9], r[10], none, none, none, none};
   }
 };
 
@@ -270,9 +301,17 @@ std::vector<at::Tensor> mom_layer_node(at::Tensor x, c10::optional<at::Tensor> m
   const bool has_noise = noise.has_value() && noise->defined();
   TORCH_CHECK(external || (m_blocks.has_value() && m_blocks->defined()), "mom_layer: no bank and no external K / V");
   TORCH_CHECK(!external || (v_ext.has_value() && v_ext->defined()), "mom_layer: external K without V");
-  return MomLayerNode::apply(x, external ? x : *m_blocks, w_down, w_up, w_q, w_k, w_v, w_o, scale,
-                             has_noise ? *noise : x, has_noise, noise_scale, n_heads, num_blocks, block_size, top_k,
-                             noise_kind, external ? *k_ext : x, external ? *v_ext : x, external, ckpt, stream);
+  // A checkpointed layer at a token count without the gated weight gradient
+  // (naylis_mom_gated_wgrad) has the o projection and gate in their own node:
+  // gradients of W_o and the gate taken with create_graph then keep the read's
+  // output, and through it the layer, in their graph.
+  const bool gate = !ckpt || x.numel() / x.size(-1) % 8 == 0;
+  std::vector<at::Tensor> r =
+      MomLayerNode::apply(x, external ? x : *m_blocks, w_down, w_up, w_q, w_k, w_v, w_o, scale, has_noise ? *noise : x,
+                          has_noise, noise_scale, n_heads, num_blocks, block_size, top_k, noise_kind,
+                          external ? *k_ext : x, external ? *v_ext : x, external, ckpt, gate, stream);
+  if (!gate) r[0] = gated_linear(r[0], w_o, scale, stream);
+  return r;
 }
 
 }  // namespace

@@ -515,12 +515,27 @@ struct GatedLinear : public Function<GatedLinear> {
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list v = ctx->get_saved_variables();
     const at::Tensor &out = v[0], &w_o = v[1], &w_os = v[2], &s = v[3];
+    const NoAutocast no_autocast;
     at::DeviceGuard guard(out.device());
+    if (at::GradMode::is_enabled()) {  // create_graph: s * (out W_o^T) in products that autograd knows
+      const at::Tensor dy = grads[0].reshape({-1, w_o.size(0)}), o = out.reshape({-1, w_o.size(1)});
+      const at::Tensor dz = (dy * s).to(o.scalar_type());
+      return {at::mm(dz, w_o).view(out.sizes()), at::mm(dz.t(), o), (dy * at::mm(o, w_o.t())).sum().view(s.sizes()),
+              at::Tensor()};
+    }
     const GatedGrads g = gated_linear_backward(grads[0].reshape({-1, w_o.size(0)}), out.reshape({-1, w_o.size(1)}),
                                                w_o, w_os, s, stream_ptr(ctx->saved_data["st"].toInt()));
     return {g.dout2.view(out.sizes()), g.dw_o, g.ds.view(s.sizes()), at::Tensor()};
   }
 };
+
+}  // namespace
+
+at::Tensor gated_linear(const at::Tensor& out, const at::Tensor& w_o, const at::Tensor& s, int64_t st) {
+  return GatedLinear::apply(out, w_o, s, st);
+}
+
+namespace {
 
 // ---- LM loss ----------------------------------------------------------------
 

@@ -371,3 +371,40 @@ def test_layer_backward_under_autocast(ckpt, B, S, dev):
             y.backward(dy)
         res.append([x.grad, Md.grad] + [p.grad for p in ld.parameters()])
     assert all(torch.equal(a, b) for a, b in zip(*res))
+
+
+@pytest.mark.parametrize("wrt", ["mom_scale", "o_proj"])
+def test_ckpt_ragged_second_derivative(wrt, dev):
+    """Gradients of the gate and of W_o taken with create_graph through a
+    checkpointed layer of 231 tokens.  Both are linear in dy: sum(r dW_o) is
+    s sum(dy (out r^T)) and ds is sum(dy (out W_o^T)), so their derivatives are
+    the first ones of a layer with r in W_o's place, or divided by s.  Each side
+    carries about six independent bf16 roundings of rms 2^-9 or less."""
+    import naylis_amd.layer as layer_mod
+
+    def make(w_o=None):
+        layer, _, M = build_pair(256, 4, 4, 128, 2, 16, seed=31, mom_scale=0.37)
+        ld = layer_mod.cast_mom_layer(layer.to(dev), torch.bfloat16).train()
+        ld.mom_grad_ckpt, ld.noise_scale = True, 0.0
+        if w_o is not None:
+            ld.o_proj.weight.data.copy_(w_o)
+        g = torch.Generator().manual_seed(6)
+        x = torch.randn(3, 77, 256, generator=g).bfloat16().to(dev).requires_grad_(True)
+        Md = M.to(dev).requires_grad_(True)
+        return ld, x, Md, [x, Md, ld.q_proj.weight, ld.v_proj.weight, ld.router_up.weight]
+
+    dy = torch.randn(3, 77, 256, generator=torch.Generator().manual_seed(7)).to(dev)
+    r = (torch.randn(256, 256, generator=torch.Generator().manual_seed(8)) / 16).bfloat16().to(dev)
+    ld, x, Md, ins = make()
+    y = ld(x, Md)
+    if wrt == "mom_scale":
+        ds, = torch.autograd.grad(y, ld.mom_scale, dy, create_graph=True)
+        got = torch.autograd.grad(ds.sum(), ins)
+        want = [t / 0.37 for t in torch.autograd.grad(ld(x, Md), ins, dy)]
+    else:
+        dw, = torch.autograd.grad(y, ld.o_proj.weight, dy, create_graph=True)
+        got = torch.autograd.grad(dw, ins, r)
+        ld, x, Md, ins = make(r)
+        want = torch.autograd.grad(ld(x, Md), ins, dy)
+    for a, b in zip(got, want):
+        assert float((a.double() - b.double()).norm() / b.double().norm()) < 12 ** 0.5 * 2.0 ** -9 * 2
