@@ -301,6 +301,26 @@ std::vector<at::Tensor> mom_layer_node(at::Tensor x, c10::optional<at::Tensor> m
   const bool has_noise = noise.has_value() && noise->defined();
   TORCH_CHECK(external || (m_blocks.has_value() && m_blocks->defined()), "mom_layer: no bank and no external K / V");
   TORCH_CHECK(!external || (v_ext.has_value() && v_ext->defined()), "mom_layer: external K without V");
+  // the kernels take every size from x and the geometry
+  TORCH_CHECK(x.dim() == 3 && n_heads > 0 && num_blocks > 0 && block_size > 0 && x.size(2) % n_heads == 0,
+              "mom_layer: x must be (B, T, D) with D a multiple of the heads");
+  const int64_t D = x.size(2), L = num_blocks * block_size;
+  if (external) {
+    TORCH_CHECK(k_ext->sizes() == at::IntArrayRef({L, D}) && v_ext->sizes() == k_ext->sizes(),
+                "mom_layer: bank K / V must be (", L, ", ", D, "), got ", k_ext->sizes(), " / ", v_ext->sizes());
+  } else {
+    TORCH_CHECK(m_blocks->numel() == L * D, "mom_layer: bank of ", m_blocks->numel(), " values, the layer expects ", L,
+                " slots of ", D);
+  }
+  for (const at::Tensor* w : {&w_q, &w_k, &w_v, &w_o})
+    TORCH_CHECK(w->sizes() == at::IntArrayRef({D, D}), "mom_layer: projection weights must be (", D, ", ", D, "), got ",
+                w->sizes());
+  TORCH_CHECK(w_down.dim() == 2 && w_down.size(1) == D &&
+                  w_up.sizes() == at::IntArrayRef({num_blocks, w_down.size(0)}),
+              "mom_layer: router weights must be (R, ", D, ") and (", num_blocks, ", R), got ", w_down.sizes(), " and ",
+              w_up.sizes());
+  TORCH_CHECK(!has_noise || noise->numel() == x.size(0) * x.size(1) * num_blocks, "mom_layer: noise must be (B, T, ",
+              num_blocks, "), got ", noise->sizes());
   // A checkpointed layer at a token count without the gated weight gradient
   // (naylis_mom_gated_wgrad) has the o projection and gate in their own node:
   // gradients of W_o and the gate taken with create_graph then keep the read's

@@ -339,3 +339,30 @@ def test_ragged_weight_gradient_one_round(lib, D_in, D_out, one):
     partials in the workspace, where those tiles fill half to all of the CUs."""
     nbytes = lib.naylis_mom_linear_wgrad_rows_workspace_bytes(3885, D_in, D_out)
     assert nbytes == 256 if one else nbytes >= 2 * 4 * D_in * D_out
+
+
+@pytest.mark.parametrize("wrong,match", [
+    (dict(m_blocks=(3, 16 * 32)), "bank of"),                  # three blocks where the layer reads four
+    (dict(k_ext=(48, 32), v_ext=(48, 32)), "bank K / V"),
+    (dict(k_ext=(64, 32), v_ext=(64, 16)), "bank K / V"),
+    (dict(w_k=(32, 16)), "projection weights"), (dict(w_v=(16, 32)), "projection weights"),
+    (dict(w_down=(8, 16)), "router weights"), (dict(w_up=(5, 8)), "router weights"),
+    (dict(noise=(2, 6, 3)), "noise"),
+])
+@pytest.mark.parametrize("ckpt", [False, True])
+def test_layer_node_refuses_wrong_sizes(lib, wrong, match, ckpt):
+    """The layer's node takes its sizes from x and the geometry; a bank or weight
+    of another size is an error, not a read past its end (host tensors: no
+    kernel is reached)."""
+    from naylis_amd import _torch_ext
+    shapes = dict(m_blocks=(4, 16 * 32), w_down=(8, 32), w_up=(4, 8), w_q=(32, 32), w_k=(32, 32), w_v=(32, 32),
+                  w_o=(32, 32), noise=None, k_ext=None, v_ext=None)
+    shapes.update(wrong)
+    f32 = ("w_down", "w_up", "noise")
+    t = {n: None if s is None else torch.zeros(s, dtype=torch.float32 if n in f32 else torch.bfloat16)
+         for n, s in shapes.items()}
+    x = torch.zeros(2, 6, 32, dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError, match=match):
+        _torch_ext.load().mom_layer(x, t["m_blocks"] if t["k_ext"] is None else None, t["w_down"], t["w_up"], t["w_q"],
+                                    t["w_k"], t["w_v"], t["w_o"], torch.ones(1), t["noise"], 1.0, 2, 4, 16, 2, 0,
+                                    t["k_ext"], t["v_ext"], ckpt, 0)
