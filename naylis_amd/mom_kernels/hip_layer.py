@@ -60,8 +60,8 @@ def _ws(nbytes, dev):
 
 
 def fused_layer_supported(x, M_blocks, w_down, w_up, w_q, w_k, w_v, w_o, scale, bank_kv=None):
-    """True when the fused node applies: bf16 activations and projection
-    weights, fp32 router weights and gate, D a multiple of 128 (the router's
+    """True when the fused node applies: bf16 activations and contiguous bf16
+    projection weights, fp32 router weights and gate, D a multiple of 128 (the router's
     accumulating backward), all on one ROCm device.  With ``bank_kv`` the
     bank's K and V come from the caller (bf16, contiguous)."""
     if torch.version.hip is None or not x.is_cuda:
@@ -70,7 +70,7 @@ def fused_layer_supported(x, M_blocks, w_down, w_up, w_q, w_k, w_v, w_o, scale, 
         return False
     dev = x.device
     for w in (w_q, w_k, w_v, w_o):
-        if w.dtype != torch.bfloat16 or w.device != dev or w.dim() != 2:
+        if w.dtype != torch.bfloat16 or w.device != dev or w.dim() != 2 or not w.is_contiguous():
             return False
     if w_q.shape != (x.shape[-1], x.shape[-1]) or w_o.shape != w_q.shape:
         return False

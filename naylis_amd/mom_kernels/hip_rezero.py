@@ -126,5 +126,5 @@ def mom_gated_linear(out, w_o, s):
             and w_o.dtype == torch.bfloat16 and s.dtype == torch.float32 and s.numel() == 1
             and out.device == w_o.device == s.device and out.shape[-1] == D_in and D_in % 8 == 0
             and D_out % 8 == 0 and (out.numel() // D_in) % 8 == 0):
-        return _torch_ext.load().gated_linear(out.contiguous(), w_o, s, _lib.stream_of(out.device))
+        return _torch_ext.load().gated_linear(out.contiguous(), w_o.contiguous(), s, _lib.stream_of(out.device))
     return s * F.linear(out, w_o)

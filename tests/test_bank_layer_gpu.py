@@ -408,3 +408,32 @@ def test_ckpt_ragged_second_derivative(wrt, dev):
         want = torch.autograd.grad(ld(x, Md), ins, dy)
     for a, b in zip(got, want):
         assert float((a.double() - b.double()).norm() / b.double().norm()) < 12 ** 0.5 * 2.0 ** -9 * 2
+
+
+@pytest.mark.parametrize("ckpt", [False, True])
+@pytest.mark.parametrize("S", [77, 80])
+def test_layer_with_strided_weights(ckpt, S, dev):
+    """Projection weights held transposed in memory give the results of the same
+    values in row order, up to the bf16 roundings in which the layer's fused and
+    separate paths differ (about six each side, rms 2^-9 or less; the gate's
+    gradient, one sum of products of either sign, against the norm of those)."""
+    import naylis_amd.layer as layer_mod
+    res = []
+    for strided in (False, True):
+        layer, _, M = build_pair(256, 4, 4, 128, 2, 16, seed=31, mom_scale=0.37)
+        ld = layer_mod.cast_mom_layer(layer.to(dev), torch.bfloat16).train()
+        ld.mom_grad_ckpt, ld.noise_scale = ckpt, 0.0
+        if strided:
+            for lin in (ld.q_proj, ld.k_proj, ld.v_proj, ld.o_proj):
+                lin.weight = torch.nn.Parameter(lin.weight.detach().t().contiguous().t())
+        g = torch.Generator().manual_seed(6)
+        x = torch.randn(2, S, 256, generator=g).bfloat16().to(dev).requires_grad_(True)
+        Md = M.to(dev).requires_grad_(True)
+        dy = torch.randn(2, S, 256, generator=g).to(dev)
+        y = ld(x, Md)
+        y.backward(dy)
+        res.append([y.detach(), x.grad, Md.grad] + [p.grad for p in ld.parameters()])
+    terms = (dy * res[0][0] / 0.37).double().norm()
+    for a, b in zip(*res):
+        size = terms if a.numel() == 1 else a.double().norm()
+        assert float((a.double() - b.double()).norm() / size) < 12 ** 0.5 * 2.0 ** -9 * 2
