@@ -375,7 +375,7 @@ int naylis_mom_bank_kv_bwd_grouped(const void* slots, const void* const* w_k, co
  *   y_i = x W_i^T for n = 1 .. 3 weights W_i (D_out, D_in) of one input x
  *         (N, D_in), in y_dtype;      dx = dy W, bf16, dy (N, D_out).
  * w and y are host arrays of n device pointers.  D_in and D_out multiples of 8,
- * any N; all pointers 16-byte aligned. */
+ * any N with N * max(D_in, D_out) < 2^30; all pointers 16-byte aligned. */
 int naylis_mom_linear_fwd(const void* x, const void* const* w, void* const* y, int n, int y_dtype, int64_t N,
                           int64_t D_in, int64_t D_out, void* stream);
 int naylis_mom_linear_dgrad(const void* dy, const void* w, void* dx, int64_t N, int64_t D_in, int64_t D_out,

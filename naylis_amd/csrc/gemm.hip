@@ -23,6 +23,8 @@
 #include "launch_gemm.h"
 #include "timing.h"
 
+#include <algorithm>
+
 namespace naylis {
 
 constexpr int kGK = 64;  // K step
@@ -514,8 +516,10 @@ static GemmLaunch linear_launch(int n, int M, int N, int K, GemmOut out) {
 }
 
 // Row counts need not be multiples of 8: x and dy are K-contiguous, so a tile's
-// rows past their end read the last one and are not stored.
+// rows past their end read the last one and are not stored.  Their buffer
+// resources reach from the tile's first row to the last one, in 32 bits.
 static bool linear_supported(GemmLaunch g) {
+  if ((long)g.M * std::max(g.N, g.K) >= 1L << 30) return false;
   g.M = (g.M + 7) / 8 * 8;
   return gemm_supported(g);
 }

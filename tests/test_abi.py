@@ -366,3 +366,14 @@ def test_layer_node_refuses_wrong_sizes(lib, wrong, match, ckpt):
         _torch_ext.load().mom_layer(x, t["m_blocks"] if t["k_ext"] is None else None, t["w_down"], t["w_up"], t["w_q"],
                                     t["w_k"], t["w_v"], t["w_o"], torch.ones(1), t["noise"], 1.0, 2, 4, 16, 2, 0,
                                     t["k_ext"], t["v_ext"], ckpt, 0)
+
+
+@pytest.mark.parametrize("N,D_in,D_out", [(1 << 20, 1024, 64), (1 << 20, 64, 1024), ((1 << 21) + 1, 1024, 8),
+                                          (1 << 30, 8, 8)])
+def test_linear_refuses_spans_past_its_offsets(lib, N, D_in, D_out):
+    """From N * max(D_in, D_out) = 2^30 on, an operand's bytes pass the 32-bit
+    extent that the kernels give it."""
+    one = (ctypes.c_void_p * 1)(16)
+    assert lib.naylis_mom_linear_fwd(16, one, one, 1, 1, N, D_in, D_out, None) == _lib.NAYLIS_ERR_ARG
+    assert b"2^30" in lib.naylis_mom_last_error()
+    assert lib.naylis_mom_linear_dgrad(16, 16, 16, N, D_in, D_out, None) == _lib.NAYLIS_ERR_ARG
