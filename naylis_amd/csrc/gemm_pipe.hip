@@ -82,7 +82,7 @@ __device__ __forceinline__ void load_to_lds(i32x4 rs, int voff, int soff, uint32
       "s_nop 0\n\t"
       "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds),
       "v"(voff), "s"(rs), "s"(soff)
-      : "memory");
+      : "memory", "m0");
 }
 
 struct PipeOp {

@@ -377,3 +377,17 @@ def test_linear_refuses_spans_past_its_offsets(lib, N, D_in, D_out):
     assert lib.naylis_mom_linear_fwd(16, one, one, 1, 1, N, D_in, D_out, None) == _lib.NAYLIS_ERR_ARG
     assert b"2^30" in lib.naylis_mom_last_error()
     assert lib.naylis_mom_linear_dgrad(16, 16, 16, N, D_in, D_out, None) == _lib.NAYLIS_ERR_ARG
+
+
+def test_inline_assembly_names_m0(lib):
+    """Inline assembly that writes m0 lists it as clobbered: the compiler keeps
+    values of its own there (LDS-destination loads, indexed register moves)."""
+    csrc = os.path.join(ROOT, "naylis_amd", "csrc")
+    seen = 0
+    for name in sorted(os.listdir(csrc)):
+        text = re.sub(r"//[^\n]*", "", open(os.path.join(csrc, name)).read())
+        for block in re.findall(r"\basm\b[^;]*;", text, flags=re.S):
+            if re.search(r"\bm0\s*,", block.split(":")[0]):
+                seen += 1
+                assert '"m0"' in block, (name, block)
+    assert seen >= 1
