@@ -653,6 +653,11 @@ void bind_nodes(pybind11::module_& m) {
     at::DeviceGuard guard(dy.device());
     return linear_dgrad(dy, w, stream_ptr(st));
   });
+  m.def("linear_wgrad", [](Tensor xin, Tensor dy, bool f32, int64_t st) {
+    at::NoGradGuard no_grad;
+    at::DeviceGuard guard(xin.device());
+    return library_wgrad(xin, dy, f32 ? at::kFloat : at::kBFloat16, stream_ptr(st));
+  });
   m.def("route", [](Tensor x, Tensor wd, Tensor wu, c10::optional<Tensor> noise, double noise_scale, int64_t top_k,
                     bool want_h, int64_t kind, int64_t st) {
     return Route::apply(x, wd, wu, noise.has_value() ? *noise : x, noise.has_value(), noise_scale, top_k, want_h, kind,

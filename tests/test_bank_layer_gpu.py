@@ -185,6 +185,7 @@ EXT_CASES = [
     (2, 256, 256, 4, 8, 128, 2, 32, torch.float32, False, True),    # fp32 bank gradient, uniform noise (Gumbel)
     (2, 256, 256, 4, 8, 128, 2, 32, torch.bfloat16, True, False),   # bank K/V from the caller
     (1, 131, 256, 2, 4, 64, 2, 16, torch.bfloat16, False, False),   # 131 tokens: the unsplit weight gradients
+    (1, 16381, 1024, 16, 8, 128, 2, 32, torch.bfloat16, False, False),  # the same in K ranges, summed in their order
 ]
 
 
