@@ -14,17 +14,12 @@ namespace naylis_ext {
 
 constexpr int kF32 = 0, kBF16 = 1;
 
-// A non-zero status of a C-ABI call; reaches Python as naylis_amd._lib.NaylisError.
-struct StatusError : std::runtime_error {
-  int code;
-  StatusError(int c, const std::string& m) : std::runtime_error(m), code(c) {}
-};
+// A non-zero status of a C-ABI call raises naylis_amd._lib.NaylisError: as a
+// Python error, which the autograd engine carries out of a backward's thread.
+[[noreturn]] void raise_status(int rc);
 
 inline void check(int rc) {
-  if (rc != NAYLIS_OK) {
-    const char* msg = naylis_mom_last_error();
-    throw StatusError(rc, msg ? msg : "unknown error");
-  }
+  if (rc != NAYLIS_OK) raise_status(rc);
 }
 
 // A workspace query's answer (0: the shape is not supported, with a message).

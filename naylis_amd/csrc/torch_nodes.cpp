@@ -55,6 +55,17 @@ bool own_dgrad(int64_t N, int64_t D_in, int64_t D_out) {
 
 }  // namespace
 
+void raise_status(int rc) {
+  const char* msg = naylis_mom_last_error();
+  namespace py = pybind11;
+  py::gil_scoped_acquire gil;
+  const py::object type = py::module_::import("naylis_amd._lib").attr("NaylisError");
+  PyErr_SetObject(type.ptr(), type(rc, msg ? msg : "unknown error").ptr());
+  python_error e;
+  e.persist();
+  throw e;
+}
+
 std::vector<at::Tensor> linear_fwd(const at::Tensor& x, const std::vector<at::Tensor>& w, at::ScalarType dtype,
                                    void* st) {
   const int64_t D_out = w[0].size(0), D_in = w[0].size(1), N = x.numel() / std::max<int64_t>(D_in, 1), n = w.size();
@@ -626,9 +637,8 @@ void bind_nodes(pybind11::module_& m) {
   py::register_exception_translator([](std::exception_ptr p) {
     try {
       if (p) std::rethrow_exception(p);
-    } catch (const StatusError& e) {
-      py::object type = py::module_::import("naylis_amd._lib").attr("NaylisError");
-      PyErr_SetObject(type.ptr(), type(e.code, e.what()).ptr());
+    } catch (python_error& e) {
+      e.restore();
     }
   });
   using at::Tensor;

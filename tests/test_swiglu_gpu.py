@@ -40,3 +40,19 @@ def test_swiglu_rejects_unsupported(dev):
     from naylis_amd.mom_kernels.hip_mlp import swiglu
     with pytest.raises(RuntimeError, match="unsupported"):
         swiglu(torch.randn(7, device=dev), torch.randn(7, device=dev))
+
+
+def test_status_error_in_a_backward_keeps_its_type(dev):
+    """A C-ABI call that refuses its arguments inside a backward (here a gradient
+    at an odd address) raises NaylisError with its code, as in a forward."""
+    from naylis_amd import _lib
+    from naylis_amd.mom_kernels.hip_mlp import swiglu
+    g, u = (torch.randn(4, 64, device=dev).bfloat16().requires_grad_() for _ in range(2))
+    buf = torch.zeros(4 * 64 + 1, device=dev).bfloat16()
+    h = swiglu(g, u)
+    with pytest.raises(_lib.NaylisError) as err:
+        h.backward(buf[1:].view(4, 64))
+    assert err.value.code == _lib.NAYLIS_ERR_ARG and "aligned" in str(err.value)
+    with pytest.raises(_lib.NaylisError) as err, torch.no_grad():
+        swiglu(buf[1:].view(4, 64), u)
+    assert err.value.code == _lib.NAYLIS_ERR_ARG
