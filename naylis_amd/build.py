@@ -64,8 +64,10 @@ def build_torch_ext(verbose=False):
     # cpp_extension imports the module it built: its C-ABI symbols come from
     # the library, loaded here with global visibility as naylis_amd._lib does
     ctypes.CDLL(LIB, mode=ctypes.RTLD_GLOBAL)
-    ce.load(name=EXT_NAME, sources=[os.path.join(CSRC, f) for f in ("torch_layer.cpp", "torch_nodes.cpp")], build_directory=EXT_DIR,
-            extra_include_paths=[INCLUDE], extra_cflags=["-O2"], verbose=verbose)
+    rocm = ce.ROCM_HOME or "/opt/rocm"  # headers of torch's stream type
+    ce.load(name=EXT_NAME, sources=[os.path.join(CSRC, f) for f in ("torch_layer.cpp", "torch_nodes.cpp")],
+            build_directory=EXT_DIR, extra_include_paths=[INCLUDE, os.path.join(rocm, "include")],
+            extra_cflags=["-O2", "-D__HIP_PLATFORM_AMD__=1"], extra_ldflags=["-lc10_hip"], verbose=verbose)
     if not os.path.exists(EXT):
         raise RuntimeError(f"torch extension build produced no {EXT}")
     return EXT

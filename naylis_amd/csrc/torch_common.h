@@ -38,6 +38,9 @@ inline void* ptr(const at::Tensor& t) { return t.defined() ? t.data_ptr() : null
 
 inline void* stream_ptr(int64_t st) { return reinterpret_cast<void*>(st); }
 
+// torch's current stream on t's device
+void* current_stream(const at::Tensor& t);
+
 // The kernels read the products' results by their pointers, as bf16: a backward
 // that the caller runs under autocast must not make them another type.
 struct NoAutocast {

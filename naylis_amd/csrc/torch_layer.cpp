@@ -246,7 +246,7 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
                               r[8], r[9], r[10], r[11], r[12], r[13]});
     ctx->saved_data["ckpt"] = ckpt;
     ctx->saved_data["gate"] = gate;
-    ctx->saved_data["geom"] = std::vector<int64_t>{n_heads, num_blocks, block_size, top_k, stream};
+    ctx->saved_data["geom"] = std::vector<int64_t>{n_heads, num_blocks, block_size, top_k};
     ctx->saved_data["external"] = external;
     ctx->saved_data["m_shape"] = external ? std::vector<int64_t>{} : m_blocks.sizes().vec();
     ctx->saved_data["m_bf16"] = !external && m_blocks.scalar_type() == at::kBFloat16;
@@ -268,7 +268,7 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
       const NoAutocast no_autocast;
       at::DeviceGuard guard(s[0].device());
       const ReadState rd = read_part(s[0], opt(s[1]), s[4], s[5], s[6], opt(s[13]), opt(s[14]), s[11], s[12], geom[0],
-                                     geom[1], geom[2], geom[3], stream_ptr(geom[4]));
+                                     geom[1], geom[2], geom[3], current_stream(s[0]));
       s[1] = rd.slots;
       s[13] = rd.k;
       s[14] = rd.v;
@@ -282,7 +282,8 @@ struct MomLayerNode : public torch::autograd::Function<MomLayerNode> {
     std::vector<at::Tensor> r =
         backward_parts(opt(grads[0]), opt(grads[1]), s[0], opt(s[1]), s[2], s[3], s[4], s[5], s[6], s[7], s[8], s[9],
                        s[10], s[11], s[12], s[13], s[14], s[15], s[16], s[17], opt(s[18]), s[19], s[20], geom[0],
-                       geom[1], geom[2], geom[3], external, m_shape, m_bf16, gate, geom[4]);
+                       geom[1], geom[2], geom[3], external, m_shape, m_bf16, gate,
+                       reinterpret_cast<int64_t>(current_stream(s[0])));
     // r: dx, d_m, dw_down, dw_up, dw_q, dw_k, dw_v, dw_o, ds, dk_ext, dv_ext
     const at::Tensor none;
     if (gate) r[8] = r[8].view(s[8].sizes());

@@ -1,7 +1,8 @@
 // The library's single operations as C++ autograd functions, and the decode
 // step: what the Python modules of mom_kernels/ call.  Each node allocates its
-// outputs, makes its C-ABI calls on the stream that the caller was on and
-// saves its tensors; the autograd engine runs the backward without Python.
+// outputs, makes its C-ABI calls on the caller's current stream (a backward on
+// the one current then) and saves its tensors; the autograd engine runs the
+// backward without Python.
 // Argument checks and dispatch rules stay in the Python wrappers.
 //
 // A Python autograd function over ctypes costs 15 - 30 us of host time per
@@ -11,6 +12,7 @@
 // half 410 -> 339 and attention half 620 -> 507, eight layers' evaluation
 // 3630 -> 3120.
 #include <ATen/autocast_mode.h>
+#include <c10/hip/HIPStream.h>
 
 #include "torch_common.h"
 
@@ -65,6 +67,8 @@ void raise_status(int rc) {
   e.persist();
   throw e;
 }
+
+void* current_stream(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
 std::vector<at::Tensor> linear_fwd(const at::Tensor& x, const std::vector<at::Tensor>& w, at::ScalarType dtype,
                                    void* st) {
@@ -197,7 +201,6 @@ struct RmsNorm : public Function<RmsNorm> {
                                  D, (float)eps, stream_ptr(st)));
     ctx->save_for_backward({x2, w, rstd});
     ctx->saved_data["shape"] = x.sizes().vec();
-    ctx->saved_data["st"] = st;
     return y.view(x.sizes());
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -210,7 +213,7 @@ struct RmsNorm : public Function<RmsNorm> {
     at::Tensor ws = workspace(naylis_mom_rmsnorm_workspace_bytes(N, D), x2);
     check(naylis_mom_rmsnorm_bwd(x2.data_ptr(), dtype_code(x2), w.data_ptr(), rstd.data_ptr<float>(), dy.data_ptr(),
                                  dx.data_ptr(), dw.data_ptr(), ws.data_ptr(), ws.numel(), N, D,
-                                 stream_ptr(ctx->saved_data["st"].toInt())));
+                                 current_stream(x2)));
     return {dx.view(ctx->saved_data["shape"].toIntVector()), dw, at::Tensor(), at::Tensor()};
   }
 };
@@ -228,7 +231,6 @@ struct AddRmsNorm : public Function<AddRmsNorm> {
                                      stream_ptr(st)));
     ctx->save_for_backward({s, w, rstd});
     ctx->saved_data["shape"] = x.sizes().vec();
-    ctx->saved_data["st"] = st;
     ctx->set_materialize_grads(false);
     return {s.view(x.sizes()), y.view(x.sizes())};
   }
@@ -243,7 +245,7 @@ struct AddRmsNorm : public Function<AddRmsNorm> {
     at::Tensor ws = workspace(naylis_mom_rmsnorm_workspace_bytes(N, D), s);
     check(naylis_mom_add_rmsnorm_bwd(s.data_ptr(), w.data_ptr(), rstd.data_ptr<float>(), dy.data_ptr(), ptr(dres),
                                      ds.data_ptr(), dw.data_ptr(), ws.data_ptr(), ws.numel(), dtype_code(s), N, D,
-                                     stream_ptr(ctx->saved_data["st"].toInt())));
+                                     current_stream(s)));
     ds = ds.view(ctx->saved_data["shape"].toIntVector());
     return {ds, ds, dw, at::Tensor(), at::Tensor()};
   }
@@ -252,13 +254,12 @@ struct AddRmsNorm : public Function<AddRmsNorm> {
 // ---- rotary embedding, causal attention, SwiGLU -----------------------------
 
 variable_list rope_call(const at::Tensor& q_in, const at::Tensor& k_in, const at::Tensor& cs, const at::Tensor& sn,
-                        bool backward, int64_t st) {
+                        bool backward, void* st) {
   at::DeviceGuard guard(q_in.device());
   const at::Tensor q = q_in.contiguous(), k = k_in.contiguous(), c = cs.contiguous(), s = sn.contiguous();
   at::Tensor qo = at::empty_like(q), ko = at::empty_like(k);
   check(naylis_mom_rope(q.data_ptr(), k.data_ptr(), c.data_ptr(), s.data_ptr(), qo.data_ptr(), ko.data_ptr(),
-                        dtype_code(q), backward, q.size(0), q.size(1), q.size(2), q.size(3), c.size(0),
-                        stream_ptr(st)));
+                        dtype_code(q), backward, q.size(0), q.size(1), q.size(2), q.size(3), c.size(0), st));
   return {qo, ko};
 }
 
@@ -266,24 +267,23 @@ struct Rope : public Function<Rope> {
   static variable_list forward(AutogradContext* ctx, at::Tensor q, at::Tensor k, at::Tensor cs, at::Tensor sn,
                                int64_t st) {
     ctx->save_for_backward({cs, sn});
-    ctx->saved_data["st"] = st;
-    return rope_call(q, k, cs, sn, false, st);
+    return rope_call(q, k, cs, sn, false, stream_ptr(st));
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
-    const variable_list g = rope_call(grads[0], grads[1], s[0], s[1], true, ctx->saved_data["st"].toInt());
+    const variable_list g = rope_call(grads[0], grads[1], s[0], s[1], true, current_stream(grads[0]));
     return {g[0], g[1], at::Tensor(), at::Tensor(), at::Tensor()};
   }
 };
 
 variable_list attention_grads(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& out,
-                              const at::Tensor& lse, const at::Tensor& grad, double scale, int64_t st) {
+                              const at::Tensor& lse, const at::Tensor& grad, double scale) {
   at::DeviceGuard guard(q.device());
   const at::Tensor dout = grad.to(q.scalar_type()).contiguous();
   at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(lse);
   check(naylis_mom_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
                             dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr<float>(),
-                            (float)scale, q.size(0), q.size(1), q.size(2), q.size(3), stream_ptr(st)));
+                            (float)scale, q.size(0), q.size(1), q.size(2), q.size(3), current_stream(q)));
   return {dq, dk, dv};
 }
 
@@ -292,8 +292,8 @@ variable_list attention_grads(const at::Tensor& q, const at::Tensor& k, const at
 // (as torch's flash attention does) instead of leaving this part out.
 struct CausalAttentionGrad : public Function<CausalAttentionGrad> {
   static variable_list forward(AutogradContext*, at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor out,
-                               at::Tensor lse, at::Tensor dout, double scale, int64_t st) {
-    return attention_grads(q, k, v, out, lse, dout, scale, st);
+                               at::Tensor lse, at::Tensor dout, double scale) {
+    return attention_grads(q, k, v, out, lse, dout, scale);
   }
   static variable_list backward(AutogradContext*, variable_list) {
     TORCH_CHECK(false, "causal_attention: the derivative of its backward is not implemented");
@@ -313,16 +313,14 @@ struct CausalAttention : public Function<CausalAttention> {
                               (float)scale, B, S, H, hd, stream_ptr(st)));
     ctx->save_for_backward({q, k, v, out, lse});
     ctx->saved_data["scale"] = scale;
-    ctx->saved_data["st"] = st;
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
     const double scale = ctx->saved_data["scale"].toDouble();
-    const int64_t st = ctx->saved_data["st"].toInt();
     variable_list g = at::GradMode::is_enabled()
-                          ? CausalAttentionGrad::apply(s[0], s[1], s[2], s[3], s[4], grads[0], scale, st)
-                          : attention_grads(s[0], s[1], s[2], s[3], s[4], grads[0], scale, st);
+                          ? CausalAttentionGrad::apply(s[0], s[1], s[2], s[3], s[4], grads[0], scale)
+                          : attention_grads(s[0], s[1], s[2], s[3], s[4], grads[0], scale);
     g.resize(5);
     return g;
   }
@@ -336,7 +334,6 @@ struct SwiGLU : public Function<SwiGLU> {
     at::Tensor h = at::empty_like(g);
     check(naylis_mom_swiglu_fwd(g.data_ptr(), u.data_ptr(), h.data_ptr(), dtype_code(g), g.numel(), stream_ptr(st)));
     ctx->save_for_backward({g, u});
-    ctx->saved_data["st"] = st;
     return h;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -346,7 +343,7 @@ struct SwiGLU : public Function<SwiGLU> {
     const at::Tensor dh = grads[0].to(g.scalar_type()).contiguous();
     at::Tensor dg = at::empty_like(g), du = at::empty_like(u);
     check(naylis_mom_swiglu_bwd(g.data_ptr(), u.data_ptr(), dh.data_ptr(), dg.data_ptr(), du.data_ptr(),
-                                dtype_code(g), g.numel(), stream_ptr(ctx->saved_data["st"].toInt())));
+                                dtype_code(g), g.numel(), current_stream(g)));
     return {dg, du, at::Tensor()};
   }
 };
@@ -364,14 +361,13 @@ struct SharedLinear : public Function<SharedLinear> {
     variable_list saved = w;
     saved.push_back(x);
     ctx->save_for_backward(saved);
-    ctx->saved_data["st"] = st;
     return linear_fwd(x, w, x.scalar_type(), stream_ptr(st));
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
     const at::Tensor& x = s.back();
     at::DeviceGuard guard(x.device());
-    void* st = stream_ptr(ctx->saved_data["st"].toInt());
+    void* st = current_stream(x);
     const size_t n = s.size() - 1;
     const at::Tensor x2 = x.reshape({-1, x.size(-1)}).contiguous();
     variable_list r(6);
@@ -412,7 +408,6 @@ struct Route : public Function<Route> {
                                 want_h ? h.data_ptr<float>() : nullptr, ws.data_ptr(), ws.numel(), B, T, D, R, E,
                                 top_k, stream_ptr(st)));
     ctx->save_for_backward({x, w_down, w_up, act, probs, idx, gates});
-    ctx->saved_data["st"] = st;
     ctx->set_materialize_grads(false);
     if (want_h) {
       ctx->mark_non_differentiable({idx, h});
@@ -437,7 +432,7 @@ struct Route : public Function<Route> {
                                 static_cast<const float*>(ptr(dp.t)), dp.stride,
                                 static_cast<const float*>(ptr(d_logits)), dx.data_ptr(), 0, dw_down.data_ptr<float>(),
                                 dw_up.data_ptr<float>(), ws.data_ptr(), ws.numel(), B, T, D, R, E, k,
-                                stream_ptr(ctx->saved_data["st"].toInt())));
+                                current_stream(x)));
     variable_list r(10);
     r[0] = dx;
     r[1] = dw_down;
@@ -491,7 +486,7 @@ struct Read : public Function<Read> {
                               lse.data_ptr<float>(), nullptr, 0, B, S, H, HD, num_blocks, block_size, top_k,
                               stream_ptr(st)));
     ctx->save_for_backward({q, k, v, idx, gates, order, out, side, lse});
-    ctx->saved_data["geom"] = std::vector<int64_t>{num_blocks, block_size, st};
+    ctx->saved_data["geom"] = std::vector<int64_t>{num_blocks, block_size};
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
@@ -508,7 +503,7 @@ struct Read : public Function<Read> {
                               gates.data_ptr<float>(), order.data_ptr<int32_t>(), out.data_ptr(), ptr(side),
                               lse.data_ptr<float>(), dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
                               dg.data_ptr<float>(), ws.data_ptr(), ws.numel(), B, S, H, HD, geom[0], geom[1], top_k,
-                              stream_ptr(geom[2])));
+                              current_stream(q)));
     return {dq, dk, dv, at::Tensor(), dg, at::Tensor(), at::Tensor(), at::Tensor()};
   }
 };
@@ -518,7 +513,6 @@ struct GatedLinear : public Function<GatedLinear> {
     at::DeviceGuard guard(out.device());
     const auto [y2, w_os] = gated_linear_forward(out.reshape({-1, w_o.size(1)}), w_o, s, stream_ptr(st));
     ctx->save_for_backward({out, w_o, w_os, s});
-    ctx->saved_data["st"] = st;
     std::vector<int64_t> shape = out.sizes().vec();
     shape.back() = w_o.size(0);
     return y2.view(shape);
@@ -535,7 +529,7 @@ struct GatedLinear : public Function<GatedLinear> {
               at::Tensor()};
     }
     const GatedGrads g = gated_linear_backward(grads[0].reshape({-1, w_o.size(0)}), out.reshape({-1, w_o.size(1)}),
-                                               w_o, w_os, s, stream_ptr(ctx->saved_data["st"].toInt()));
+                                               w_o, w_os, s, current_stream(out));
     return {g.dout2.view(out.sizes()), g.dw_o, g.ds.view(s.sizes()), at::Tensor()};
   }
 };
@@ -561,13 +555,13 @@ struct Xent : public Function<Xent> {
     check(naylis_mom_xent_fwd(logits.data_ptr(), labels.data_ptr<int64_t>(), loss.data_ptr<float>(),
                               lse.data_ptr<float>(), N, V, ignore_index, stream_ptr(st)));
     ctx->save_for_backward({logits, labels, lse});
-    ctx->saved_data["args"] = std::vector<int64_t>{ignore_index, st};
+    ctx->saved_data["ignore_index"] = ignore_index;
     return loss;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
     const at::Tensor &logits = s[0], &labels = s[1], &lse = s[2];
-    const std::vector<int64_t> args = ctx->saved_data["args"].toIntVector();
+    const int64_t ignore_index = ctx->saved_data["ignore_index"].toInt();
     at::DeviceGuard guard(logits.device());
     const int64_t N = logits.size(0), V = logits.size(1);
     at::Tensor g = grads[0].to(at::kFloat);
@@ -575,8 +569,8 @@ struct Xent : public Function<Xent> {
     if (!one) g = g.contiguous();
     at::Tensor dlogits = at::empty_like(logits);
     check(naylis_mom_xent_bwd(logits.data_ptr(), labels.data_ptr<int64_t>(), lse.data_ptr<float>(),
-                              g.data_ptr<float>(), one ? 0 : 1, dlogits.data_ptr(), N, V, args[0],
-                              stream_ptr(args[1])));
+                              g.data_ptr<float>(), one ? 0 : 1, dlogits.data_ptr(), N, V, ignore_index,
+                              current_stream(logits)));
     return {dlogits, at::Tensor(), at::Tensor(), at::Tensor()};
   }
 };

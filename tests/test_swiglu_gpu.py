@@ -56,3 +56,25 @@ def test_status_error_in_a_backward_keeps_its_type(dev):
     with pytest.raises(_lib.NaylisError) as err, torch.no_grad():
         swiglu(buf[1:].view(4, 64), u)
     assert err.value.code == _lib.NAYLIS_ERR_ARG
+
+
+def test_backward_launches_on_the_current_stream(dev):
+    """A backward called directly on another stream than the forward's launches
+    there: under capture its kernel is in the graph, and replays follow their
+    inputs."""
+    from naylis_amd.mom_kernels.hip_mlp import swiglu
+    gen = torch.Generator(device=dev).manual_seed(3)
+    g, u = (torch.randn(64, 64, generator=gen, device=dev).bfloat16().requires_grad_() for _ in range(2))
+    dys = [torch.randn(64, 64, generator=gen, device=dev).bfloat16() for _ in range(3)]
+    h = swiglu(g, u)
+    want = [torch.autograd.grad(h, (g, u), d, retain_graph=True) for d in dys]
+    dy = dys[0].clone()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        got = h.grad_fn(dy)
+    for d, w in zip(dys, want):
+        dy.copy_(d)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], w[0]) and torch.equal(got[1], w[1])
