@@ -11,6 +11,7 @@ attention with heads of 64 runs on the library's kernels
 from __future__ import annotations
 
 import torch
+from transformers.integrations.sdpa_attention import sdpa_attention_forward
 from transformers.models.llama.modeling_llama import ALL_ATTENTION_FUNCTIONS, LlamaAttention, eager_attention_forward
 
 from .. import _lib, _torch_ext
@@ -55,9 +56,11 @@ class NaylisAttention(LlamaAttention):
 
     def _plain_causal(self, attention_mask, kwargs):
         """The SDPA call is softmax(q k^T) v over the causal triangle and
-        nothing else: no mask, no dropout, no option of its own, and torch's
-        flash backend (the same arithmetic) not switched off by the program."""
+        nothing else: no mask, no dropout, no option of its own, transformers'
+        "sdpa" entry not replaced and torch's flash backend (the same
+        arithmetic) not switched off by the program."""
         return (self.config._attn_implementation == "sdpa" and attention_mask is None and not kwargs
+                and ALL_ATTENTION_FUNCTIONS.get_interface("sdpa", None) is sdpa_attention_forward
                 and self.is_causal and self.scaling > 0 and not (self.training and self.attention_dropout)
                 and torch.backends.cuda.flash_sdp_enabled())
 

@@ -378,3 +378,18 @@ def test_trunk_nodes_at_config3_shapes(block, dev):
         err, floor = _rel_frob(got, want), _rel_frob(eager, want)
         print(f"{block} {name:20s} err {err:.3e}  bf16 eager {floor:.3e}  library vs eager {_rel_frob(got, eager):.3e}")
         assert err <= max(1e-2, 2 * floor), (name, err, floor)
+
+
+def test_attention_keeps_a_replaced_sdpa_entry():
+    """A program that puts its own function under transformers' "sdpa" name gets
+    it called, not the library's causal kernels."""
+    from naylis_amd.mom_kernels import hip_rope
+    cfg = naylis_config(vocab_size=256, d_model=128, n_layers=1, n_heads=2, intermediate_size=256, seq_len=32)
+    attn = hip_rope.NaylisAttention(cfg, 0)
+    assert attn._plain_causal(None, {})
+    hip_rope.ALL_ATTENTION_FUNCTIONS["sdpa"] = lambda *args, **kwargs: None
+    try:
+        assert not attn._plain_causal(None, {})
+    finally:
+        del hip_rope.ALL_ATTENTION_FUNCTIONS["sdpa"]
+    assert attn._plain_causal(None, {})
