@@ -276,10 +276,16 @@ struct Rope : public Function<Rope> {
   }
 };
 
+// Contiguous at an address that the kernels' 16-byte loads take.
+at::Tensor aligned(const at::Tensor& t) {
+  const at::Tensor c = t.contiguous();
+  return (uintptr_t)c.data_ptr() % 16 == 0 ? c : c.clone();
+}
+
 variable_list attention_grads(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& out,
                               const at::Tensor& lse, const at::Tensor& grad, double scale) {
   at::DeviceGuard guard(q.device());
-  const at::Tensor dout = grad.to(q.scalar_type()).contiguous();
+  const at::Tensor dout = aligned(grad.to(q.scalar_type()));
   at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), delta = at::empty_like(lse);
   check(naylis_mom_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
                             dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr<float>(),
@@ -305,9 +311,9 @@ struct CausalAttention : public Function<CausalAttention> {
                             int64_t st) {
     at::DeviceGuard guard(q.device());
     const int64_t B = q.size(0), S = q.size(1), H = q.size(2), hd = q.size(3);
-    q = q.contiguous();
-    k = k.contiguous();
-    v = v.contiguous();
+    q = aligned(q);
+    k = aligned(k);
+    v = aligned(v);
     at::Tensor out = at::empty_like(q), lse = at::empty({B, H, S}, f32_of(q));
     check(naylis_mom_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr<float>(),
                               (float)scale, B, S, H, hd, stream_ptr(st)));

@@ -114,3 +114,23 @@ def test_attention_second_derivative_raises(dev):
                               create_graph=True)
     with pytest.raises(RuntimeError, match="not implemented"):
         torch.autograd.grad(dx.float().square().sum(), attn.v_proj.weight)
+
+
+def test_attention_takes_any_address(dev):
+    """Contiguous q, k, v and gradients at addresses that are no multiple of 16
+    bytes (views into larger buffers), as torch's attention takes them."""
+    from naylis_amd.mom_kernels.hip_attention import causal_attention
+    g = torch.Generator(device=dev).manual_seed(4)
+    x = [torch.randn(2, 40, 2, 64, generator=g, device=dev).bfloat16() for _ in range(4)]
+
+    def odd(t):
+        b = torch.empty(t.numel() + 1, device=dev, dtype=t.dtype)[1:].view(t.shape)
+        return b.copy_(t)
+
+    def run(ts):
+        q, k, v = (t.requires_grad_() for t in ts[:3])
+        o = causal_attention(q, k, v, 0.125)
+        return [o, *torch.autograd.grad(o, (q, k, v), ts[3])]
+
+    for a, b in zip(run(x), run([odd(t.detach()) for t in x])):
+        assert torch.equal(a, b)
