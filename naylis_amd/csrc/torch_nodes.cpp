@@ -450,7 +450,7 @@ struct Route : public Function<Route> {
 struct RouterStats : public Function<RouterStats> {
   static at::Tensor forward(AutogradContext* ctx, at::Tensor probs, at::Tensor idx, int64_t st) {
     at::DeviceGuard guard(probs.device());
-    const int64_t E = probs.size(-1), N = probs.numel() / E;
+    const int64_t E = probs.size(-1), N = probs.numel() / std::max<int64_t>(E, 1);
     at::Tensor stats = at::empty({2 * E + 3}, probs.options());
     at::Tensor ws = workspace(need(naylis_mom_router_stats_workspace_bytes(N, E)), probs);
     check(naylis_mom_router_stats(probs.data_ptr<float>(), idx.data_ptr<int32_t>(), stats.data_ptr<float>(),

@@ -39,8 +39,8 @@ def _library_ok(x, weight, rows=8):
     token count a multiple of ``rows``."""
     D_out, D_in = weight.shape
     return (x.is_cuda and torch.version.hip is not None and x.dtype == torch.bfloat16
-            and weight.dtype == torch.bfloat16 and weight.device == x.device and D_in % 8 == 0 and D_out % 8 == 0
-            and x.shape[-1] == D_in and (x.numel() // D_in) % rows == 0)
+            and weight.dtype == torch.bfloat16 and weight.device == x.device and D_in > 0 and D_in % 8 == 0
+            and D_out % 8 == 0 and x.shape[-1] == D_in and (x.numel() // D_in) % rows == 0)
 
 
 def _untransformed(x, *weights):

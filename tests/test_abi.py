@@ -391,3 +391,10 @@ def test_inline_assembly_names_m0(lib):
                 seen += 1
                 assert '"m0"' in block, (name, block)
     assert seen >= 1
+
+
+def test_router_stats_of_no_blocks_raises(lib):
+    """A routing over no blocks is an error (host tensors: no kernel is reached)."""
+    from naylis_amd import _torch_ext
+    with pytest.raises(RuntimeError):
+        _torch_ext.load().router_stats(torch.zeros(4, 0), torch.zeros(4, 2, dtype=torch.int32), 0)

@@ -275,6 +275,19 @@ def test_linear_routes(dev):
         assert not torch.equal(traced(x), traced(2 * x))
 
 
+@pytest.mark.parametrize("grad", [False, True])
+def test_linear_of_no_features(grad, dev):
+    """Layers of no input features give zeros, as torch's do."""
+    from naylis_amd.mom_kernels.hip_linear import mom_linear, shared_input_linear
+    mods = [torch.nn.Linear(8, 16, bias=False).to(dev, torch.bfloat16) for _ in range(2)]
+    for m in mods:
+        m.weight = torch.nn.Parameter(m.weight.detach()[:, :0])
+    x = torch.zeros(8, 0, device=dev, dtype=torch.bfloat16)
+    with torch.set_grad_enabled(grad):
+        ys = [mom_linear(x, mods[0].weight), *shared_input_linear(x, mods)]
+    assert all(torch.equal(y, torch.zeros(8, 16, device=dev, dtype=torch.bfloat16)) for y in ys)
+
+
 def test_linear_keeps_global_hooks_and_replaced_forwards(dev):
     from naylis_amd.mom_kernels.hip_linear import NaylisLinear, shared_input_linear
     mods = [NaylisLinear(256, 384, bias=False).to(dev, torch.bfloat16) for _ in range(2)]
