@@ -87,3 +87,25 @@ def test_xent_forward_masked_rows(chunks, dev):
     assert bool(((got - want).abs() <= 2.0 ** -21 + 2.0 ** -22 * scale).all()), (got, want)
     x[0] = -float("inf")                       # nothing to choose from: NaN, as log_softmax
     assert bool(cross_entropy_rows(x.to(dev), labels.to(dev))[0].isnan())
+
+
+@pytest.mark.parametrize("V", [2048, 24576])
+def test_xent_gradients_of_unlikely_classes(V, dev):
+    """Logits of deviation 40: gradients down to bf16's subnormal range, each within
+    a bf16 rounding (2^-8, or half of the subnormal spacing 2^-133) of fp64 and p's
+    own error.  That is the row's log-sum-exp, under 2^8, rounded to fp32, 2^-17
+    at most, and few ulp of the exponential; a value lies so near a rounding
+    boundary that it may go the other way with probability 2 * 2^-17 / 2^-8."""
+    from naylis_amd.mom_kernels.hip_xent import cross_entropy_rows
+    g = torch.Generator(device=dev).manual_seed(V)
+    z = (torch.randn(256, V, generator=g, device=dev) * 40).bfloat16().requires_grad_(True)
+    y = torch.randint(0, V, (256,), generator=g, device=dev)
+    cross_entropy_rows(z, y).sum().backward()
+    logp = torch.log_softmax(z.detach().double(), -1)
+    assert float((z.detach().double() - logp).max()) < 2 ** 8
+    p = logp.exp()  # (torch's softmax drops values under e^-87 here)
+    d = p.scatter_add(1, y[:, None], -torch.ones_like(y[:, None], dtype=p.dtype))
+    err = (z.grad.double() - d).abs()
+    assert bool((err <= 2.0 ** -8 * d.abs() + 2.0 ** -16 * p + 2.0 ** -134).all())
+    assert float((z.grad != d.bfloat16()).double().mean()) < 2.0 ** -8
+    assert bool(((z.grad != 0) & (z.grad.abs() < 2.0 ** -126)).any())
