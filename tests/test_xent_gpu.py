@@ -64,7 +64,7 @@ def test_xent_rejects_unsupported(dev):
         cross_entropy_rows(torch.randn(4, 1000, device=dev).bfloat16(), torch.zeros(4, dtype=torch.long, device=dev))
 
 
-@pytest.mark.parametrize("chunks", [1, 4, 5, 8, 9, 17])
+@pytest.mark.parametrize("chunks", [1, 2, 3, 4, 5, 8, 9, 17])
 def test_xent_forward_masked_rows(chunks, dev):
     """Rows around the forward's register tiles (4 or 8 chunks of 2048), with
     -inf and lowest-value masks over whole threads, chunks and rows, against
