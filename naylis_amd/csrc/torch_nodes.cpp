@@ -34,25 +34,41 @@ bool bf16_products() {
          at::autocast::get_autocast_dtype(at::kCUDA) == at::kBFloat16;
 }
 
-// Where the library's GEMM takes a forward product (whole 128-column tiles):
-// one product up to 6 M outputs, where its kernel is level with hipBLASLt's or
-// ahead from 1024 rows on (8.6 against 11.2 us at 2042 x 1024 x 1024, 17.0
-// against 22.0 at 2042 x 1024 -> 2816, 22.6 against 22.9 at 4096 x 1536 x 1536;
-// below, up to 6 us behind) and its host call takes 6 us against 20; two or
-// three of one input up to 768 tiles of 128 x 128, in one launch (q/k/v of 2042
-// tokens at d 1024: 17.2 us against 34; gate/up 1024 -> 2816: 29 against 44;
-// three at 3885 tokens: 30 against 41).  Past that hipBLASLt's tiles win (two of
-// 3885 x 1024 -> 2816, 1335 tiles: 50 against 47).
+// A product of more 128 x 128 tiles than CUs and too few 256 x 128 ones for
+// theirs: on the library's GEMM it runs with padded tiles and one stage ahead,
+// 1.3 to 2 times hipBLASLt's time (K 1024, 1533 x 2816: 23.1 us against 14.5, as
+// an input gradient 30.9 against 22.2; K 2816, 4221 x 1024: 49 / 29, 67 / 35).
+bool between_tiles(int64_t rows, int64_t cols) {
+  const int64_t n = (cols + 127) / 128;
+  return (rows + 127) / 128 * n > 256 && (rows + 255) / 256 * n < 144;
+}
+
+// Where the library's GEMM takes a forward product (whole 128-column tiles).
+// One product up to 6 M outputs: from 1000 rows on its kernel is level with
+// hipBLASLt's or ahead (2042 x 1024 over 1024: 9.5 against 10.3 us, x 2816 17.9
+// against 20.9), below that behind on the device and ahead where the host sets
+// the pace, with a call of 6 us against 18 (64 rows, 1024 over 1024: kernels 7.2
+// against 6.7 us, calls back to back 7.1 against 17.7; over 2816 13.8 against 6.9
+// and 13.6 against 17.8; 1 row over 2816: 15.9 / 6.3 and 16.1 / 17.8).  Longer K
+// leaves it behind everywhere (over 4096, 2042 x 1024 25.8 against 25.4, 512 rows
+// 19.4 against 14.3; over 5632, 2042 x 2048 53.6 against 49.5).  Two or three of
+// one input up to 768 tiles of 128 x 128, in one launch: q/k/v of 2042 tokens at
+// d 1024 18.6 us against 31.4, of 64 7.4 / 19.4; gate/up 1024 -> 2816 27.6 / 41.8.
+// Past that hipBLASLt's tiles win (two of 3885 x 1024 -> 2816, 1335 tiles: 50
+// against 47).
 bool own_fwd(int64_t n, int64_t N, int64_t D_in, int64_t D_out) {
   return N > 0 && D_in % 64 == 0 && D_out % 128 == 0 && D_in <= 2816 &&
-         (n == 1 ? N * D_out <= 6 << 20 : n * N * D_out <= 12 << 20);
+         (n == 1 ? N * D_out <= 6 << 20 && !between_tiles(N, D_out) : n * N * D_out <= 12 << 20);
 }
 
 // ... and an input gradient: ahead of hipBLASLt's kernel from 64 rows to 6 M
-// outputs (2042 x 1024 x 1024: 9.2 against 12.6 us; 4096 x 1536 x 1536: 23.0
-// against 26.6; past it level, 4096 x 2048 x 2048 33.2 against 34.1).
+// outputs (1021 x 1024 over 1024 7.6 against 9.5 us, 2042 rows 9.9 / 12.0, 2042 x
+// 2048 over 2048 22.2 / 25.6, 1021 x 2816 over 1024 12.3 / 17.0).  Past it neither
+// is ahead by a rule of size: over 2048 and 5632, 8192 to 16384 rows, hipBLASLt by
+// 2 - 9 %, 16384 x 2816 over 1024 the library (97 against 111).
 bool own_dgrad(int64_t N, int64_t D_in, int64_t D_out) {
-  return N >= 64 && D_in % 128 == 0 && D_out % 64 == 0 && D_out <= 2816 && N * D_in <= 6 << 20;
+  return N >= 64 && D_in % 128 == 0 && D_out % 64 == 0 && D_out <= 2816 && N * D_in <= 6 << 20 &&
+         !between_tiles(N, D_in);
 }
 
 }  // namespace

@@ -275,6 +275,26 @@ def test_linear_routes(dev):
         assert not torch.equal(traced(x), traced(2 * x))
 
 
+@pytest.mark.parametrize("N,D_in,D_out,fwd,dgrad", [
+    (1400, 1024, 2816, True, True),     # 242 tiles of 128 x 128: one round
+    (1533, 1024, 2816, False, True),    # 264 and 132 of 256 x 128: between (dx: 1533 x 1024, 96 tiles)
+    (1533, 2816, 1024, True, False),    # the same for dx
+    (1661, 1024, 2816, True, True),     # 286 and 154
+])
+def test_linear_leaves_between_tiles_to_torch(N, D_in, D_out, fwd, dgrad, dev):
+    """Products that neither the one-round tiles nor the large ones take stay on
+    torch's GEMM (the kernels that ran, by their timer's names)."""
+    from naylis_amd import _lib, _torch_ext
+    x, dy = (torch.ones(N, d, device=dev, dtype=torch.bfloat16) for d in (D_in, D_out))
+    w = torch.ones(D_out, D_in, device=dev, dtype=torch.bfloat16)
+    ext, st = _torch_ext.load(), _lib.stream_of(dev)
+    with _lib.KernelTimer():
+        ext.linear(x, [w], False, st)
+        ext.linear_dgrad(dy, w, st)
+    names = _lib.KernelTimer.results()
+    assert ("linear_fwd" in names, "linear_dgrad" in names) == (fwd, dgrad)
+
+
 @pytest.mark.parametrize("grad", [False, True])
 def test_linear_of_no_features(grad, dev):
     """Layers of no input features give zeros, as torch's do."""
