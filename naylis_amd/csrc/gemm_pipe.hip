@@ -544,9 +544,14 @@ static Ranges ranges_of(int M, int N, int K) {
 // per workgroup above all, leave it level with gemm.hip's splits or 10 - 20 %
 // behind), few enough tiles that K has to be cut at all, and at most 4 % of the
 // steps empty (unaligned ranges of 10016 tokens, 1024 x 1024: 47 us against 35
-// with gemm.hip's splits).
+// with gemm.hip's splits).  Nor an odd number of tiles: the 256 ranges then start
+// at 256 distinct K steps, and no two workgroups walk the same rows together
+// (16384 tokens, 1152 x 1152, 45 tiles: 88 us against 71 with splits, 1032 x 1032
+// 114 against 70, 1152 x 2304 164 against 123; at 128 starts, 2 mod 4 tiles, they
+// are between 25 % ahead, 896 x 2432, and 3 - 8 % behind, 18 tiles).
 bool gemm_ranges_ok(int M, int N, int K) {
-  if (K <= 0 || M < 256 || N < 128 || M % 8 || N % 8 || pipe_tiles<Cfg128>(M, N) >= 144) return false;
+  const int tiles = pipe_tiles<Cfg128>(M, N);
+  if (K <= 0 || M < 256 || N < 128 || M % 8 || N % 8 || tiles >= 144 || tiles % 2) return false;
   const Ranges r = ranges_of(M, N, K);
   return r.per >= 16 && ((long)r.nk * Cfg128::BK - K) * 25 <= K;
 }

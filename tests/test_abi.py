@@ -398,3 +398,16 @@ def test_router_stats_of_no_blocks_raises(lib):
     from naylis_amd import _torch_ext
     with pytest.raises(RuntimeError):
         _torch_ext.load().router_stats(torch.zeros(4, 0), torch.zeros(4, 2, dtype=torch.int32), 0)
+
+
+@pytest.mark.parametrize("D_in,D_out,tiles", [(1024, 1024, 32), (1408, 512, 22), (1152, 1152, None), (640, 640, None),
+                                              (264, 520, None), (2304, 1152, None)])
+def test_weight_gradient_ranges(lib, D_in, D_out, tiles):
+    """Long weight gradients of an even number of 256 x 128 tiles are cut into 256
+    K ranges (a partial tile per range and per tile); an odd number, whose ranges
+    would all start at other rows, into whole K splits."""
+    nbytes = lib.naylis_mom_linear_wgrad_workspace_bytes(32768, D_in, D_out)
+    if tiles is None:
+        assert nbytes % (4 * D_in * D_out) == 0
+    else:
+        assert tiles == -(-D_out // 256) * -(-D_in // 128) and nbytes == (256 + tiles) * 256 * 128 * 4
