@@ -22,11 +22,11 @@
 // conflicts.
 //
 // Large products are bound by the matrix units at the clock that the card holds
-// under them: operands of zeros run 15 - 20 % faster, and without any load or
-// LDS read the K loop takes 53 us of the 62 below.  Against gemm.hip (kernel
-// and reduction, 16384 tokens): 1024 x 1024 51.5 -> 42.8 us, 2048 x 1024 80 ->
-// 72, 1024 x 2816 135 -> 99 (0.96 PFLOP/s), 1536 x 1536 107 -> 84; whole tiles,
-// 5632 x 2048 over 4096: 116 -> 85 (1.11 PFLOP/s).
+// under them: operands of zeros run 15 - 20 % faster.  Against gemm.hip (kernel
+// and reduction, 16384 tokens, launches back to back): 1024 x 1024 48.5 -> 42.7
+// us (39.4 + 7.4 in the layer's backward, operands out of the caches), 1024 x
+// 2816 127 -> 97 (0.97 PFLOP/s), 1536 x 1536 107 -> 82, 2048 x 2048 149 -> 134;
+// whole tiles, 5632 x 2048 over 4096: 117 -> 86 (1.10 PFLOP/s).
 #include "common.h"
 #include "launch_gemm.h"
 #include "timing.h"

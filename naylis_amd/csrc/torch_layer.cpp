@@ -5,9 +5,9 @@
 // the folded ReZero gate, and their gradients -- as one call each from
 // Python instead of about fifteen ctypes and torch calls.  They make the same
 // library calls in the same order, with the same allocations and products
-// (linear_fwd / linear_dgrad: the library's GEMM, or hipBLASLt through at::mm /
-// at::linear on torch's current stream), so their results are bitwise those of
-// the Python node.
+// (linear_fwd, linear_dgrad, library_wgrad: the library's GEMM, or hipBLASLt
+// through at::mm / at::linear on torch's current stream), which the Python node
+// takes from here, so their results are bitwise those of the Python node.
 //
 // MomLayerNode is the same node as a C++ autograd function: its forward
 // calls layer_fwd and saves what the Python node saves, its backward calls

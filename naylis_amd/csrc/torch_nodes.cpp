@@ -6,11 +6,11 @@
 // Argument checks and dispatch rules stay in the Python wrappers.
 //
 // A Python autograd function over ctypes costs 15 - 30 us of host time per
-// call and direction, a node here about 6.  Host time to enqueue a pass: one
-// decode step 15.6 -> 7 us, the checkpointed layer (3885 tokens, forward and
-// backward, its recompute in the layer's node) 960 -> 427, the decoder's MLP
-// half 410 -> 339 and attention half 620 -> 507, eight layers' evaluation
-// 3630 -> 3120.
+// call and direction, a node here about 6.  Host time to enqueue a pass, with
+// Python functions and now (fewer launches included): one decode step 16.7 and
+// 8.6 us, the checkpointed layer (3885 tokens, forward and backward, its
+// recompute in the layer's node) 1222 and 295, the decoder's MLP half 596 and
+// 367 and attention half 793 and 531, eight layers' evaluation 3770 and 1826.
 #include <ATen/autocast_mode.h>
 #include <c10/hip/HIPStream.h>
 

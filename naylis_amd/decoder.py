@@ -22,9 +22,10 @@ There is no eager MoM path: off ROCm the MoM layers raise.  The norms
 RMSNorm (``NaylisRMSNorm``, the role of the reference's ``use_liger`` norm)
 when the hidden size is a multiple of 512 up to 4096, LlamaRMSNorm otherwise;
 the attention applies the rotary embedding with the library's fused kernel
-(``NaylisAttention``, same parameters and SDPA backend), the MLP its fused
-SwiGLU (``NaylisMLP``), the bias-free projections of both take their
-weight gradient from the library's split-K GEMM (``use_library_wgrad``), and
+(``NaylisAttention``, same parameters; plain causal bf16 attention with heads
+of 64 on the library's kernels, any other on the configured backend), the MLP
+its fused SwiGLU (``NaylisMLP``), the bias-free projections of both take their
+products from the library's GEMM by size (``use_library_wgrad``), and
 the LM loss reads the bf16 logits once (``cross_entropy_rows``) when the
 vocabulary is a multiple of 2048.
 """

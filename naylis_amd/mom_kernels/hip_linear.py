@@ -12,7 +12,8 @@ torch GEMMs (hipBLASLt) otherwise.
 The decoder trunk's projections (the Llama attention's q/k/v/o and the MLP's
 gate/up/down inside every Naylis decoder layer, model.py:279-345) are the same
 bias-free nn.Linear; ``NaylisLinear`` / ``use_library_wgrad`` give them this
-weight gradient too.  At the config-3 shapes (16384 tokens) hipBLASLt's
+weight gradient too, in training at token counts that are multiples of 8 (other
+counts train on torch's GEMMs and evaluate on the library's).  At the config-3 shapes (16384 tokens) hipBLASLt's
 weight-gradient GEMM runs d x d at about 340 TFLOP/s and d x 2816 at about
 620, the library's at about 800 and 950.
 """
@@ -62,9 +63,10 @@ def _plain_module(m):
 
 def mom_linear(x, weight):
     """y = x W^T (no bias).  For bf16 activations and weights on a ROCm device
-    with dimensions that are multiples of 8 the weight gradient runs on the
-    library's GEMM, and so do the forward and the input gradient at the sizes
-    where it is faster; any other combination is the plain torch linear."""
+    with widths, and in training a token count, that are multiples of 8 the
+    weight gradient runs on the library's GEMM, and so do the forward and the
+    input gradient at the sizes where it is faster; any other combination is
+    the plain torch linear."""
     if not torch.is_grad_enabled():
         if _untransformed(x, weight) and _library_ok(x, weight, 1):
             return _torch_ext.load().linear(x, [weight], False, _lib.stream_of(x.device))[0]
@@ -77,7 +79,7 @@ def shared_input_linear(x, linears):
     """The outputs of several bias-free linear layers applied to one input,
     as a tuple.  One autograd node for up to three of them (the attention's
     q/k/v, the MLP's gate/up) for bf16 activations and weights on a ROCm device
-    with dimensions that are multiples of 8: autograd would sum their input
+    with widths and a token count that are multiples of 8: autograd would sum their input
     gradients with separate elementwise adds, the node accumulates each
     further product into the first in the GEMM's epilogue (one rounding of the
     sum).  Where the library's GEMM is faster it takes all forward products in
