@@ -17,7 +17,7 @@
 //
 // Bound by the vector units: per 32 x 32 tile a forward wave issues 8 MFMAs
 // (256 cycles) and about 16 exp2, 16 fma, 16 adds, 8 max3 and 8 packs.
-// B 8, S 2048, H 16: forward 219 -> 88 us, backward 955 -> 290 us (dQ 115, dK/dV
+// B 8, S 2048, H 16: forward 219 -> 108 us, backward 955 -> 280 us (dQ 115, dK/dV
 // 165 - 176) against torch's scaled_dot_product_attention.
 #include "common.h"
 #include "launch.h"
@@ -125,9 +125,12 @@ struct AttnDims {
 // 200 registers and two waves a SIMD: 98 against 87 us at B 8, S 2048, H 16,
 // and twice the time where they leave CUs idle).  Workgroups run longest first (a query
 // block's work grows with its position), heads innermost so that an XCD keeps
-// its heads' K and V in its L2.  The running reference m moves only when a
-// score exceeds it by more than 2^8 (p stays below 2^8, in range for bf16 and
-// exact in the fp32 sums), so most tiles rescale nothing.
+// its heads' K and V in its L2.  The running reference m is the largest score so
+// far, so that the largest weight is exactly 1 in bf16: a reference that moves
+// only by factors over 2^8 rescales less (95 against 108 us) but rounds that
+// weight too, and the output's error (2-norm, fp64) is 2.08e-3 against 1.99e-3 on
+// normal scores of 1021 keys, 2.13e-3 against 1.75e-3 on scores three times that
+// (torch's flash attention 2.00e-3 and 1.76e-3).
 __global__ __launch_bounds__(256, 4) void attn_fwd_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                                           const bf16_t* __restrict__ v, bf16_t* __restrict__ o,
                                                           float* __restrict__ lse, AttnDims d, int nqb, float c) {
@@ -178,10 +181,10 @@ __global__ __launch_bounds__(256, 4) void attn_fwd_kernel(const bf16_t* __restri
       float mx = s[0];
 #pragma unroll
       for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-      if (__any(mx * c > m + 8.f)) {
+      if (__any(mx * c > m)) {
         // per query, so that a row's result does not depend on its neighbours'
         const float mr = xor32_f32(mx, [](float a, float b) { return fmaxf(a, b); }) * c;
-        const float mn = mr > m + 8.f ? mr : m;
+        const float mn = fmaxf(m, mr);
         const float al = __builtin_amdgcn_exp2f(m - mn);
         m = mn;
         l *= al;

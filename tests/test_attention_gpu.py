@@ -134,3 +134,28 @@ def test_attention_takes_any_address(dev):
 
     for a, b in zip(run(x), run([odd(t.detach()) for t in x])):
         assert torch.equal(a, b)
+
+
+def test_attention_rounds_no_largest_weight(dev):
+    """The largest weight, the exponential of the largest score less itself, is
+    exactly 1 in bf16. The output's squared error is then that of its own rounding
+    plus, for each of the other weights p, that of p's: d^2 p^2 |v|^2 with d the
+    mean relative error of rounding, 10 % spared; with the largest weight's the
+    error would be a fifth larger on these scores."""
+    from naylis_amd.mom_kernels.hip_attention import causal_attention
+    g = torch.Generator(device=dev).manual_seed(6)
+    q, k, v = (torch.randn(2, 1021, 4, 64, generator=g, device=dev).bfloat16() for _ in range(3))
+    q = 3 * q
+    o = causal_attention(q, k, v, 0.125).double().transpose(1, 2)
+    qd, kd, vd = (t.double().transpose(1, 2) for t in (q, k, v))
+    s = qd @ kd.transpose(-1, -2) * 0.125
+    s.masked_fill_(torch.ones(1021, 1021, dtype=torch.bool, device=dev).triu(1), -math.inf)
+    p = torch.softmax(s, -1)
+    ref = p @ vd
+    own = (ref.bfloat16().double() - ref).square().sum()
+    d2 = (p.bfloat16().double() - p).square().sum() / p.square().sum()
+    weights = p.square() @ vd.square().sum(-1, keepdim=True)
+    top = p.amax(-1, keepdim=True).square() * vd.square().sum(-1, keepdim=True).gather(2, p.argmax(-1, keepdim=True))
+    bound = (own + d2 * (weights - top).sum()).sqrt()
+    assert float((own + d2 * weights.sum()).sqrt()) > 1.15 * float(bound)
+    assert float((o - ref).norm()) < 1.1 * float(bound)
